@@ -10,6 +10,8 @@
 // target's tile bit. Barriers are placed only where ownership changes.
 #include "kernels.hpp"
 
+#include <type_traits>
+
 namespace hgm {
 
 namespace {
@@ -577,50 +579,77 @@ __global__ void k_set_basis(typename Vec<T>::type *state, uint64_t n, uint64_t i
     }
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_prob_halves(const typename Vec<T>::type *state, uint64_t n, int bit,
-                                                      double *partial) {
-    __shared__ double s0[256], s1[256];
-    double a0 = 0, a1 = 0;
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const auto v = state[i];
-        const double p = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
-        if (bit >= 0 && ((i >> bit) & 1)) a1 += p; else a0 += p;
+// Reductions over a whole state read every amplitude once and write a few
+// bytes, so they are bound by the bytes in flight: W amplitudes per 16-byte
+// load, and U loads per lane issued before any of them is used. One 8-byte
+// load per lane and iteration read a 4 GiB FP32 state at 3.6 TB/s (1200 us per
+// sum), W = 2 and U = 8 at 6.1 (700 us; a copy moves 6.2). A lane takes every
+// 256th vector of its block's U * 256, so it sees increasing indices.
+template <class T, int W, int U, class F>
+__device__ __forceinline__ void for_amps(const typename Vec<T>::type *state, uint64_t n, F fn) {
+    typedef T Wide __attribute__((ext_vector_type(2 * W)));
+    const Wide *p = reinterpret_cast<const Wide *>(state);
+    const uint64_t nv = n / W, step = (uint64_t)gridDim.x * (256 * U);
+    for (uint64_t v0 = blockIdx.x * (uint64_t)(256 * U) + threadIdx.x; v0 < nv; v0 += step) {
+        Wide w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = p[v0 + u * 256];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                const double x = w[u][2 * j], y = w[u][2 * j + 1];
+                fn((v0 + u * 256) * W + j, x * x + y * y);
+            }
     }
-    s0[threadIdx.x] = a0;
-    s1[threadIdx.x] = a1;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) { s0[threadIdx.x] += s0[threadIdx.x + w]; s1[threadIdx.x] += s1[threadIdx.x + w]; }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) { partial[2 * blockIdx.x] = s0[0]; partial[2 * blockIdx.x + 1] = s1[0]; }
 }
 
-template <class T>
+template <class T, int W, int U>
+__global__ void __launch_bounds__(256) k_prob_halves(const typename Vec<T>::type *state, uint64_t n, int bit,
+                                                      double *partial) {
+    __shared__ double s0[4], s1[4];
+    double a0 = 0, a1 = 0;
+    const uint64_t sel = bit >= 0 ? uint64_t(1) << bit : 0;
+    for_amps<T, W, U>(state, n, [&](uint64_t i, double p) {
+        const bool one = (i & sel) != 0;
+        a0 += one ? 0.0 : p;
+        a1 += one ? p : 0.0;
+    });
+    for (int off = 32; off > 0; off >>= 1) {
+        a0 += __shfl_xor(a0, off);
+        a1 += __shfl_xor(a1, off);
+    }
+    if ((threadIdx.x & 63) == 0) { s0[threadIdx.x >> 6] = a0; s1[threadIdx.x >> 6] = a1; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        partial[2 * blockIdx.x] = (s0[0] + s0[1]) + (s0[2] + s0[3]);
+        partial[2 * blockIdx.x + 1] = (s1[0] + s1[1]) + (s1[2] + s1[3]);
+    }
+}
+
+template <class T, int W, int U>
 __global__ void __launch_bounds__(256) k_argmax(const typename Vec<T>::type *state, uint64_t n, double *pmax,
                                                  uint64_t *pidx) {
-    __shared__ double sm[256];
-    __shared__ uint64_t si[256];
+    __shared__ double sm[4];
+    __shared__ uint64_t si[4];
     double best = -1.0;
     uint64_t bi = ~uint64_t(0);
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        const auto v = state[i];
-        const double p = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+    for_amps<T, W, U>(state, n, [&](uint64_t i, double p) {
         if (p > best) { best = p; bi = i; }
+    });
+    for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(best, off);
+        const uint64_t oi = __shfl_xor(bi, off);
+        if (o > best || (o == best && oi < bi)) { best = o; bi = oi; }
     }
-    sm[threadIdx.x] = best;
-    si[threadIdx.x] = bi;
+    if ((threadIdx.x & 63) == 0) { sm[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bi; }
     __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            const double o = sm[threadIdx.x + w];
-            const uint64_t oi = si[threadIdx.x + w];
-            if (o > sm[threadIdx.x] || (o == sm[threadIdx.x] && oi < si[threadIdx.x])) { sm[threadIdx.x] = o; si[threadIdx.x] = oi; }
-        }
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w)
+            if (sm[w] > best || (sm[w] == best && si[w] < bi)) { best = sm[w]; bi = si[w]; }
+        pmax[blockIdx.x] = best;
+        pidx[blockIdx.x] = bi;
     }
-    if (threadIdx.x == 0) { pmax[blockIdx.x] = sm[0]; pidx[blockIdx.x] = si[0]; }
 }
 
 // Per-block partials of the comparison of two states of any amplitude types:
@@ -801,22 +830,45 @@ hipError_t launch_set_basis(int dtype, void *state, uint64_t n, uint64_t index, 
     return hipGetLastError();
 }
 
+namespace {
+
+// Blocks and loads per lane of a whole-state reduction: 8 loads of 16 bytes
+// when that gives every block at least one full round, else one load (more
+// blocks at work); a borrowed FP32 state that is only 8-byte aligned is read
+// one amplitude at a time.
+template <class F>
+hipError_t reduce_launch(int dtype, const void *state, uint64_t n, int blocks, F launch) {
+    const bool f32 = dtype == HGM_C64;
+    const int W = f32 && n >= 2 && (reinterpret_cast<uintptr_t>(state) & 15) == 0 ? 2 : 1;
+    const bool deep = n / W >= (uint64_t)blocks * 256 * 8;
+    using std::integral_constant;
+    if (!f32) { if (deep) launch(double(), integral_constant<int, 1>(), integral_constant<int, 8>());
+                else launch(double(), integral_constant<int, 1>(), integral_constant<int, 1>()); }
+    else if (W == 2) { if (deep) launch(float(), integral_constant<int, 2>(), integral_constant<int, 8>());
+                       else launch(float(), integral_constant<int, 2>(), integral_constant<int, 1>()); }
+    else { if (deep) launch(float(), integral_constant<int, 1>(), integral_constant<int, 8>());
+           else launch(float(), integral_constant<int, 1>(), integral_constant<int, 1>()); }
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_prob_halves(int dtype, const void *state, uint64_t n, int bit, double *partial, int blocks,
                               hipStream_t s) {
-    if (dtype == HGM_C64)
-        hipLaunchKernelGGL(k_prob_halves<float>, dim3(blocks), dim3(256), 0, s, (const float2 *)state, n, bit, partial);
-    else
-        hipLaunchKernelGGL(k_prob_halves<double>, dim3(blocks), dim3(256), 0, s, (const double2 *)state, n, bit, partial);
-    return hipGetLastError();
+    return reduce_launch(dtype, state, n, blocks, [&](auto t, auto w, auto u) {
+        using T = decltype(t);
+        hipLaunchKernelGGL((k_prob_halves<T, w(), u()>), dim3(blocks), dim3(256), 0, s,
+                           static_cast<const typename Vec<T>::type *>(state), n, bit, partial);
+    });
 }
 
 hipError_t launch_argmax(int dtype, const void *state, uint64_t n, double *pmax, uint64_t *pidx, int blocks,
                          hipStream_t s) {
-    if (dtype == HGM_C64)
-        hipLaunchKernelGGL(k_argmax<float>, dim3(blocks), dim3(256), 0, s, (const float2 *)state, n, pmax, pidx);
-    else
-        hipLaunchKernelGGL(k_argmax<double>, dim3(blocks), dim3(256), 0, s, (const double2 *)state, n, pmax, pidx);
-    return hipGetLastError();
+    return reduce_launch(dtype, state, n, blocks, [&](auto t, auto w, auto u) {
+        using T = decltype(t);
+        hipLaunchKernelGGL((k_argmax<T, w(), u()>), dim3(blocks), dim3(256), 0, s,
+                           static_cast<const typename Vec<T>::type *>(state), n, pmax, pidx);
+    });
 }
 
 hipError_t launch_compare(int dtype_a, const void *a, int dtype_b, const void *b, uint64_t n, double *partial,

@@ -102,10 +102,10 @@ struct Ctx {
     size_t mems_cap = 0;
     void *cache = nullptr;      // device buffer of hgm_execute (grow-only)
     size_t cache_cap = 0;
-    double *partial = nullptr;  // reduction partials (device, 8 doubles per block)
+    // reduction partials, in pinned host memory that the kernels write directly
+    // (a few bytes per block; a copy after the kernel cost about 8 us a call)
+    double *partial = nullptr;  // 8 doubles per block
     uint64_t *pidx = nullptr;
-    double *h_partial = nullptr;  // pinned host mirror
-    uint64_t *h_pidx = nullptr;
     char *h_stage[2] = {nullptr, nullptr};          // pinned chunks of the region copies
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
 };
@@ -185,10 +185,8 @@ int init_locked(int device) {
     HGM_HIP(hipGetDeviceProperties(&prop, device), "hipGetDeviceProperties");
     c.cus = prop.multiProcessorCount;
     if (!c.partial) {
-        HGM_HIP(hipMalloc(&c.partial, 8 * kRedBlocks * sizeof(double)), "hipMalloc(partials)");
-        HGM_HIP(hipMalloc(&c.pidx, kRedBlocks * sizeof(uint64_t)), "hipMalloc(partials)");
-        HGM_HIP(hipHostMalloc(&c.h_partial, 8 * kRedBlocks * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
-        HGM_HIP(hipHostMalloc(&c.h_pidx, kRedBlocks * sizeof(uint64_t), hipHostMallocDefault), "hipHostMalloc");
+        HGM_HIP(hipHostMalloc(&c.partial, 8 * kRedBlocks * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
+        HGM_HIP(hipHostMalloc(&c.pidx, kRedBlocks * sizeof(uint64_t), hipHostMallocDefault), "hipHostMalloc");
     }
     if (device < kMaxDevices && !g_scratch_ptr[device]) {
         void *ptr = nullptr;
@@ -458,11 +456,9 @@ int prob_halves_locked(const hgm_state *s, int bit, double *zero, double *one) {
     const uint64_t n = uint64_t(1) << s->qubits;
     const int blocks = blocks_for(n);
     HGM_HIP(launch_prob_halves(s->dtype, s->d, n, bit, c.partial, blocks, c.stream), "prob kernel");
-    HGM_HIP(hipMemcpyAsync(c.h_partial, c.partial, 2 * blocks * sizeof(double), hipMemcpyDeviceToHost, c.stream),
-            "hipMemcpyAsync(partials)");
     HGM_HIP(hipStreamSynchronize(c.stream), "prob kernel");
     double z = 0, o = 0;
-    for (int b = 0; b < blocks; ++b) { z += c.h_partial[2 * b]; o += c.h_partial[2 * b + 1]; }
+    for (int b = 0; b < blocks; ++b) { z += c.partial[2 * b]; o += c.partial[2 * b + 1]; }
     *zero = z;
     *one = o;
     return HGM_OK;
@@ -1067,13 +1063,11 @@ int hgm_state_argmax(const hgm_state *s, uint64_t *index, double *prob) {
     const uint64_t n = uint64_t(1) << s->qubits;
     const int blocks = blocks_for(n);
     HGM_HIP(launch_argmax(s->dtype, s->d, n, c.partial, c.pidx, blocks, c.stream), "argmax");
-    HGM_HIP(hipMemcpyAsync(c.h_partial, c.partial, blocks * sizeof(double), hipMemcpyDeviceToHost, c.stream), "argmax");
-    HGM_HIP(hipMemcpyAsync(c.h_pidx, c.pidx, blocks * sizeof(uint64_t), hipMemcpyDeviceToHost, c.stream), "argmax");
     HGM_HIP(hipStreamSynchronize(c.stream), "argmax");
     double best = -1;
     uint64_t bi = 0;
     for (int b = 0; b < blocks; ++b)
-        if (c.h_partial[b] > best || (c.h_partial[b] == best && c.h_pidx[b] < bi)) { best = c.h_partial[b]; bi = c.h_pidx[b]; }
+        if (c.partial[b] > best || (c.partial[b] == best && c.pidx[b] < bi)) { best = c.partial[b]; bi = c.pidx[b]; }
     *index = bi;
     if (prob) *prob = best;
     return HGM_OK;
@@ -1087,12 +1081,10 @@ int hgm_state_compare(const hgm_state *a, const hgm_state *b, double *fidelity, 
     const uint64_t n = uint64_t(1) << a->qubits;
     const int blocks = blocks_for(n);
     HGM_HIP(launch_compare(a->dtype, a->d, b->dtype, b->d, n, c.partial, blocks, c.stream), "compare");
-    HGM_HIP(hipMemcpyAsync(c.h_partial, c.partial, 5 * blocks * sizeof(double), hipMemcpyDeviceToHost, c.stream),
-            "compare");
     HGM_HIP(hipStreamSynchronize(c.stream), "compare");
     double re = 0, im = 0, na = 0, nb = 0, mx = 0;
     for (int k = 0; k < blocks; ++k) {
-        const double *q = c.h_partial + 5 * k;
+        const double *q = c.partial + 5 * k;
         re += q[0]; im += q[1]; na += q[2]; nb += q[3];
         mx = std::max(mx, q[4]);
     }
