@@ -41,6 +41,7 @@ struct Gen {
     bool f32;
     bool split;   // remaps move real parts, then imaginary parts, through an LDS tile of scalars
     std::string V, T;
+    const char *ld = "hgm_ld", *st = "hgm_st";   // state accessors (state_access)
 
     double round(double v) const { return f32 ? (double)(float)v : v; }
 
@@ -109,13 +110,12 @@ uint32_t unswizzle(uint32_t x) { return x ^ ((x >> 4) & 15u) ^ ((x >> 8) & 15u) 
 // per-thread part plus a per-register constant (an immediate offset).
 uint32_t padded(uint32_t x) { return x + (x >> 4) + (x >> 8); }
 
-// Amplitude types of the generated kernels and their state accessors. A pass
-// of the plan-compiled kernels reads and writes every amplitude once and
-// nothing re-reads it before the next pass: their loads and stores carry the
-// nontemporal (streaming) hint (random30 FP64 99.4-99.9 -> 96.7-97.1 ms per
-// step, random32 FP32 221 -> 215 ms, on one box). The serving kernels do not:
-// with the hint the mix served 1086-1089 against 1093 circuits/s, and with it
-// on states above 256 MiB only (26 qubits) 1066-1068 against 1088-1090.
+// Amplitude types of the generated kernels and their state accessors: with
+// the nontemporal (streaming) hint (hgm_ld, hgm_st) and without (hgm_ldp,
+// hgm_stp); state_access chooses for the plan-compiled kernels. The serving
+// kernels use plain accesses: with the hint the mix served 1086-1089 against
+// 1093 circuits/s, and with it on states above 256 MiB only (26 qubits)
+// 1066-1068 against 1088-1090.
 const char *const kAmpTypes =
     "struct __attribute__((aligned(16))) hgm_d2 { double x, y; };\n"
     "struct __attribute__((aligned(8))) hgm_f2 { float x, y; };\n"
@@ -128,7 +128,27 @@ const char *const kAmpTypes =
     "__device__ inline void hgm_st(hgm_d2 *p, hgm_d2 a) {\n"
     "    hgm_v2d v = {a.x, a.y}; __builtin_nontemporal_store(v, (hgm_v2d *)p); }\n"
     "__device__ inline void hgm_st(hgm_f2 *p, hgm_f2 a) {\n"
-    "    hgm_v2f v = {a.x, a.y}; __builtin_nontemporal_store(v, (hgm_v2f *)p); }\n";
+    "    hgm_v2f v = {a.x, a.y}; __builtin_nontemporal_store(v, (hgm_v2f *)p); }\n"
+    "template <class V> __device__ inline V hgm_ldp(const V *p) { return *p; }\n"
+    "template <class V> __device__ inline void hgm_stp(V *p, V a) { *p = a; }\n";
+
+// How a pass of a plan-compiled plan reads and writes a state of `bytes`
+// bytes. Nothing re-reads an amplitude before the next pass, so what matters
+// is where the state lies between passes. 64-256 MiB: in the 256 MiB
+// last-level cache, which the hint keeps it out of (FP64 Grover, 24
+// iterations: 22 qubits 2537 -> 2057 us, 24 qubits 10340 -> 8002; random
+// layers of depth 6 at 24 qubits 478 -> 443). Larger: in HBM, where the hint
+// is worth 3-5% (26 qubits 41.3 against 42.7 ms). 16-32 MiB: about the 32 MiB
+// of the eight L2s, whose dirty lines every kernel boundary writes back; with
+// the hint they leave early (20 qubits 642 against 738 us). Up to 8 MiB plain
+// loads hit the L2s (16 qubits 305 -> 273 us), and the stores keep the hint
+// (20 qubits FP32, 8 MiB: 572 us; stores plain too 607; both with the hint 587).
+void state_access(size_t bytes, const char **ld, const char **st) {
+    const size_t mib = size_t(1) << 20;
+    const bool cached = bytes >= 64 * mib && bytes <= 256 * mib;
+    *ld = cached || bytes <= 8 * mib ? "hgm_ldp" : "hgm_ld";
+    *st = cached ? "hgm_stp" : "hgm_st";
+}
 
 // base = deposit of the tile id into the non-local state bits, by runs
 std::string base_expr(uint64_t nonlocal) {
@@ -331,7 +351,7 @@ std::string kernel_body(const Gen &g, const Plan &plan, const Pass &ps, const st
     o += "        const unsigned long long tid = blockIdx.x;\n";
     o += "        const unsigned long long base = " + base_expr(nonlocal) + ";\n";
     for (int k = 0; k < A; ++k)
-        o += "        " + g.V + " " + reg(k) + " = hgm_ld(&s[(base | " + hex64(pm.lreg[k]) + ") + lt]);\n";
+        o += "        " + g.V + " " + reg(k) + " = " + g.ld + "(&s[(base | " + hex64(pm.lreg[k]) + ") + lt]);\n";
     int cur = m_first;
     std::vector<RegOp> ops(plan.rops.begin() + ps.rop_begin, plan.rops.begin() + ps.rop_begin + ps.rop_count);
     schedule_waves(ops);
@@ -424,7 +444,7 @@ std::string kernel_body(const Gen &g, const Plan &plan, const Pass &ps, const st
     flush_factors();
     flush_scales();
     for (int k = 0; k < A; ++k)
-        o += "        hgm_st(&s[(base | " + hex64(pm.sreg[k]) + ") + st], " + reg(k) + ");\n";
+        o += std::string("        ") + g.st + "(&s[(base | " + hex64(pm.sreg[k]) + ") + st], " + reg(k) + ");\n";
     o += "    }\n}\n";
     return o;
 }
@@ -480,6 +500,7 @@ void jit_generate(const Plan &plan, JitCode *out) {
     const uint64_t last = (uint64_t(1) << plan.shape.r) - 1;
     const size_t entries = (size_t)padded((uint32_t)last) + 1;
     g.split = entries * amp_bytes(plan.dtype) > 32 * 1024;
+    state_access((size_t(1) << plan.qubits) * amp_bytes(plan.dtype), &g.ld, &g.st);
     out->lds_bytes = entries * amp_bytes(plan.dtype) / (g.split ? 2 : 1);
     out->source = std::string("// generated pass kernels\n") + kAmpTypes;
     out->pass_kernel.clear();
