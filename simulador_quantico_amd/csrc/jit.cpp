@@ -41,7 +41,7 @@ struct Gen {
     bool f32;
     bool split;   // remaps move real parts, then imaginary parts, through an LDS tile of scalars
     std::string V, T;
-    const char *ld = "hgm_ld", *st = "hgm_st";   // state accessors (state_access)
+    const char *ld = "hgm_ld", *st = "hgm_st";   // state accessors (state_streams)
 
     double round(double v) const { return f32 ? (double)(float)v : v; }
 
@@ -112,7 +112,7 @@ uint32_t padded(uint32_t x) { return x + (x >> 4) + (x >> 8); }
 
 // Amplitude types of the generated kernels and their state accessors: with
 // the nontemporal (streaming) hint (hgm_ld, hgm_st) and without (hgm_ldp,
-// hgm_stp); state_access chooses for the plan-compiled kernels. The serving
+// hgm_stp); state_streams chooses for the plan-compiled kernels. The serving
 // kernels use plain accesses: with the hint the mix served 1086-1089 against
 // 1093 circuits/s, and with it on states above 256 MiB only (26 qubits)
 // 1066-1068 against 1088-1090.
@@ -131,24 +131,6 @@ const char *const kAmpTypes =
     "    hgm_v2f v = {a.x, a.y}; __builtin_nontemporal_store(v, (hgm_v2f *)p); }\n"
     "template <class V> __device__ inline V hgm_ldp(const V *p) { return *p; }\n"
     "template <class V> __device__ inline void hgm_stp(V *p, V a) { *p = a; }\n";
-
-// How a pass of a plan-compiled plan reads and writes a state of `bytes`
-// bytes. Nothing re-reads an amplitude before the next pass, so what matters
-// is where the state lies between passes. 64-256 MiB: in the 256 MiB
-// last-level cache, which the hint keeps it out of (FP64 Grover, 24
-// iterations: 22 qubits 2537 -> 2057 us, 24 qubits 10340 -> 8002; random
-// layers of depth 6 at 24 qubits 478 -> 443). Larger: in HBM, where the hint
-// is worth 3-5% (26 qubits 41.3 against 42.7 ms). 16-32 MiB: about the 32 MiB
-// of the eight L2s, whose dirty lines every kernel boundary writes back; with
-// the hint they leave early (20 qubits 642 against 738 us). Up to 8 MiB plain
-// loads hit the L2s (16 qubits 305 -> 273 us), and the stores keep the hint
-// (20 qubits FP32, 8 MiB: 572 us; stores plain too 607; both with the hint 587).
-void state_access(size_t bytes, const char **ld, const char **st) {
-    const size_t mib = size_t(1) << 20;
-    const bool cached = bytes >= 64 * mib && bytes <= 256 * mib;
-    *ld = cached || bytes <= 8 * mib ? "hgm_ldp" : "hgm_ld";
-    *st = cached ? "hgm_stp" : "hgm_st";
-}
 
 // base = deposit of the tile id into the non-local state bits, by runs
 std::string base_expr(uint64_t nonlocal) {
@@ -255,65 +237,9 @@ void emit_factor(const Gen &g, std::string &o, double fr, double fi, int k) {
 
 void emit_phase(const Gen &g, std::string &o, const RegOp &op, int k) { emit_factor(g, o, op.m[0], op.m[1], k); }
 
-bool is_phase(const RegOp &o) { return o.kind == R_PHASE || o.kind == R_PHASE_REAL; }
-
 // A phase that tests register bits only: its factor per register slot is a
 // constant of the generated code.
 bool slot_phase(const RegOp &o) { return is_phase(o) && !o.tmask && !o.gmask; }
-
-// Whether two register-program ops commute: phases always do; a phase and a
-// gate on register bit b do when the phase does not depend on b; two gates do
-// when their register bits differ and neither tests the other's bit.
-bool commute(const RegOp &a, const RegOp &b) {
-    const bool pa = is_phase(a), pb = is_phase(b);
-    if (pa && pb) return true;
-    if (pa) return !((a.rmask >> b.rbit) & 1);
-    if (pb) return !((b.rmask >> a.rbit) & 1);
-    return a.rbit != b.rbit && !((a.rmask >> b.rbit) & 1) && !((b.rmask >> a.rbit) & 1);
-}
-
-// Reorders the ops between two remaps into waves: every phase whose
-// predecessors (the earlier ops it does not commute with) are done, then
-// every gate whose predecessors are done, and again. The phases in front of
-// a wave of rotations then form one run, and a run costs one multiply per
-// register slot. The order stays a topological order of the non-commuting
-// pairs, so the product is unchanged.
-void schedule_waves(std::vector<RegOp> &ops) {
-    size_t a = 0;
-    while (a < ops.size()) {
-        size_t b = a;
-        while (b < ops.size() && ops[b].kind != R_REMAP) ++b;
-        const size_t n = b - a;
-        if (n > 2) {
-            std::vector<std::vector<uint32_t>> succ(n);
-            std::vector<uint32_t> preds(n, 0);
-            for (size_t i = 0; i < n; ++i)
-                for (size_t j = i + 1; j < n; ++j)
-                    if (!commute(ops[a + i], ops[a + j])) { succ[i].push_back((uint32_t)j); ++preds[j]; }
-            std::vector<RegOp> out;
-            out.reserve(n);
-            std::vector<char> done(n, 0);
-            size_t emitted = 0;
-            while (emitted < n) {
-                for (int want_phase = 1; want_phase >= 0; --want_phase) {
-                    bool again = true;
-                    while (again) {
-                        again = false;
-                        for (size_t i = 0; i < n; ++i) {
-                            if (done[i] || preds[i] || is_phase(ops[a + i]) != (want_phase == 1)) continue;
-                            done[i] = 1;
-                            ++emitted;
-                            out.push_back(ops[a + i]);
-                            for (uint32_t j : succ[i]) if (--preds[j] == 0 && j < i) again = true;
-                        }
-                    }
-                }
-            }
-            std::copy(out.begin(), out.end(), ops.begin() + a);
-        }
-        a = b + 1;
-    }
-}
 
 std::string kernel_body(const Gen &g, const Plan &plan, const Pass &ps, const std::string &name) {
     const int r = plan.shape.r, B = plan.shape.B, A = 2 * plan.shape.R;
@@ -500,7 +426,10 @@ void jit_generate(const Plan &plan, JitCode *out) {
     const uint64_t last = (uint64_t(1) << plan.shape.r) - 1;
     const size_t entries = (size_t)padded((uint32_t)last) + 1;
     g.split = entries * amp_bytes(plan.dtype) > 32 * 1024;
-    state_access((size_t(1) << plan.qubits) * amp_bytes(plan.dtype), &g.ld, &g.st);
+    bool ld, st;
+    state_streams((size_t(1) << plan.qubits) * amp_bytes(plan.dtype), &ld, &st);
+    if (!ld) g.ld = "hgm_ldp";
+    if (!st) g.st = "hgm_stp";
     out->lds_bytes = entries * amp_bytes(plan.dtype) / (g.split ? 2 : 1);
     out->source = std::string("// generated pass kernels\n") + kAmpTypes;
     out->pass_kernel.clear();

@@ -9,6 +9,7 @@
 // pair-mixing gate it takes pairs t + k*B (k < R) and inserts a zero at the
 // target's tile bit. Barriers are placed only where ownership changes.
 #include "kernels.hpp"
+#include "program.hpp"
 
 #include <type_traits>
 
@@ -156,286 +157,295 @@ __global__ void __launch_bounds__(1024) k_pass_lds(typename Vec<T>::type *__rest
 
 // ---------------------------------------------------------------------------
 // k_pass_reg: the register kernel. Each thread keeps A amplitudes of its tile
-// in registers for the whole pass. Gates act on register pairs only (the
-// planner's second level schedules them in phases); between phases the tile
-// makes one round trip through LDS into the next phase's bit assignment.
-// HBM traffic per pass: one read and one write of every amplitude.
+// in registers for the whole pass and runs the pass's program (program.hpp):
+// gates act on register pairs, between stages the tile makes one round trip
+// through LDS. HBM traffic per pass: one read and one write of every
+// amplitude.
 //
-// Every per-gate condition is resolved by selecting the operator, never by
-// branching per amplitude: a register-bit condition picks the matrix or the
-// identity per register pair (tile-uniform, scalar selects), a thread-bit
-// condition picks it per lane once per gate; the updates themselves are
-// straight-line FMA code.
+// What an interpreted gate costs beyond its multiply-adds is issue slots, so
+// the program leaves nothing to work out per amplitude: a condition on tile
+// bits skips the record (scalar), one on thread bits masks lanes (one
+// divergent branch, no selected matrices), one on register bits is a mask of
+// pairs; phases are gathered per lane and applied once per group; the next
+// record's scalar loads are in flight while a record runs. A remap writes to
+// the LDS slots the thread itself read last, so it needs one barrier, and none
+// where a tile lies within a wave.
 
-template <class T> struct Mat {
-    T m0r, m0i, m1r, m1i, m2r, m2i, m3r, m3i;
-};
-
-template <class T>
-__device__ __forceinline__ Mat<T> load_mat(const RegOp &o) {
-    return {(T)o.m[0], (T)o.m[1], (T)o.m[2], (T)o.m[3], (T)o.m[4], (T)o.m[5], (T)o.m[6], (T)o.m[7]};
-}
-
-template <class T>
-__device__ __forceinline__ Mat<T> or_identity(const Mat<T> &m, bool id) {
-    return {id ? T(1) : m.m0r, id ? T(0) : m.m0i, id ? T(0) : m.m1r, id ? T(0) : m.m1i,
-            id ? T(0) : m.m2r, id ? T(0) : m.m2i, id ? T(1) : m.m3r, id ? T(0) : m.m3i};
-}
-
-template <class T, int A, int BIT, bool COND>
-__device__ __forceinline__ void reg_dense(typename Vec<T>::type (&a)[A], const Mat<T> &m, uint32_t rmask,
-                                          uint32_t rval) {
+template <class T, int KIND>
+__device__ __forceinline__ void pair_update(typename Vec<T>::type &x, typename Vec<T>::type &y, const T (&m)[8]) {
     using V = typename Vec<T>::type;
-#pragma unroll
-    for (int k0 = 0; k0 < A; ++k0) {
-        if (k0 & (1 << BIT)) continue;
-        const int k1 = k0 | (1 << BIT);
-        const Mat<T> u = COND ? or_identity(m, ((uint32_t)k0 & rmask) != rval) : m;
-        const V x = a[k0], y = a[k1];
-        a[k0] = cmul2<V, T>(u.m0r, u.m0i, x, u.m1r, u.m1i, y);
-        a[k1] = cmul2<V, T>(u.m2r, u.m2i, x, u.m3r, u.m3i, y);
+    const V p = x, q = y;
+    if constexpr (KIND == X_DENSE) {
+        x = cmul2<V, T>(m[0], m[1], p, m[2], m[3], q);
+        y = cmul2<V, T>(m[4], m[5], p, m[6], m[7], q);
+    } else if constexpr (KIND == X_DENSE_REAL) {
+        x.x = m[0] * p.x + m[2] * q.x;
+        x.y = m[0] * p.y + m[2] * q.y;
+        y.x = m[4] * p.x + m[6] * q.x;
+        y.y = m[4] * p.y + m[6] * q.y;
+    } else {
+        static_assert(KIND == X_ROT);
+        x.x = p.x + m[0] * q.x;
+        x.y = p.y + m[0] * q.y;
+        y.x = q.x + m[1] * p.x;
+        y.y = q.y + m[1] * p.y;
     }
 }
 
-// Real 2x2 matrix (imaginary parts zero): half the multiply-adds of reg_dense.
-template <class T, int A, int BIT, bool COND>
-__device__ __forceinline__ void reg_dense_real(typename Vec<T>::type (&a)[A], const Mat<T> &m, uint32_t rmask,
-                                               uint32_t rval) {
-    using V = typename Vec<T>::type;
+// Gates under a condition resolve it by selection: the matrix or the identity
+// per lane (once per gate) and per pair.
+template <class T, int A, int KIND, int BIT>
+__device__ __forceinline__ void gate_bit(typename Vec<T>::type (&a)[A], const T (&m)[8], bool lane, uint32_t pmask) {
+    constexpr bool kMask = KIND == X_DENSE_MASK || KIND == X_REAL_MASK;
+    constexpr bool kCond = kMask || KIND == X_DENSE_LANE || KIND == X_REAL_LANE;
+    constexpr bool kReal = KIND == X_REAL_LANE || KIND == X_REAL_MASK;
+    T u[8];
+    if constexpr (kCond) {
 #pragma unroll
-    for (int k0 = 0; k0 < A; ++k0) {
-        if (k0 & (1 << BIT)) continue;
-        const int k1 = k0 | (1 << BIT);
-        const bool id = COND && (((uint32_t)k0 & rmask) != rval);
-        const T u0 = id ? T(1) : m.m0r, u1 = id ? T(0) : m.m1r, u2 = id ? T(0) : m.m2r, u3 = id ? T(1) : m.m3r;
-        const V x = a[k0], y = a[k1];
-        V p, q;
-        p.x = u0 * x.x + u1 * y.x;
-        p.y = u0 * x.y + u1 * y.y;
-        q.x = u2 * x.x + u3 * y.x;
-        q.y = u2 * x.y + u3 * y.y;
-        a[k0] = p;
-        a[k1] = q;
+        for (int e = 0; e < 8; ++e) u[e] = lane ? m[e] : T(e == 0 || e == 6 ? 1 : 0);
     }
-}
-
-// dispatch on the runtime register bit (tile-uniform) to unrolled code. With
-// STRICT, the cases no bit can reach (the planner emits register bits below
-// log2(A) only) are marked unreachable: every remaining case then updates the
-// amplitudes in place, and the compiler stops copying them to a second
-// register set per gate, for a few more VGPRs (used by the batched kernel,
-// whose register budget allows it)
-#define HGM_NO_CASE                               \
-    if constexpr (STRICT) __builtin_unreachable(); \
-    break;
-#define HGM_REG_BITS(CALL)                                             \
-    switch (bit) {                                                     \
-        case 0: CALL(0); break;                                        \
-        case 1: if constexpr (A > 2) { CALL(1); break; } HGM_NO_CASE   \
-        case 2: if constexpr (A > 4) { CALL(2); break; } HGM_NO_CASE   \
-        case 3: if constexpr (A > 8) { CALL(3); break; } HGM_NO_CASE   \
-        case 4: if constexpr (A > 16) { CALL(4); break; } HGM_NO_CASE  \
-        default: HGM_NO_CASE                                           \
-    }
-
-// Rows with an exact unit entry (R_DENSE_PIV*): out_i = x[P_i] + t_i * x[1 - P_i],
-// 8 multiply-adds per pair, 4 when t0 and t1 are real.
-template <class T, int A, int BIT, int P0, int P1, bool REAL>
-__device__ __forceinline__ void reg_dense_piv(typename Vec<T>::type (&a)[A], T t0r, T t0i, T t1r, T t1i) {
-    using V = typename Vec<T>::type;
 #pragma unroll
-    for (int k0 = 0; k0 < A; ++k0) {
-        if (k0 & (1 << BIT)) continue;
-        const int k1 = k0 | (1 << BIT);
-        const V x[2] = {a[k0], a[k1]};
-        V p, q;
-        if constexpr (REAL) {
-            p.x = x[P0].x + t0r * x[1 - P0].x;
-            p.y = x[P0].y + t0r * x[1 - P0].y;
-            q.x = x[P1].x + t1r * x[1 - P1].x;
-            q.y = x[P1].y + t1r * x[1 - P1].y;
+    for (int k = 0; k < A; ++k) {
+        if (k & (1 << BIT)) continue;
+        typename Vec<T>::type &x = a[k], &y = a[k | (1 << BIT)];
+        if constexpr (KIND == X_SWAP) {
+            const typename Vec<T>::type p = x;
+            x.x = lane ? y.x : p.x;
+            x.y = lane ? y.y : p.y;
+            y.x = lane ? p.x : y.x;
+            y.y = lane ? p.y : y.y;
+        } else if constexpr (kMask) {
+            const bool on = (pmask >> k) & 1u;
+            T w[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) w[e] = on ? u[e] : T(e == 0 || e == 6 ? 1 : 0);
+            pair_update<T, kReal ? X_DENSE_REAL : X_DENSE>(x, y, w);
+        } else if constexpr (kCond) {
+            pair_update<T, kReal ? X_DENSE_REAL : X_DENSE>(x, y, u);
         } else {
-            p.x = x[P0].x + t0r * x[1 - P0].x - t0i * x[1 - P0].y;
-            p.y = x[P0].y + t0r * x[1 - P0].y + t0i * x[1 - P0].x;
-            q.x = x[P1].x + t1r * x[1 - P1].x - t1i * x[1 - P1].y;
-            q.y = x[P1].y + t1r * x[1 - P1].y + t1i * x[1 - P1].x;
+            pair_update<T, KIND>(x, y, m);
         }
-        a[k0] = p;
-        a[k1] = q;
     }
 }
 
-template <class T, int A, int P0, int P1, bool REAL, bool STRICT>
-__device__ __forceinline__ void reg_dense_piv_bits(typename Vec<T>::type (&a)[A], int bit, T t0r, T t0i, T t1r,
-                                                   T t1i) {
-#define HGM_CALL(B) reg_dense_piv<T, A, B, P0, P1, REAL>(a, t0r, t0i, t1r, t1i)
-    HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-}
-
-template <class T, int A, bool REAL, bool STRICT>
-__device__ __forceinline__ void reg_dense_piv_any(typename Vec<T>::type (&a)[A], const RegOp &o) {
-    const T t0r = (T)o.m[0], t0i = (T)o.m[1], t1r = (T)o.m[2], t1i = (T)o.m[3];
-    switch (o.tval & 3u) {
-        case 0: reg_dense_piv_bits<T, A, 0, 0, REAL, STRICT>(a, o.rbit, t0r, t0i, t1r, t1i); break;
-        case 1: reg_dense_piv_bits<T, A, 1, 0, REAL, STRICT>(a, o.rbit, t0r, t0i, t1r, t1i); break;
-        case 2: reg_dense_piv_bits<T, A, 0, 1, REAL, STRICT>(a, o.rbit, t0r, t0i, t1r, t1i); break;
-        default: reg_dense_piv_bits<T, A, 1, 1, REAL, STRICT>(a, o.rbit, t0r, t0i, t1r, t1i); break;
+// Dispatch on the runtime register bit (wave-uniform) to unrolled code; bits
+// at log2(A) and above do not occur.
+template <class T, int A, int KIND>
+__device__ __forceinline__ void gate(typename Vec<T>::type (&a)[A], const T (&m)[8], int bit, bool lane = true,
+                                     uint32_t pmask = 0) {
+    switch (bit) {
+        case 0: gate_bit<T, A, KIND, 0>(a, m, lane, pmask); break;
+        case 1: if constexpr (A > 2) { gate_bit<T, A, KIND, 1>(a, m, lane, pmask); break; } __builtin_unreachable();
+        case 2: if constexpr (A > 4) { gate_bit<T, A, KIND, 2>(a, m, lane, pmask); break; } __builtin_unreachable();
+        case 3: if constexpr (A > 8) { gate_bit<T, A, KIND, 3>(a, m, lane, pmask); break; } __builtin_unreachable();
+        case 4: if constexpr (A > 16) { gate_bit<T, A, KIND, 4>(a, m, lane, pmask); break; } __builtin_unreachable();
+        default: __builtin_unreachable();
     }
 }
 
-template <class T, int A, int BIT>
-__device__ __forceinline__ void reg_anti(typename Vec<T>::type (&a)[A], const Mat<T> &m) {
-    using V = typename Vec<T>::type;
+// Multiplies the registers k with (k & BITS) == VAL by the lane's factor.
+template <class T, int A, int BITS, int VAL>
+__device__ __forceinline__ void phase_on(typename Vec<T>::type (&a)[A], T fr, T fi, bool real) {
+    if constexpr (BITS < A) {
+        if (real) {
 #pragma unroll
-    for (int k0 = 0; k0 < A; ++k0) {
-        if (k0 & (1 << BIT)) continue;
-        const int k1 = k0 | (1 << BIT);
-        const V x = a[k0], y = a[k1];
-        a[k0] = cmul<V, T>(m.m1r, m.m1i, y);
-        a[k1] = cmul<V, T>(m.m2r, m.m2i, x);
-    }
-}
-
-template <class T, int A, int BIT>
-__device__ __forceinline__ void reg_swap(typename Vec<T>::type (&a)[A]) {
-    using V = typename Vec<T>::type;
-#pragma unroll
-    for (int k0 = 0; k0 < A; ++k0) {
-        if (k0 & (1 << BIT)) continue;
-        const int k1 = k0 | (1 << BIT);
-        const V x = a[k0];
-        a[k0] = a[k1];
-        a[k1] = x;
-    }
-}
-
-template <class T, int A, bool STRICT>
-__device__ __forceinline__ void reg_gate(typename Vec<T>::type (&a)[A], const RegOp &o, int t) {
-    const int bit = o.rbit;
-    if (o.kind == R_DENSE_PIV) { reg_dense_piv_any<T, A, false, STRICT>(a, o); return; }
-    if (o.kind == R_DENSE_PIV_REAL) { reg_dense_piv_any<T, A, true, STRICT>(a, o); return; }
-    if (o.kind == R_SWAP) {
-#define HGM_CALL(B) reg_swap<T, A, B>(a)
-        HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-        return;
-    }
-    Mat<T> m = load_mat<T>(o);
-    if (o.kind == R_ANTI) {
-#define HGM_CALL(B) reg_anti<T, A, B>(a, m)
-        HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-        return;
-    }
-    if (o.kind == R_DENSE_REAL) {
-        if (o.tmask) m = or_identity(m, ((uint32_t)t & o.tmask) != o.tval);   // per lane, once per gate
-        if (o.rmask) {
-#define HGM_CALL(B) reg_dense_real<T, A, B, true>(a, m, o.rmask, o.rval)
-            HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
+            for (int k = 0; k < A; ++k)
+                if ((k & BITS) == VAL) { a[k].x *= fr; a[k].y *= fr; }
         } else {
-#define HGM_CALL(B) reg_dense_real<T, A, B, false>(a, m, 0u, 0u)
-            HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-        }
-        return;
-    }
-    if (o.tmask == 0) {   // tile-uniform matrix (scalar registers)
-        if (o.rmask) {
-#define HGM_CALL(B) reg_dense<T, A, B, true>(a, m, o.rmask, o.rval)
-            HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-        } else {
-#define HGM_CALL(B) reg_dense<T, A, B, false>(a, m, 0u, 0u)
-            HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-        }
-        return;
-    }
-    m = or_identity(m, ((uint32_t)t & o.tmask) != o.tval);   // per lane, once per gate
-#define HGM_CALL(B) reg_dense<T, A, B, true>(a, m, o.rmask, o.rval)
-    HGM_REG_BITS(HGM_CALL)
-#undef HGM_CALL
-}
-
-template <class T, int A>
-__device__ __forceinline__ void reg_phase_apply(typename Vec<T>::type (&a)[A], T fr, T fi, bool real,
-                                                uint32_t rmask, uint32_t rval) {
-    if (real) {
 #pragma unroll
-        for (int k = 0; k < A; ++k) {
-            const T fk = (((uint32_t)k & rmask) == rval) ? fr : T(1);
-            a[k].x *= fk;
-            a[k].y *= fk;
+            for (int k = 0; k < A; ++k)
+                if ((k & BITS) == VAL) a[k] = cmul<typename Vec<T>::type, T>(fr, fi, a[k]);
         }
     } else {
+        __builtin_unreachable();
+    }
+}
+
+template <class T, int A>
+__device__ __forceinline__ void phase_apply(typename Vec<T>::type (&a)[A], T fr, T fi, bool real, uint32_t pat,
+                                            uint32_t pmask) {
+#define HGM_SET(S) case S: phase_on<T, A, S, S>(a, fr, fi, real); break;
+#define HGM_CLEAR(B) case X_PAT_CLEAR + B: phase_on<T, A, (1 << B), 0>(a, fr, fi, real); break;
+    switch (pat) {   // one or two register bits set: the phases of controlled phase gates
+        HGM_CLEAR(0) HGM_CLEAR(1) HGM_CLEAR(2) HGM_CLEAR(3) HGM_CLEAR(4)
+        HGM_SET(0) HGM_SET(1) HGM_SET(2) HGM_SET(3) HGM_SET(4) HGM_SET(5) HGM_SET(6) HGM_SET(8) HGM_SET(9)
+        HGM_SET(10) HGM_SET(12) HGM_SET(16) HGM_SET(17) HGM_SET(18) HGM_SET(20) HGM_SET(24)
+        default:
 #pragma unroll
-        for (int k = 0; k < A; ++k) {
-            const bool hit = ((uint32_t)k & rmask) == rval;
-            a[k] = cmul<typename Vec<T>::type, T>(hit ? fr : T(1), hit ? fi : T(0), a[k]);
+            for (int k = 0; k < A; ++k) {
+                const bool on = (pmask >> k) & 1u;
+                a[k] = cmul<typename Vec<T>::type, T>(on ? fr : T(1), on ? fi : T(0), a[k]);
+            }
+    }
+#undef HGM_SET
+#undef HGM_CLEAR
+}
+
+// Rotations on every register bit (up to 4), one after the other in straight
+// line: one record, and one settling of the registers, for a layer of gates.
+template <class T, int A>
+__device__ __forceinline__ void rotations(typename Vec<T>::type (&a)[A], const T (&m)[8]) {
+#pragma unroll
+    for (int b = 0; b < 4 && (2 << b) <= A; ++b) {
+        const T u[8] = {m[2 * b], m[2 * b + 1]};
+#pragma unroll
+        for (int k = 0; k < A; ++k)
+            if (!((k >> b) & 1)) pair_update<T, X_ROT>(a[k], a[k | (1 << b)], u);
+    }
+}
+
+// Thread part of an LDS slot, in bytes: the thread index with a zero at every
+// register bit, swizzled.
+template <class T, int A>
+__device__ __forceinline__ uint32_t lds_pos(uint32_t t, const XMap &m) {
+    constexpr int L = A == 2 ? 1 : A == 4 ? 2 : A == 8 ? 3 : A == 16 ? 4 : 5;
+    uint32_t x = t;
+#pragma unroll
+    for (int i = 0; i < L; ++i) x += x & ~(uint32_t)m.low[i];
+    x = x_swizzle<sizeof(T) == 4 ? 5 : 4>(x) * (uint32_t)sizeof(typename Vec<T>::type);
+    asm("" : "+v"(x));   // keeps the scaling here, once, instead of after the XOR with each register's part
+    return x;
+}
+
+template <class T, int A>
+__device__ __forceinline__ uint32_t lds_reg(int k, const XMap &m) {
+    uint32_t x = 0;
+#pragma unroll
+    for (int i = 0; (1 << i) < A; ++i)
+        if ((k >> i) & 1) x ^= m.sw[i];
+    return x * (uint32_t)sizeof(typename Vec<T>::type);
+}
+
+__device__ __forceinline__ uint64_t run_bits(uint64_t v, const XRun &r) {
+    return ((v >> r.from) & r.mask) << r.to;
+}
+
+// Deposit of v by runs; most deposits have up to 4, whose loads go out together.
+__device__ __forceinline__ uint64_t deposit(uint64_t v, const XRun *__restrict__ runs, int n) {
+    uint64_t x = run_bits(v, runs[0]) | run_bits(v, runs[1]) | run_bits(v, runs[2]) | run_bits(v, runs[3]);
+    for (int i = 4; i < n; ++i) x |= run_bits(v, runs[i]);
+    return x;
+}
+
+template <int A>
+__device__ __forceinline__ uint64_t reg_bits(int k, const uint64_t *__restrict__ bit, uint64_t flip) {
+#pragma unroll
+    for (int i = 0; (1 << i) < A; ++i)
+        if ((k >> i) & 1) flip ^= bit[i];
+    return flip;
+}
+
+// Runs the records of a pass on the registers of one tile.
+template <class T, int A>
+__device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const XPass *__restrict__ xp, uint64_t base,
+                                            unsigned char *lds, bool sync) {
+    using V = typename Vec<T>::type;
+    const uint32_t t = threadIdx.x;
+    const XOp<T> *__restrict__ ops = reinterpret_cast<const XOp<T> *>(xp + 1);
+    const T *__restrict__ table = reinterpret_cast<const T *>(reinterpret_cast<const char *>(xp) + xp->table);
+    const int n = xp->n_ops;
+    XMap cur = xp->first;
+    uint32_t pos = lds_pos<T, A>(t, cur);
+    T fr = T(1), fi = T(0);
+    XOp<T> next = ops[0];
+    for (int i = 0; i < n; ++i) {
+        const XOp<T> o = next;
+        next = ops[i + 1];   // the program ends with a spare record
+        if (o.kind == X_REMAP) {
+            XMap to;
+            __builtin_memcpy(&to, o.m, sizeof to);
+#pragma unroll
+            for (int k = 0; k < A; ++k) *reinterpret_cast<V *>(lds + (pos ^ lds_reg<T, A>(k, cur))) = a[k];
+            if (sync) __syncthreads();
+            else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            pos = lds_pos<T, A>(t, to);
+#pragma unroll
+            for (int k = 0; k < A; ++k) a[k] = *reinterpret_cast<const V *>(lds + (pos ^ lds_reg<T, A>(k, to)));
+            cur = to;
+            continue;
+        }
+        const bool tile = (base & o.gmask) == o.gval;
+        if (o.kind == X_PHASE) {
+            if (!tile && (o.flags & (X_FIRST | X_LAST)) == (X_FIRST | X_LAST)) continue;
+            const bool on = tile && (t & o.tmask) == o.tval;
+            const T gr = on ? o.m[0] : T(1), gi = on ? o.m[1] : T(0);
+            if (o.flags & X_FIRST) {
+                fr = gr;
+                fi = gi;
+            } else if (o.flags & X_REAL) {
+                fr *= gr;
+            } else {
+                const T r = fr * gr - fi * gi;
+                fi = fr * gi + fi * gr;
+                fr = r;
+            }
+            if (o.flags & X_LAST) phase_apply<T, A>(a, fr, fi, (o.flags & X_REAL) != 0, o.pat, o.pmask);
+            continue;
+        }
+        if (!tile) continue;
+        const bool lane = (t & o.tmask) == o.tval;
+        switch (o.kind) {
+            case X_ROTS: rotations<T, A>(a, o.m); break;
+            case X_VEC: {
+                const T *__restrict__ f = table + o.pmask;
+#pragma unroll
+                for (int k = 0; k < A; ++k) a[k] = cmul<V, T>(f[2 * k], f[2 * k + 1], a[k]);
+                break;
+            }
+            case X_VEC_REAL: {
+                const T *__restrict__ f = table + o.pmask;
+#pragma unroll
+                for (int k = 0; k < A; ++k) {
+                    a[k].x *= f[k];
+                    a[k].y *= f[k];
+                }
+                break;
+            }
+            case X_ROT: gate<T, A, X_ROT>(a, o.m, o.bit); break;
+            case X_DENSE: gate<T, A, X_DENSE>(a, o.m, o.bit); break;
+            case X_DENSE_REAL: gate<T, A, X_DENSE_REAL>(a, o.m, o.bit); break;
+            case X_SWAP: gate<T, A, X_SWAP>(a, o.m, o.bit, lane); break;
+            case X_DENSE_LANE: gate<T, A, X_DENSE_LANE>(a, o.m, o.bit, lane); break;
+            case X_REAL_LANE: gate<T, A, X_REAL_LANE>(a, o.m, o.bit, lane); break;
+            case X_DENSE_MASK: gate<T, A, X_DENSE_MASK>(a, o.m, o.bit, lane, o.pmask); break;
+            case X_REAL_MASK: gate<T, A, X_REAL_MASK>(a, o.m, o.bit, lane, o.pmask); break;
+            default: __builtin_unreachable();
         }
     }
 }
 
-template <class T, int A>
-__device__ __forceinline__ void reg_phase(typename Vec<T>::type (&a)[A], const RegOp &o, int t) {
-    const bool real = o.kind == R_PHASE_REAL;
-    if (o.tmask == 0) {   // tile-uniform factor (scalar registers)
-        reg_phase_apply<T, A>(a, (T)o.m[0], (T)o.m[1], real, o.rmask, o.rval);
-        return;
-    }
-    const bool lane_ok = ((uint32_t)t & o.tmask) == o.tval;
-    reg_phase_apply<T, A>(a, lane_ok ? (T)o.m[0] : T(1), lane_ok ? (T)o.m[1] : T(0), real, o.rmask, o.rval);
-}
-
-// Moves the tile into another bit assignment through LDS. The maps hold
-// swizzled tile indices (the swizzle is linear, so thread and register parts
-// combine with XOR).
-template <class T, int A>
-__device__ __forceinline__ void reg_remap(typename Vec<T>::type (&a)[A], typename Vec<T>::type *lds,
-                                          const PhaseMap &from, const PhaseMap &to, int t) {
-    __syncthreads();   // the previous users of the LDS tile are done
-    const uint32_t tf = (uint32_t)from.thr[0][t & 31] ^ (uint32_t)from.thr[1][(t >> 5) & 31];
-#pragma unroll
-    for (int k = 0; k < A; ++k) lds[tf ^ (uint32_t)from.reg[k]] = a[k];
-    __syncthreads();
-    const uint32_t tt = (uint32_t)to.thr[0][t & 31] ^ (uint32_t)to.thr[1][(t >> 5) & 31];
-#pragma unroll
-    for (int k = 0; k < A; ++k) a[k] = lds[tt ^ (uint32_t)to.reg[k]];
-}
+// How a pass reads and writes the state, and whether remaps need barriers.
+constexpr uint32_t kStreamLoads = 1, kStreamStores = 2, kBarriers = 4;
 
 template <class T, int A>
-__global__ void __launch_bounds__(reg_kernel_max_threads(A, sizeof(typename Vec<T>::type))) k_pass_reg(typename Vec<T>::type *__restrict__ state,
-                                                   const RegOp *__restrict__ ops, int n_ops,
-                                                   const PhaseMap *__restrict__ maps, const PassMem *__restrict__ pm,
-                                                   uint64_t nonlocal_mask, int64_t n_tiles, int r) {
+__global__ void __launch_bounds__(reg_kernel_max_threads(A, sizeof(typename Vec<T>::type)))
+    k_pass_reg(typename Vec<T>::type *__restrict__ state, const XPass *__restrict__ xp, int64_t n_tiles, uint32_t mode) {
     using V = typename Vec<T>::type;
     extern __shared__ __align__(16) unsigned char smem[];
-    V *lds = reinterpret_cast<V *>(smem);
-    const int t = threadIdx.x;
-    (void)r;
-    const uint64_t lt = pm->lthr[0][t & 31] | pm->lthr[1][(t >> 5) & 31];
-    const uint64_t st = pm->sthr[0][t & 31] | pm->sthr[1][(t >> 5) & 31];
+    const uint32_t t = threadIdx.x;
+    const uint64_t lt = deposit(t, xp->load, xp->n_load);
+    const uint64_t st = deposit(t, xp->store, xp->n_store) ^ xp->sflip;
     for (int64_t tid = blockIdx.x; tid < n_tiles; tid += gridDim.x) {
-        const uint64_t base = pdep64((uint64_t)tid, nonlocal_mask);
+        const uint64_t base = deposit((uint64_t)tid, xp->base, xp->n_base);
         V a[A];
+        const V *src = state + (base | lt);
+        if (mode & kStreamLoads) {
 #pragma unroll
-        for (int k = 0; k < A; ++k) a[k] = load_stream<T>(&state[base | lt | pm->lreg[k]]);
-        int cur = pm->first_map;
-        for (int i = 0; i < n_ops; ++i) {
-            const RegOp &o = ops[i];
-            if (o.kind == R_REMAP) {
-                reg_remap<T, A>(a, lds, maps[cur], maps[o.rbit], t);
-                cur = o.rbit;
-                continue;
-            }
-            if ((base & o.gmask) != o.gval) continue;   // tile-uniform
-            if (o.kind == R_PHASE || o.kind == R_PHASE_REAL) reg_phase<T, A>(a, o, t);
-            else reg_gate<T, A, false>(a, o, t);
+            for (int k = 0; k < A; ++k) a[k] = load_stream<T>(src + reg_bits<A>(k, xp->lbit, 0));
+        } else {
+#pragma unroll
+            for (int k = 0; k < A; ++k) a[k] = src[reg_bits<A>(k, xp->lbit, 0)];
         }
+        run_program<T, A>(a, xp, base, smem, (mode & kBarriers) != 0);
+        V *dst = state + (base | st);
+        if (mode & kStreamStores) {
 #pragma unroll
-        for (int k = 0; k < A; ++k) store_stream<T>(&state[base | st | pm->sreg[k]], a[k]);
+            for (int k = 0; k < A; ++k) store_stream<T>(dst + reg_bits<A>(k, xp->sbit, xp->rflip), a[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < A; ++k) dst[reg_bits<A>(k, xp->sbit, xp->rflip)] = a[k];
+        }
+        if (tid + gridDim.x < n_tiles) __syncthreads();   // the next tile writes LDS slots that others may still read
     }
 }
 
@@ -456,7 +466,6 @@ __global__ void __launch_bounds__(reg_kernel_max_threads(A, sizeof(typename Vec<
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double red_s[16], red_m[16];
     __shared__ uint64_t red_i[16];
-    V *lds = reinterpret_cast<V *>(smem);
     const int t = threadIdx.x;
     const int64_t b = blockIdx.x;
     int lo = 0, hi = n_items - 1;
@@ -466,38 +475,24 @@ __global__ void __launch_bounds__(reg_kernel_max_threads(A, sizeof(typename Vec<
     }
     const BatchItem &it = items[lo];
     V *__restrict__ state = reinterpret_cast<V *>(states + it.state_off);
-    const RegOp *__restrict__ ops = reinterpret_cast<const RegOp *>(progs + it.ops_off);
-    const PhaseMap *__restrict__ maps = reinterpret_cast<const PhaseMap *>(progs + it.maps_off);
-    const PassMem *__restrict__ pm = reinterpret_cast<const PassMem *>(progs + it.pm_off);
-    const int n_ops = it.n_ops;
+    const XPass *__restrict__ xp = reinterpret_cast<const XPass *>(progs + it.xpass_off);
     const int64_t tid = b - it.tile_begin;
-    const uint64_t base = pdep64((uint64_t)tid, it.nonlocal_mask);
-    const uint64_t lt = pm->lthr[0][t & 31] | pm->lthr[1][(t >> 5) & 31];
-    const uint64_t st = pm->sthr[0][t & 31] | pm->sthr[1][(t >> 5) & 31];
+    const uint64_t base = deposit((uint64_t)tid, xp->base, xp->n_base);
+    const uint64_t lt = deposit(t, xp->load, xp->n_load);
     V a[A];
 #pragma unroll
-    for (int k = 0; k < A; ++k) a[k] = state[base | lt | pm->lreg[k]];
-    int cur = pm->first_map;
-    for (int i = 0; i < n_ops; ++i) {
-        const RegOp &o = ops[i];
-        if (o.kind == R_REMAP) {
-            reg_remap<T, A>(a, lds, maps[cur], maps[o.rbit], t);
-            cur = o.rbit;
-            continue;
-        }
-        if ((base & o.gmask) != o.gval) continue;
-        if (o.kind == R_PHASE || o.kind == R_PHASE_REAL) reg_phase<T, A>(a, o, t);
-        else reg_gate<T, A, true>(a, o, t);
-    }
+    for (int k = 0; k < A; ++k) a[k] = state[(base | lt) + reg_bits<A>(k, xp->lbit, 0)];
+    run_program<T, A>(a, xp, base, smem, it.sync != 0);
+    const uint64_t to = base | (deposit(t, xp->store, xp->n_store) ^ xp->sflip);
 #pragma unroll
-    for (int k = 0; k < A; ++k) state[base | st | pm->sreg[k]] = a[k];
+    for (int k = 0; k < A; ++k) state[to + reg_bits<A>(k, xp->sbit, xp->rflip)] = a[k];
     if (it.partials_off < 0) return;
     double sum = 0.0, best = -1.0;
     uint64_t bi = ~uint64_t(0);
 #pragma unroll
     for (int k = 0; k < A; ++k) {
         const double p = (double)a[k].x * (double)a[k].x + (double)a[k].y * (double)a[k].y;
-        const uint64_t idx = base | st | pm->sreg[k];
+        const uint64_t idx = to + reg_bits<A>(k, xp->sbit, xp->rflip);
         sum += p;
         if (p > best || (p == best && idx < bi)) { best = p; bi = idx; }
     }
@@ -748,24 +743,23 @@ hipError_t pass_lds(void *state, const DevOp *ops, int n_ops, const PassArgs &a,
 }
 
 template <class T, int A>
-hipError_t pass_reg(void *state, const RegOp *ops, int n_ops, const PhaseMap *maps, const PassMem *pm,
-                    uint64_t nonlocal, int64_t n_tiles, int r, int B, size_t lds, hipStream_t s) {
+hipError_t pass_reg(void *state, const XPass *xp, int64_t n_tiles, int B, size_t lds, uint32_t mode, hipStream_t s) {
     pass_reg_attr<T, A>();
     const int64_t grid = tile_grid(n_tiles, B);
     hipLaunchKernelGGL((k_pass_reg<T, A>), dim3((unsigned)grid), dim3(B), lds, s,
-                       reinterpret_cast<typename Vec<T>::type *>(state), ops, n_ops, maps, pm, nonlocal, n_tiles, r);
+                       reinterpret_cast<typename Vec<T>::type *>(state), xp, n_tiles, mode);
     return hipGetLastError();
 }
 
 template <class T>
-hipError_t pass_reg_any(int A, void *state, const RegOp *ops, int n_ops, const PhaseMap *maps, const PassMem *pm,
-                        uint64_t nonlocal, int64_t n_tiles, int r, int B, size_t lds, hipStream_t s) {
+hipError_t pass_reg_any(int A, void *state, const XPass *xp, int64_t n_tiles, int B, size_t lds, uint32_t mode,
+                        hipStream_t s) {
     switch (A) {
-        case 2: return pass_reg<T, 2>(state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds, s);
-        case 4: return pass_reg<T, 4>(state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds, s);
-        case 8: return pass_reg<T, 8>(state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds, s);
-        case 16: return pass_reg<T, 16>(state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds, s);
-        case 32: return pass_reg<T, 32>(state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds, s);
+        case 2: return pass_reg<T, 2>(state, xp, n_tiles, B, lds, mode, s);
+        case 4: return pass_reg<T, 4>(state, xp, n_tiles, B, lds, mode, s);
+        case 8: return pass_reg<T, 8>(state, xp, n_tiles, B, lds, mode, s);
+        case 16: return pass_reg<T, 16>(state, xp, n_tiles, B, lds, mode, s);
+        case 32: return pass_reg<T, 32>(state, xp, n_tiles, B, lds, mode, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -798,11 +792,15 @@ hipError_t batch_reg_any(int A, const BatchItem *items, int n_items, int64_t tot
 
 }  // namespace
 
-hipError_t launch_pass_reg(int dtype, int A, void *state, const RegOp *ops, int n_ops, const PhaseMap *maps,
-                           const PassMem *pm, uint64_t nonlocal, int64_t n_tiles, int r, int B, size_t lds_bytes,
+hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, void *state, const XPass *xp, size_t lds_bytes,
                            hipStream_t s) {
-    return dtype == HGM_C64 ? pass_reg_any<float>(A, state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds_bytes, s)
-                            : pass_reg_any<double>(A, state, ops, n_ops, maps, pm, nonlocal, n_tiles, r, B, lds_bytes, s);
+    const size_t bytes = (size_t(1) << qubits) * amp_bytes(dtype);
+    bool ld, st;
+    state_streams(bytes, &ld, &st);
+    const uint32_t mode = (ld ? kStreamLoads : 0) | (st ? kStreamStores : 0) | (e.sync ? kBarriers : 0);
+    const int64_t n_tiles = int64_t(1) << (qubits - e.r);
+    return dtype == HGM_C64 ? pass_reg_any<float>(e.A, state, xp, n_tiles, e.B, lds_bytes, mode, s)
+                            : pass_reg_any<double>(e.A, state, xp, n_tiles, e.B, lds_bytes, mode, s);
 }
 
 hipError_t launch_pass_lds(int dtype, void *state, const DevOp *ops, int n_ops, const PassArgs &a, hipStream_t s) {

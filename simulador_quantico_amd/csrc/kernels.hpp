@@ -8,6 +8,8 @@
 
 namespace hgm {
 
+struct XPass;
+
 // Per-pass launch arguments shared by the pass kernels.
 struct PassArgs {
     uint64_t nonlocal_mask;            // state-index bits that number the tiles
@@ -25,10 +27,10 @@ hipError_t launch_pass_lds(int dtype, void *state, const DevOp *ops, int n_ops, 
 // launches into a graph.
 hipError_t prepare_pass_kernels(int dtype);
 
-// One full-state pass of the register kernel (A amplitudes per thread, B
-// threads per tile of 2^r); lds_bytes is 0 for a pass without remaps.
-hipError_t launch_pass_reg(int dtype, int A, void *state, const RegOp *ops, int n_ops, const PhaseMap *maps,
-                           const PassMem *pm, uint64_t nonlocal, int64_t n_tiles, int r, int B, size_t lds_bytes,
+// One full-state pass of the register kernel: the program at xp (device) on a
+// state of `qubits` qubits in execution shape e; lds_bytes is 0 for a pass of
+// one stage.
+hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, void *state, const XPass *xp, size_t lds_bytes,
                            hipStream_t s);
 
 // Readout of one tile or of a whole state: FP64 sum of |a|^2 and the largest
@@ -47,14 +49,13 @@ static_assert(sizeof(ReadoutPartial) == 32, "shared with the kernels");
 // the compiler sees global memory and reads the programs with scalar loads.
 struct BatchItem {
     uint64_t state_off;          // the state (2^qubits amplitudes)
-    uint64_t ops_off;            // the pass's register program (RegOp[n_ops])
-    uint64_t maps_off;           // the plan's phase maps
-    uint64_t pm_off;             // the pass's load/store table (PassMem)
-    uint64_t nonlocal_mask;      // state-index bits that number the tiles
+    uint64_t ops_off;            // compiled kernels: the pass's register program (RegOp[])
+    uint64_t xpass_off;          // interpreter: the pass's program (XPass, XOp[])
+    uint64_t pad[2];
     int64_t tile_begin;          // first workgroup of this item in the launch
     int64_t partials_off;        // >= 0: per-tile readout of the pass output (ReadoutPartial[])
-    int32_t n_ops;
-    int32_t pad;
+    int32_t sync;                // interpreter: remaps need barriers
+    int32_t pad2;
 };
 static_assert(sizeof(BatchItem) == 64, "shared with the kernels");
 

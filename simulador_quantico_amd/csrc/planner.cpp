@@ -7,6 +7,7 @@
 #include <cstring>
 
 #include "jit.hpp"
+#include "program.hpp"
 
 namespace hgm {
 
@@ -249,6 +250,13 @@ int classify(const double m[8]) {
 }
 
 size_t amp_bytes(int dtype) { return dtype == HGM_C64 ? 8 : 16; }
+
+void state_streams(size_t bytes, bool *loads, bool *stores) {
+    const size_t mib = size_t(1) << 20;
+    const bool cached = bytes >= 64 * mib && bytes <= 256 * mib;
+    *loads = !cached && bytes > 8 * mib;
+    *stores = !cached;
+}
 
 int make_shape(int qubits, int dtype, const hgm_tuning &t, TileShape *out, std::string *err) {
     if (qubits < 1 || qubits > kMaxQubits) {
@@ -882,6 +890,7 @@ int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iter
     if (t.kernel == HGM_KERNEL_REG || t.kernel == HGM_KERNEL_JIT || (t.kernel == HGM_KERNEL_AUTO && reg_ok)) {
         plan.kernel = t.kernel == HGM_KERNEL_JIT ? HGM_KERNEL_JIT : HGM_KERNEL_REG;
         build_register_program(plan);
+        if (plan.kernel == HGM_KERNEL_REG) build_exec_program(plan);
         if (plan.kernel == HGM_KERNEL_JIT) {
             // one workgroup per tile: a dispatch holds at most 2^32 - 1 work-items
             const uint64_t items = (uint64_t(1) << (qubits - plan.shape.r)) * (uint64_t)plan.shape.B;
@@ -983,6 +992,66 @@ bool unit_pivot(const double m[8], int row, int *col) {
 }
 
 }  // namespace
+
+namespace {
+
+// Whether two register-program ops commute: phases always do; a phase and a
+// gate on register bit b do when the phase does not depend on b; two gates do
+// when their register bits differ and neither tests the other's bit.
+bool commute(const RegOp &a, const RegOp &b) {
+    const bool pa = is_phase(a), pb = is_phase(b);
+    if (pa && pb) return true;
+    if (pa) return !((a.rmask >> b.rbit) & 1);
+    if (pb) return !((b.rmask >> a.rbit) & 1);
+    return a.rbit != b.rbit && !((a.rmask >> b.rbit) & 1) && !((b.rmask >> a.rbit) & 1);
+}
+
+}  // namespace
+
+bool is_phase(const RegOp &o) { return o.kind == R_PHASE || o.kind == R_PHASE_REAL; }
+
+// Reorders the ops between two remaps into waves: every phase whose
+// predecessors (the earlier ops it does not commute with) are done, then
+// every gate whose predecessors are done, and again. The phases in front of
+// a wave of rotations then form one run, and a run costs one multiply per
+// register slot. The order stays a topological order of the non-commuting
+// pairs, so the product is unchanged.
+void schedule_waves(std::vector<RegOp> &ops) {
+    size_t a = 0;
+    while (a < ops.size()) {
+        size_t b = a;
+        while (b < ops.size() && ops[b].kind != R_REMAP) ++b;
+        const size_t n = b - a;
+        if (n > 2) {
+            std::vector<std::vector<uint32_t>> succ(n);
+            std::vector<uint32_t> preds(n, 0);
+            for (size_t i = 0; i < n; ++i)
+                for (size_t j = i + 1; j < n; ++j)
+                    if (!commute(ops[a + i], ops[a + j])) { succ[i].push_back((uint32_t)j); ++preds[j]; }
+            std::vector<RegOp> out;
+            out.reserve(n);
+            std::vector<char> done(n, 0);
+            size_t emitted = 0;
+            while (emitted < n) {
+                for (int want_phase = 1; want_phase >= 0; --want_phase) {
+                    bool again = true;
+                    while (again) {
+                        again = false;
+                        for (size_t i = 0; i < n; ++i) {
+                            if (done[i] || preds[i] || is_phase(ops[a + i]) != (want_phase == 1)) continue;
+                            done[i] = 1;
+                            ++emitted;
+                            out.push_back(ops[a + i]);
+                            for (uint32_t j : succ[i]) if (--preds[j] == 0 && j < i) again = true;
+                        }
+                    }
+                }
+            }
+            std::copy(out.begin(), out.end(), ops.begin() + a);
+        }
+        a = b + 1;
+    }
+}
 
 // Second-level schedule: inside each pass, the same commutation-aware greedy
 // as the pass planner, with the tile as the "state" and the log2(A) register

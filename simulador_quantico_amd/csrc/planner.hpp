@@ -84,6 +84,8 @@ struct Pass {
     int64_t rop_count = 0;
     int64_t mem = -1;                 // PassMem index of the register program
     int32_t phases = 0;               // register phases (LDS remaps = phases - 1)
+    int64_t x_off = 0;                // interpreter's program: byte offset of its XPass in Plan::xprog
+    int32_t x_stages = 0;             // its stages (LDS remaps = stages - 1)
 };
 
 // ---- register kernel program --------------------------------------------
@@ -142,6 +144,15 @@ struct PassMem {
 };
 static_assert(sizeof(PassMem) == 2056, "PassMem layout is shared with the kernels");
 
+// How the interpreted kernels run a plan's tiles: workgroups of B threads with
+// A amplitudes each take tiles of 2^r amplitudes, the plan's own tile plus
+// r - shape.r of the lowest non-local bits; the workgroup needs barriers around
+// a remap when a plan's tile spans more than one wave.
+struct ExecShape {
+    int r, A, B;
+    bool sync;
+};
+
 struct Plan {
     int qubits = 0;
     int dtype = HGM_C128;
@@ -158,13 +169,36 @@ struct Plan {
     std::vector<PhaseMap> maps;
     std::vector<PassMem> mems;
     int max_phases = 0;
+    ExecShape exec{};
+    std::vector<uint64_t> xprog;      // the interpreted kernels' programs (XPass and XOp records)
     std::shared_ptr<JitCode> jit;     // HGM_KERNEL_JIT: generated and compiled pass kernels
 };
 
 // Builds the register program of every pass (fills rops/maps/mems).
 void build_register_program(Plan &plan);
 
+// Reorders the ops between two remaps into waves: every phase whose
+// predecessors (the earlier ops it does not commute with) are done, then
+// every gate whose predecessors are done, and again.
+void schedule_waves(std::vector<RegOp> &ops);
+
+bool is_phase(const RegOp &o);
+
 size_t amp_bytes(int dtype);
+
+// Whether a pass over a state of `bytes` bytes loads and stores it with the
+// nontemporal (streaming) hint. Nothing re-reads an amplitude before the next
+// pass, so what matters is where the state lies between passes. 64-256 MiB: in
+// the 256 MiB last-level cache, which the hint keeps it out of (plan-compiled
+// FP64 Grover, 24 iterations: 22 qubits 2537 -> 2057 us, 24 qubits 10340 ->
+// 8002; random layers of depth 6 at 24 qubits 478 -> 443). Larger: in HBM,
+// where the hint is worth 3-5% (26 qubits 41.3 against 42.7 ms). 16-32 MiB:
+// about the 32 MiB of the eight L2s, whose dirty lines every kernel boundary
+// writes back; with the hint they leave early (20 qubits 642 against 738 us).
+// Up to 8 MiB plain loads hit the L2s (16 qubits 305 -> 273 us), and the
+// stores keep the hint (20 qubits FP32, 8 MiB: 572 us; stores plain too 607;
+// both with the hint 587).
+void state_streams(size_t bytes, bool *loads, bool *stores);
 
 // Validates a tuning tuple (the reference's rules of src/core/dgm_core.cpp:177-241
 // plus this library's limits) and derives the tile shape used for a state of

@@ -1,0 +1,536 @@
+// Builds the interpreted kernels' programs (see program.hpp).
+#include "program.hpp"
+
+#include <algorithm>
+#include <complex>
+#include <cstring>
+
+namespace hgm {
+
+namespace {
+
+// Factors are multiplied together in extended precision and rounded once, to
+// the amplitude type: a rotation's phases and coefficients are then as exact
+// as the entries of its gate.
+using R = long double;
+using C = std::complex<R>;
+
+int popc(uint64_t v) { return __builtin_popcountll(v); }
+
+// A gate of a pass in tile coordinates of the execution shape, before it is
+// placed in a stage: a pair gate or (diagonal) two conditional phases.
+struct Item {
+    const DevOp *d;
+    int32_t kind;          // K_DENSE, K_ANTI, K_DIAG or K_DIAG_GLOBAL
+    int32_t tbit;          // tile bit (K_DIAG_GLOBAL: state-index bit)
+    uint32_t lmask, lval;
+    uint64_t gmask, gval;
+    uint32_t need, wr, rd; // tile bits to be registers, mixed, tested
+};
+
+// A physical operation on registers (coordinates of one stage).
+struct ROp {
+    bool phase;
+    XKind kind;
+    int bit = 0;
+    uint32_t rmask = 0, rval = 0, tmask = 0, tval = 0;
+    uint64_t gmask = 0, gval = 0;
+    R m[8] = {0};
+    int slot = 0;          // wave: phases even, gates odd
+};
+
+void split_cond(uint32_t mask, uint32_t val, uint32_t S, ROp &o) {
+    for (; mask; mask &= mask - 1) {
+        const int b = __builtin_ctz(mask);
+        const uint32_t v = (val >> b) & 1, below = (1u << b) - 1;
+        if ((S >> b) & 1) {
+            const int i = popc(S & below);
+            o.rmask |= 1u << i;
+            o.rval |= v << i;
+        } else {
+            const int j = popc(~S & below);
+            o.tmask |= 1u << j;
+            o.tval |= v << j;
+        }
+    }
+}
+
+bool is_one(R re, R im) { return re == 1.0 && im == 0.0; }
+
+// Largest entry beside the 1 of a rotation's row: 1 for a unitary gate, up to
+// the rounding of its entries.
+constexpr R kMaxTurn = 1.0L + 1e-6L;
+
+// Phases x0, x1, y of modulus 1 with v[i][j] = x_i * o[i][j] * y_j (y_0 = 1)
+// and every o[i][j] real; false when there are none up to the rounding of v's
+// entries to double (16 units in the last place). Nonzero entries link rows to
+// columns: with column 0's phase 1 the links give the others, and the fourth
+// entry is the check. Every unitary matrix has them.
+bool real_middle(const C v[2][2], C x[2], C *y, R o[2][2]) {
+    C row[2] = {C(1, 0), C(1, 0)}, col[2] = {C(1, 0), C(1, 0)};
+    bool have_r[2] = {false, false}, have_c[2] = {true, false};
+    for (int pass = 0; pass < 3; ++pass)
+        for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < 2; ++j) {
+                if (v[i][j] == C(0, 0)) continue;
+                const C u = v[i][j] / std::abs(v[i][j]);
+                if (have_c[j] && !have_r[i]) { row[i] = u * std::conj(col[j]); have_r[i] = true; }
+                else if (have_r[i] && !have_c[j]) { col[j] = u * std::conj(row[i]); have_c[j] = true; }
+            }
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) {
+            const C w = v[i][j] * std::conj(row[i] * col[j]);
+            if (std::abs(w.imag()) > 16 * 0x1p-52L * std::abs(w)) return false;
+            o[i][j] = w.real();
+        }
+    x[0] = row[0];
+    x[1] = row[1];
+    *y = col[1];
+    return true;
+}
+
+// Emits one item as register operations. `flip` holds the tile bits whose two
+// values are exchanged in the registers (physical = logical ^ flip): an
+// uncontrolled X, anti-diagonal gate or row-exchanged gate toggles its bit
+// instead of moving amplitudes. `scale` is a factor of the whole state that is
+// still to be applied.
+void emit(const Item &it, uint32_t S, uint32_t &flip, C &scale, std::vector<ROp> &out) {
+    const DevOp &d = *it.d;
+    const uint32_t lval = it.lval ^ (flip & it.lmask);
+    auto phase = [&](C f, uint32_t lm, uint32_t lv, uint64_t gm, uint64_t gv) {
+        if (f == C(1, 0)) return;
+        ROp o;
+        o.phase = true;
+        o.kind = X_PHASE;
+        split_cond(lm, lv, S, o);
+        o.gmask = gm;
+        o.gval = gv;
+        o.m[0] = f.real();
+        o.m[1] = f.imag();
+        out.push_back(o);
+    };
+    if (it.kind == K_DIAG_GLOBAL) {
+        for (int v = 0; v < 2; ++v)
+            phase(C(d.m[6 * v], d.m[6 * v + 1]), it.lmask, lval, it.gmask | (uint64_t(1) << it.tbit),
+                  it.gval | (uint64_t(v) << it.tbit));
+        return;
+    }
+    const uint32_t tb = 1u << it.tbit, f = (flip >> it.tbit) & 1u;
+    if (it.kind == K_DIAG) {
+        for (uint32_t v = 0; v < 2; ++v)
+            phase(C(d.m[6 * v], d.m[6 * v + 1]), it.lmask | tb, lval | ((v ^ f) << it.tbit), it.gmask, it.gval);
+        return;
+    }
+    R m[8];   // row-major on the physical pair
+    for (int row = 0; row < 2; ++row)
+        for (int col = 0; col < 2; ++col)
+            for (int c = 0; c < 2; ++c) m[4 * row + 2 * col + c] = d.m[4 * (row ^ (int)f) + 2 * (col ^ (int)f) + c];
+    const bool free_gate = !it.lmask && !it.gmask;
+    if (it.kind == K_ANTI && free_gate) {   // values exchanged, then a phase on each
+        flip ^= tb;
+        phase(C(m[4], m[5]), tb, 0, 0, 0);
+        phase(C(m[2], m[3]), tb, tb, 0, 0);
+        return;
+    }
+    ROp o;
+    o.phase = false;
+    o.bit = popc(S & (tb - 1));
+    if (free_gate) {
+        const C v[2][2] = {{C(m[0], m[1]), C(m[2], m[3])}, {C(m[4], m[5]), C(m[6], m[7])}};
+        C x[2], y;
+        R w[2][2];
+        if (real_middle(v, x, &y, w)) {
+            // the larger entry of each row becomes 1; with the off-diagonal ones the larger, rows are exchanged
+            const int ex = std::abs(w[0][0]) < std::abs(w[0][1]) ? 1 : 0;
+            const R d0 = w[ex][0], d1 = w[1 - ex][1];   // of the new rows 0 and 1
+            if (d0 != 0 && d1 != 0) {
+                const R t0 = w[ex][1] / d0, t1 = w[1 - ex][0] / d1;
+                if (std::abs(t0) <= kMaxTurn && std::abs(t1) <= kMaxTurn) {
+                    phase(y, tb, tb, 0, 0);
+                    if (ex) flip ^= tb;
+                    o.kind = X_ROT;
+                    o.m[0] = t0;
+                    o.m[1] = t1;
+                    out.push_back(o);
+                    const C e0 = x[ex] * d0, e1 = x[1 - ex] * d1;
+                    scale *= e0;
+                    phase(e1 / e0, tb, tb, 0, 0);
+                    return;
+                }
+            }
+        }
+    }
+    split_cond(it.lmask, lval, S, o);
+    o.gmask = it.gmask;
+    o.gval = it.gval;
+    std::copy(m, m + 8, o.m);
+    const bool real = m[1] == 0 && m[3] == 0 && m[5] == 0 && m[7] == 0;
+    const bool swap = it.kind == K_ANTI && is_one(m[2], m[3]) && is_one(m[4], m[5]);
+    if (o.rmask) o.kind = real ? X_REAL_MASK : X_DENSE_MASK;
+    else if (swap) o.kind = X_SWAP;
+    else if (o.tmask) o.kind = real ? X_REAL_LANE : X_DENSE_LANE;
+    else o.kind = real ? X_DENSE_REAL : X_DENSE;
+    out.push_back(o);
+}
+
+// Orders a stage's operations into waves (phases as early as they commute,
+// then gates), keeping the order of every pair that does not commute: gates
+// on a register bit conflict with gates on it and with whatever tests it.
+void into_waves(std::vector<ROp> &ops) {
+    int gate[8] = {0}, test[8] = {0};
+    for (ROp &o : ops) {
+        int s = 0;
+        for (uint32_t m = o.rmask; m; m &= m - 1) s = std::max(s, gate[__builtin_ctz(m)]);
+        if (!o.phase) s = std::max({s, gate[o.bit], test[o.bit]});
+        if ((s & 1) == (o.phase ? 1 : 0)) ++s;
+        o.slot = s;
+        for (uint32_t m = o.rmask; m; m &= m - 1) test[__builtin_ctz(m)] = std::max(test[__builtin_ctz(m)], s);
+        if (!o.phase) gate[o.bit] = std::max(gate[o.bit], s);
+    }
+    std::stable_sort(ops.begin(), ops.end(), [](const ROp &a, const ROp &b) { return a.slot < b.slot; });
+}
+
+template <class T>
+XOp<T> record(const ROp &o, uint32_t A) {
+    XOp<T> x;
+    std::memset(&x, 0, sizeof x);
+    x.kind = (uint8_t)o.kind;
+    x.bit = (uint8_t)o.bit;
+    x.tmask = o.tmask;
+    x.tval = o.tval;
+    x.gmask = o.gmask;
+    x.gval = o.gval;
+    for (int i = 0; i < 8; ++i) x.m[i] = (T)o.m[i];
+    for (uint32_t k = 0; k < A; ++k)
+        if ((o.phase || !((k >> o.bit) & 1)) && (k & o.rmask) == o.rval) x.pmask |= 1u << k;
+    if (o.phase) {
+        x.pat = X_PAT_MASK;
+        if (popc(o.rmask) <= 2 && o.rval == o.rmask) x.pat = (uint8_t)o.rmask;
+        else if (popc(o.rmask) == 1) x.pat = (uint8_t)(X_PAT_CLEAR + __builtin_ctz(o.rmask));
+    }
+    return x;
+}
+
+// Records of one pass, and the factors of its X_VEC records.
+template <class T>
+struct Records {
+    uint32_t A;
+    std::vector<XOp<T>> ops;
+    std::vector<T> table;
+    C scale = C(1, 0);   // factor of the whole state still to be applied
+
+    // A factor per register, the pending scale included.
+    void vec(std::vector<C> &f) {
+        bool real = true, one = true;
+        for (C &z : f) {
+            z *= scale;
+            real = real && (T)z.imag() == T(0);
+            one = one && z == C(1, 0);
+        }
+        scale = C(1, 0);
+        if (one) return;
+        XOp<T> x;
+        std::memset(&x, 0, sizeof x);
+        x.kind = real ? X_VEC_REAL : X_VEC;
+        x.pmask = (uint32_t)table.size();
+        for (const C &z : f) {
+            table.push_back((T)z.real());
+            if (!real) table.push_back((T)z.imag());
+        }
+        ops.push_back(x);
+    }
+
+    // The phases [b, e) of a wave that test register bits only: one record when
+    // a pattern of set (or one clear) register bits says it, else one factor
+    // per register.
+    void uniform(const ROp *b, const ROp *e) {
+        if (b == e) return;
+        if (e - b == 1 && scale == C(1, 0)) {
+            XOp<T> x = record<T>(*b, A);
+            if (x.pat != X_PAT_MASK) {
+                x.flags = (uint8_t)(X_FIRST | X_LAST | (b->m[1] == 0.0 ? X_REAL : 0));
+                ops.push_back(x);
+                return;
+            }
+        }
+        std::vector<C> f(A, C(1, 0));
+        for (const ROp *o = b; o != e; ++o)
+            for (uint32_t k = 0; k < A; ++k)
+                if ((k & o->rmask) == o->rval) f[k] *= C(o->m[0], o->m[1]);
+        vec(f);
+    }
+
+    // Phases with conditions on threads or tiles, grouped by the registers they
+    // act on (the caller sorted them), equal conditions multiplied together.
+    void groups(const ROp *b, const ROp *e) {
+        while (b != e) {
+            std::vector<ROp> group;
+            const ROp head = *b;
+            for (; b != e && b->rmask == head.rmask && b->rval == head.rval; ++b) {
+                auto same = std::find_if(group.begin(), group.end(), [&](const ROp &g) {
+                    return g.tmask == b->tmask && g.tval == b->tval && g.gmask == b->gmask && g.gval == b->gval;
+                });
+                if (same == group.end()) { group.push_back(*b); continue; }
+                const C f = C(same->m[0], same->m[1]) * C(b->m[0], b->m[1]);
+                same->m[0] = f.real();
+                same->m[1] = f.imag();
+            }
+            bool real = true;
+            for (const ROp &g : group) real = real && g.m[1] == 0.0;
+            for (size_t k = 0; k < group.size(); ++k) {
+                XOp<T> x = record<T>(group[k], A);
+                x.flags = (uint8_t)((k == 0 ? X_FIRST : 0) | (k + 1 == group.size() ? X_LAST : 0) | (real ? X_REAL : 0));
+                ops.push_back(x);
+            }
+        }
+    }
+
+    // A run of rotations: those on different register bits commute, and three
+    // of a full set of four (two of two or three) already cost less as one
+    // record than one by one.
+    void rotations(const ROp *b, const ROp *e) {
+        const int bits = A == 2 ? 1 : A == 4 ? 2 : A == 8 ? 3 : 4;
+        while (b != e) {
+            uint32_t used = 0;
+            const ROp *n = b;
+            for (; n != e && n->bit < bits && !((used >> n->bit) & 1u); ++n) used |= 1u << n->bit;
+            if (n == b) ++n;   // a fifth register bit
+            if (popc(used) >= (bits + 2) / 2 && bits > 1) {
+                XOp<T> x;
+                std::memset(&x, 0, sizeof x);
+                x.kind = X_ROTS;
+                for (; b != n; ++b) {
+                    x.m[2 * b->bit] = (T)b->m[0];
+                    x.m[2 * b->bit + 1] = (T)b->m[1];
+                }
+                ops.push_back(x);
+            } else {
+                for (; b != n; ++b) ops.push_back(record<T>(*b, A));
+            }
+        }
+    }
+
+    void stage(std::vector<ROp> &list) {
+        into_waves(list);
+        for (size_t i = 0; i < list.size();) {
+            size_t e = i;
+            if (!list[i].phase) {
+                if (list[i].kind != X_ROT) { ops.push_back(record<T>(list[i++], A)); continue; }
+                while (e < list.size() && !list[e].phase && list[e].kind == X_ROT) ++e;
+                rotations(list.data() + i, list.data() + e);
+                i = e;
+                continue;
+            }
+            while (e < list.size() && list[e].phase && list[e].slot == list[i].slot) ++e;
+            auto uniform_op = [](const ROp &o) { return !o.tmask && !o.gmask; };
+            std::stable_sort(list.begin() + i, list.begin() + e, [&](const ROp &a, const ROp &b) {
+                if (uniform_op(a) != uniform_op(b)) return uniform_op(a);
+                return a.rmask != b.rmask ? a.rmask < b.rmask : a.rval < b.rval;
+            });
+            size_t u = i;
+            while (u < e && uniform_op(list[u])) ++u;
+            uniform(list.data() + i, list.data() + u);
+            groups(list.data() + u, list.data() + e);
+            i = e;
+        }
+    }
+
+    // The pending scale, when it is due: at the end of the pass, and before it
+    // moves the amplitudes far from 1.
+    void flush(bool end) {
+        const R s = std::abs(scale);
+        if (scale == C(1, 0) || (!end && s >= 0x1p-20L && s <= 0x1p20L)) return;
+        std::vector<C> f(A, C(1, 0));
+        vec(f);
+    }
+};
+
+// Runs of an ascending bit deposit: index bit j goes to state bit pos[j].
+int deposit_runs(const int *pos, int n, XRun *out, int cap) {
+    int runs = 0;
+    for (int j = 0; j < n;) {
+        int len = 1;
+        while (j + len < n && pos[j + len] == pos[j] + len && len < 32) ++len;
+        if (runs < cap) out[runs] = {len >= 32 ? ~0u : (1u << len) - 1, (uint16_t)j, (uint16_t)pos[j]};
+        ++runs;
+        j += len;
+    }
+    return runs;
+}
+
+template <class T>
+void build(Plan &plan) {
+    constexpr int F = sizeof(T) == 4 ? 5 : 4;
+    const ExecShape &ex = plan.exec;
+    const int r = plan.shape.r, c = plan.shape.c, rx = ex.r, n = plan.qubits;
+    int a = 0;
+    while ((1 << a) < ex.A) ++a;
+    const uint32_t own = (uint32_t)((uint64_t(1) << r) - 1);
+    const uint32_t forbid = (r - c >= a) ? (uint32_t)((1u << c) - 1) : 0u;
+    plan.xprog.clear();
+    std::vector<Item> items;
+    std::vector<ROp> ops;
+    for (Pass &ps : plan.passes) {
+        // tile bits of the execution shape: the plan's, then the lowest non-local state bits
+        int pos[32];
+        for (int j = 0; j < r; ++j) pos[j] = ps.local_pos[j];
+        uint64_t local = ps.local_mask;
+        for (int j = r, b = 0; j < rx; ++b)
+            if (!((local >> b) & 1)) { pos[j++] = b; local |= uint64_t(1) << b; }
+        int tile_of[64];
+        std::fill(tile_of, tile_of + 64, -1);
+        for (int j = r; j < rx; ++j) tile_of[pos[j]] = j;
+        items.clear();
+        for (int64_t i = 0; i < ps.op_count; ++i) {
+            const DevOp &d = plan.ops[ps.op_begin + i];
+            Item it{&d, d.kind, d.tbit, d.lmask, d.lval, 0, 0, 0, 0, 0};
+            for (uint64_t g = d.gmask; g; g &= g - 1) {
+                const int b = __builtin_ctzll(g);
+                const uint64_t v = (d.gval >> b) & 1;
+                if (tile_of[b] >= 0) {
+                    it.lmask |= 1u << tile_of[b];
+                    it.lval |= (uint32_t)v << tile_of[b];
+                } else {
+                    it.gmask |= uint64_t(1) << b;
+                    it.gval |= v << b;
+                }
+            }
+            if (it.kind == K_DIAG_GLOBAL && tile_of[it.tbit] >= 0) {
+                it.kind = K_DIAG;
+                it.tbit = tile_of[it.tbit];
+            }
+            it.rd = it.lmask;
+            if (it.kind == K_DENSE || it.kind == K_ANTI) it.need = it.wr = 1u << it.tbit;
+            else if (it.kind == K_DIAG) {
+                it.rd |= 1u << it.tbit;
+                if (plan.pre_phase[ps.op_begin + i]) it.need = it.wr = 1u << it.tbit;
+            }
+            items.push_back(it);
+        }
+        // stages: the same greedy as the pass planner, with the tile as the state and the register bits as the
+        // tile; the first and last keep the coalesced bits on the threads
+        std::vector<uint32_t> sets;
+        std::vector<std::vector<int>> lists;
+        std::vector<char> done(items.size(), 0);
+        for (size_t head = 0; head < items.size();) {
+            uint32_t S = 0, bw = 0, br = 0;
+            int nS = 0;
+            std::vector<int> list;
+            for (size_t k = head; k < items.size(); ++k) {
+                if (done[k]) continue;
+                const Item &it = items[k];
+                bool ok = !(it.wr & (bw | br)) && !(it.rd & bw);
+                if (ok && (it.need & ~S)) {
+                    if (nS < a && !(sets.empty() && (it.need & forbid))) { S |= it.need; ++nS; }
+                    else ok = false;
+                }
+                if (ok) { list.push_back((int)k); done[k] = 1; }
+                else { bw |= it.wr; br |= it.rd; if ((bw & own) == own) break; }
+            }
+            while (head < items.size() && done[head]) ++head;
+            sets.push_back(S);
+            lists.push_back(std::move(list));
+        }
+        if (sets.empty() || (sets.back() & forbid)) { sets.push_back(0); lists.emplace_back(); }
+        for (size_t i = 0; i < sets.size(); ++i) {
+            const bool edge = i == 0 || i + 1 == sets.size();
+            for (int b = r - 1; b >= 0 && popc(sets[i]) < a; --b)
+                if (!((sets[i] >> b) & 1) && !(edge && ((forbid >> b) & 1))) sets[i] |= 1u << b;
+            for (int b = r - 1; b >= 0 && popc(sets[i]) < a; --b) sets[i] |= 1u << b;
+        }
+        // records
+        auto map_of = [&](uint32_t S) {
+            XMap m;
+            std::memset(&m, 0, sizeof m);
+            int i = 0;
+            for (int b = 0; b < rx; ++b)
+                if ((S >> b) & 1) {
+                    m.low[i] = (uint16_t)((1u << b) - 1);
+                    m.sw[i++] = (uint16_t)x_swizzle<F>(1u << b);
+                }
+            return m;
+        };
+        Records<T> recs;
+        recs.A = (uint32_t)ex.A;
+        uint32_t flip = 0;
+        for (size_t i = 0; i < sets.size(); ++i) {
+            if (i > 0) {
+                XOp<T> x;
+                std::memset(&x, 0, sizeof x);
+                x.kind = X_REMAP;
+                const XMap m = map_of(sets[i]);
+                std::memcpy(x.m, &m, sizeof m);
+                recs.ops.push_back(x);
+            }
+            ops.clear();
+            for (int k : lists[i]) {
+                emit(items[k], sets[i], flip, recs.scale, ops);
+                if (ops.size() >= 64) { recs.stage(ops); recs.flush(false); ops.clear(); }
+            }
+            recs.stage(ops);
+            recs.flush(i + 1 == sets.size());
+        }
+        XPass xp;
+        std::memset(&xp, 0, sizeof xp);
+        xp.n_ops = (int32_t)recs.ops.size();
+        xp.first = map_of(sets.front());
+        auto lanes = [&](uint32_t S, uint64_t *bit, XRun *runs) {
+            int p[32], np = 0, i = 0;
+            for (int b = 0; b < rx; ++b) {
+                if ((S >> b) & 1) bit[i++] = uint64_t(1) << pos[b];
+                else p[np++] = pos[b];
+            }
+            return deposit_runs(p, np, runs, kXLaneRuns);
+        };
+        xp.n_load = lanes(sets.front(), xp.lbit, xp.load);
+        xp.n_store = lanes(sets.back(), xp.sbit, xp.store);
+        for (int b = 0; b < rx; ++b)
+            if ((flip >> b) & 1) ((sets.back() >> b) & 1 ? xp.rflip : xp.sflip) |= uint64_t(1) << pos[b];
+        int p[64], np = 0;
+        for (int b = 0; b < n; ++b)
+            if (!((local >> b) & 1)) p[np++] = b;
+        xp.n_base = deposit_runs(p, np, xp.base, kXBaseRuns);
+        ps.x_stages = (int32_t)sets.size();
+        ps.x_off = (int64_t)(plan.xprog.size() * 8);
+        // one zero record past the end (the kernel loads ahead), then the factor table
+        const size_t op_bytes = (recs.ops.size() + 1) * sizeof(XOp<T>);
+        const size_t table_at = (sizeof(XPass) + op_bytes + 63) / 64 * 64;
+        xp.table = (int64_t)table_at;
+        const size_t at = plan.xprog.size();
+        plan.xprog.resize(at + (table_at + recs.table.size() * sizeof(T) + 63) / 64 * 8, 0);
+        char *to = reinterpret_cast<char *>(&plan.xprog[at]);
+        std::memcpy(to, &xp, sizeof xp);
+        if (!recs.ops.empty()) std::memcpy(to + sizeof xp, recs.ops.data(), recs.ops.size() * sizeof(XOp<T>));
+        if (!recs.table.empty()) std::memcpy(to + table_at, recs.table.data(), recs.table.size() * sizeof(T));
+    }
+}
+
+// The execution shape of a plan: the plan's own threads and amplitudes per
+// thread, with more amplitudes per thread where the tuning asks for fewer than
+// a register kernel does well with, and several tiles per workgroup where a
+// tile has less than a wave.
+ExecShape choose_shape(const Plan &plan) {
+    const int r = plan.shape.r, c = plan.shape.c, n = plan.qubits;
+    int a = 0;
+    while ((2 << a) <= 2 * plan.shape.R) ++a;
+    const int want = plan.dtype == HGM_C64 ? 4 : 3;
+    if (n - want >= 16)
+        while (a < want && a < r - c) ++a;
+    ExecShape e;
+    e.A = 1 << a;
+    e.r = r;
+    e.sync = r - a > 6;
+    while (e.r - a < 6 && e.r < n) ++e.r;
+    e.B = 1 << (e.r - a);
+    return e;
+}
+
+}  // namespace
+
+void build_exec_program(Plan &plan) {
+    plan.exec = choose_shape(plan);
+    if (plan.dtype == HGM_C64) build<float>(plan);
+    else build<double>(plan);
+}
+
+}  // namespace hgm

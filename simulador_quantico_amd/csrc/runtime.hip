@@ -24,6 +24,7 @@
 
 #include "hgm_gpu.h"
 #include "kernels.hpp"
+#include "program.hpp"
 #include "planner.hpp"
 #include "runtime.hpp"
 #include "jit.hpp"
@@ -92,14 +93,8 @@ struct Ctx {
     hipStream_t stream = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr, e4 = nullptr, e5 = nullptr;
     int cus = 0;
-    DevOp *ops = nullptr;       // op tables of the current call (grow-only)
-    size_t ops_cap = 0;
-    void *rops = nullptr;       // register-kernel programs, phase maps, pass tables (grow-only)
-    size_t rops_cap = 0;
-    void *maps = nullptr;
-    size_t maps_cap = 0;
-    void *mems = nullptr;
-    size_t mems_cap = 0;
+    void *prog = nullptr;       // register-kernel programs or op tables of the current call (grow-only)
+    size_t prog_cap = 0;
     void *cache = nullptr;      // device buffer of hgm_execute (grow-only)
     size_t cache_cap = 0;
     // reduction partials, in pinned host memory that the kernels write directly
@@ -239,16 +234,6 @@ int jit_load_locked(const JitCode &jc, JitModule **out) {
     return HGM_OK;
 }
 
-int reserve_ops(size_t n) {
-    Ctx &c = ctx();
-    if (n <= c.ops_cap) return HGM_OK;
-    if (c.ops) { hipStreamSynchronize(c.stream); hipFree(c.ops); c.ops = nullptr; c.ops_cap = 0; }
-    size_t cap = n < 1024 ? 1024 : n + n / 2;
-    HGM_HIP(hipMalloc(&c.ops, cap * sizeof(DevOp)), "hipMalloc(op tables)");
-    c.ops_cap = cap;
-    return HGM_OK;
-}
-
 int reserve(void **buf, size_t *cap, size_t bytes, const char *what) {
     Ctx &c = ctx();
     if (bytes <= *cap) return HGM_OK;
@@ -338,25 +323,28 @@ int run_plan_graph_locked(hgm_state *s, const hgm_plan *hp, hgm_stats *st) {
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
-// Bytes of device tables the register or LDS kernels read for plan p.
+// Device table of a register or LDS plan, as one block: the register
+// kernels' programs or the LDS kernel's op tables.
+const void *plan_table(const Plan &p) {
+    return p.kernel == HGM_KERNEL_REG ? static_cast<const void *>(p.xprog.data()) : p.ops.data();
+}
 size_t plan_table_bytes(const Plan &p) {
-    if (p.kernel == HGM_KERNEL_REG)
-        return align256(p.rops.size() * sizeof(RegOp)) + align256(p.maps.size() * sizeof(PhaseMap)) +
-               align256(p.mems.size() * sizeof(PassMem));
-    return align256(p.ops.size() * sizeof(DevOp));
+    return p.kernel == HGM_KERNEL_REG ? p.xprog.size() * sizeof(uint64_t) : p.ops.size() * sizeof(DevOp);
 }
 
-// Device tables of a register or LDS plan: where its kernels read their
-// programs (unused by plan-compiled plans).
-struct PlanTables {
-    const void *rops, *maps, *mems;
-    const DevOp *dops;
-};
+// Bytes of a register plan's inspectable program (hgm_plan_program,
+// hgm_plan_maps): part of the size limit of hgm_state_apply_noalloc.
+size_t register_program_bytes(const Plan &p) {
+    return p.kernel == HGM_KERNEL_REG ? align256(p.rops.size() * sizeof(RegOp)) +
+                                            align256(p.maps.size() * sizeof(PhaseMap)) +
+                                            align256(p.mems.size() * sizeof(PassMem))
+                                      : 0;
+}
 
 // Launches every non-empty pass of the plan on `stream`, with no events or
-// waits (jm: the plan's loaded module, for plan-compiled plans). Assumes the
-// lock.
-int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const PlanTables &t, hipStream_t stream) {
+// waits (jm: the plan's loaded module, for plan-compiled plans; table: the
+// plan's table on the device, for the others). Assumes the lock.
+int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const void *table, hipStream_t stream) {
     const bool reg = p.kernel == HGM_KERNEL_REG;
     const bool jit = p.kernel == HGM_KERNEL_JIT;
     PassArgs a;
@@ -364,7 +352,7 @@ int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const PlanT
     a.r = p.shape.r; a.c = p.shape.c; a.B = p.shape.B; a.R = p.shape.R;
     a.n_tiles = int64_t(1) << (p.qubits - p.shape.r);
     const uint64_t all = (uint64_t(1) << p.qubits) - 1;
-    const size_t tile_bytes = (size_t(1) << p.shape.r) * amp_bytes(p.dtype);
+    const size_t tile_bytes = reg ? (size_t(1) << p.exec.r) * amp_bytes(p.dtype) : 0;
     for (size_t pi = 0; pi < p.passes.size(); ++pi) {
         const Pass &ps = p.passes[pi];
         if (ps.op_count == 0) continue;
@@ -372,14 +360,14 @@ int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const PlanT
         if (jit) {
             if (int rc = launch_jit_pass_locked(s, p, jm, pi, stream)) return rc;
         } else if (reg) {
-            HGM_HIP(launch_pass_reg(p.dtype, 2 * p.shape.R, s->d, static_cast<const RegOp *>(t.rops) + ps.rop_begin,
-                                    (int)ps.rop_count, static_cast<const PhaseMap *>(t.maps),
-                                    static_cast<const PassMem *>(t.mems) + ps.mem, a.nonlocal_mask, a.n_tiles,
-                                    p.shape.r, p.shape.B, ps.phases > 1 ? tile_bytes : 0, stream),
+            const XPass *xp = reinterpret_cast<const XPass *>(static_cast<const char *>(table) + ps.x_off);
+            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, s->d, xp, ps.x_stages > 1 ? tile_bytes : 0, stream),
                     "pass launch");
         } else {
             std::memcpy(a.local_pos, ps.local_pos, sizeof(a.local_pos));
-            HGM_HIP(launch_pass_lds(p.dtype, s->d, t.dops + ps.op_begin, (int)ps.op_count, a, stream), "pass launch");
+            HGM_HIP(launch_pass_lds(p.dtype, s->d, static_cast<const DevOp *>(table) + ps.op_begin, (int)ps.op_count, a,
+                                    stream),
+                    "pass launch");
         }
     }
     return HGM_OK;
@@ -395,51 +383,22 @@ int run_plan_locked(hgm_state *s, const Plan &p, hgm_stats *st, double plan_ms, 
         t_err = "plan was built for another qubit count or dtype";
         return HGM_E_STATE;
     }
-    const bool reg = p.kernel == HGM_KERNEL_REG;
-    const bool jit = p.kernel == HGM_KERNEL_JIT;
     int rc;
     JitModule *jm = nullptr;
-    if (jit) {
+    void *table = workspace;
+    if (p.kernel == HGM_KERNEL_JIT) {
         if ((rc = jit_load_locked(*p.jit, &jm))) return rc;
-    }
-    void *rops = c.rops, *maps = c.maps, *mems = c.mems;
-    DevOp *dops = c.ops;
-    if (workspace && !jit) {
-        char *w = static_cast<char *>(workspace);
-        if (reg) {
-            rops = w;
-            maps = w + align256(p.rops.size() * sizeof(RegOp));
-            mems = static_cast<char *>(maps) + align256(p.maps.size() * sizeof(PhaseMap));
-        } else {
-            dops = reinterpret_cast<DevOp *>(w);
+    } else {
+        const size_t bytes = plan_table_bytes(p);
+        if (!table) {
+            if ((rc = reserve(&c.prog, &c.prog_cap, bytes, "hipMalloc(programs)"))) return rc;
+            table = c.prog;
         }
-    } else if (reg) {
-        if ((rc = reserve(&c.rops, &c.rops_cap, p.rops.size() * sizeof(RegOp), "hipMalloc(programs)"))) return rc;
-        if ((rc = reserve(&c.maps, &c.maps_cap, p.maps.size() * sizeof(PhaseMap), "hipMalloc(maps)"))) return rc;
-        if ((rc = reserve(&c.mems, &c.mems_cap, p.mems.size() * sizeof(PassMem), "hipMalloc(pass tables)"))) return rc;
-        rops = c.rops;
-        maps = c.maps;
-        mems = c.mems;
-    } else if (!jit) {
-        if ((rc = reserve_ops(p.ops.size()))) return rc;
-        dops = c.ops;
-    }
-    if (reg) {
-        if (!p.rops.empty())
-            HGM_HIP(hipMemcpyAsync(rops, p.rops.data(), p.rops.size() * sizeof(RegOp), hipMemcpyHostToDevice,
-                                   c.stream), "hipMemcpyAsync(programs)");
-        if (!p.maps.empty())
-            HGM_HIP(hipMemcpyAsync(maps, p.maps.data(), p.maps.size() * sizeof(PhaseMap), hipMemcpyHostToDevice,
-                                   c.stream), "hipMemcpyAsync(maps)");
-        if (!p.mems.empty())
-            HGM_HIP(hipMemcpyAsync(mems, p.mems.data(), p.mems.size() * sizeof(PassMem), hipMemcpyHostToDevice,
-                                   c.stream), "hipMemcpyAsync(pass tables)");
-    } else if (!jit && !p.ops.empty()) {
-        HGM_HIP(hipMemcpyAsync(dops, p.ops.data(), p.ops.size() * sizeof(DevOp), hipMemcpyHostToDevice, c.stream),
-                "hipMemcpyAsync(op tables)");
+        if (bytes) HGM_HIP(hipMemcpyAsync(table, plan_table(p), bytes, hipMemcpyHostToDevice, c.stream),
+                           "hipMemcpyAsync(programs)");
     }
     HGM_HIP(hipEventRecord(c.e0, c.stream), "hipEventRecord");
-    if ((rc = launch_passes_locked(s, p, jm, {rops, maps, mems, dops}, c.stream))) return rc;
+    if ((rc = launch_passes_locked(s, p, jm, table, c.stream))) return rc;
     HGM_HIP(hipEventRecord(c.e1, c.stream), "hipEventRecord");
     HGM_HIP(hipEventSynchronize(c.e1), "pass execution");
     add_stats(st, p, elapsed(c.e0, c.e1), plan_ms);
@@ -479,21 +438,9 @@ int batch_modules_locked(hgm_batch *b, std::vector<JitModule *> *jms, bool *stal
     return HGM_OK;
 }
 
-// Where the kernels of state i's register or LDS plan read their tables: the
-// batch's device copy, laid out as plan_table_bytes counts it.
-PlanTables batch_tables(const hgm_batch *b, size_t i) {
-    PlanTables t{nullptr, nullptr, nullptr, nullptr};
-    if (b->table_off[i] < 0) return t;
-    const Plan &p = b->plans[i]->plan;
-    char *base = static_cast<char *>(b->tables) + b->table_off[i];
-    if (p.kernel == HGM_KERNEL_REG) {
-        t.rops = base;
-        t.maps = base + align256(p.rops.size() * sizeof(RegOp));
-        t.mems = static_cast<const char *>(t.maps) + align256(p.maps.size() * sizeof(PhaseMap));
-    } else {
-        t.dops = reinterpret_cast<const DevOp *>(base);
-    }
-    return t;
+// The batch's device copy of state i's register or LDS plan's table.
+const void *batch_table(const hgm_batch *b, size_t i) {
+    return b->table_off[i] < 0 ? nullptr : static_cast<const char *>(b->tables) + b->table_off[i];
 }
 
 // Captures the batch: a fork on the context stream, each state's passes in
@@ -506,7 +453,7 @@ int capture_batch_locked(hgm_batch *b, const std::vector<JitModule *> &jms) {
     hipError_t e = hipEventRecord(b->fork, c.stream);
     for (int k = 0; k < b->n_branches && e == hipSuccess; ++k) e = hipStreamWaitEvent(b->streams[k], b->fork, 0);
     for (size_t i = 0; i < b->plans.size() && e == hipSuccess && !rc; ++i)
-        rc = launch_passes_locked(b->states[i], b->plans[i]->plan, jms[i], batch_tables(b, i), b->streams[b->branch[i]]);
+        rc = launch_passes_locked(b->states[i], b->plans[i]->plan, jms[i], batch_table(b, i), b->streams[b->branch[i]]);
     for (int k = 0; k < b->n_branches && e == hipSuccess && !rc; ++k) {
         e = hipEventRecord(b->join[k], b->streams[k]);
         if (e == hipSuccess) e = hipStreamWaitEvent(c.stream, b->join[k], 0);
@@ -687,10 +634,7 @@ int hgm_release_cache(void) {
         *cap = 0;
     };
     drop(&c.cache, &c.cache_cap);
-    drop(reinterpret_cast<void **>(&c.ops), &c.ops_cap);
-    drop(&c.rops, &c.rops_cap);
-    drop(&c.maps, &c.maps_cap);
-    drop(&c.mems, &c.mems_cap);
+    drop(&c.prog, &c.prog_cap);
     for (char *&h : c.h_stage) {
         if (h) hipHostFree(h);
         h = nullptr;
@@ -999,7 +943,7 @@ int hgm_state_apply_noalloc(hgm_state *s, const hgm_op *ops, int64_t n_ops, cons
     double plan_ms = 0;
     int rc = cached_plan(s->qubits, s->dtype, ops, n_ops, iterations, t, &p, &plan_ms);
     if (rc) return rc;
-    const size_t need = plan_table_bytes(*p);
+    const size_t need = std::max(plan_table_bytes(*p), register_program_bytes(*p));
     if (need > kScratchBytes) {
         t_err = "hgm_state_apply_noalloc: the plan's tables take " + std::to_string(need) + " bytes, above the " +
                 std::to_string(kScratchBytes) + "-byte workspace (fewer passes or gates per call)";
@@ -1315,21 +1259,9 @@ int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int
     for (int i = 0; i < n && e == hipSuccess; ++i) {
         const Plan &p = plans[i]->plan;
         if (b->table_off[i] < 0 || (i > 0 && std::find(plans, plans + i, plans[i]) != plans + i)) continue;
-        const PlanTables t = batch_tables(b.get(), (size_t)i);
-        if (p.kernel == HGM_KERNEL_REG) {
-            if (!p.rops.empty())
-                e = hipMemcpy(const_cast<void *>(t.rops), p.rops.data(), p.rops.size() * sizeof(RegOp),
-                              hipMemcpyHostToDevice);
-            if (e == hipSuccess && !p.maps.empty())
-                e = hipMemcpy(const_cast<void *>(t.maps), p.maps.data(), p.maps.size() * sizeof(PhaseMap),
-                              hipMemcpyHostToDevice);
-            if (e == hipSuccess && !p.mems.empty())
-                e = hipMemcpy(const_cast<void *>(t.mems), p.mems.data(), p.mems.size() * sizeof(PassMem),
-                              hipMemcpyHostToDevice);
-        } else if (!p.ops.empty()) {
-            e = hipMemcpy(const_cast<DevOp *>(t.dops), p.ops.data(), p.ops.size() * sizeof(DevOp),
+        if (const size_t bytes = plan_table_bytes(p))
+            e = hipMemcpy(const_cast<void *>(batch_table(b.get(), (size_t)i)), plan_table(p), bytes,
                           hipMemcpyHostToDevice);
-        }
     }
     if (e != hipSuccess) {
         rc = hip_fail(e, "batch streams and tables");

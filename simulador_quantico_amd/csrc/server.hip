@@ -130,7 +130,7 @@ struct Req {
     size_t next = 0;
     int lane = 0;
     int64_t n_tiles = 1;
-    size_t state_bytes = 0, prog_bytes = 0, part_bytes = 0, total_bytes = 0, off = 0, stage_off = 0;
+    size_t state_bytes = 0, rop_bytes = 0, prog_bytes = 0, part_bytes = 0, total_bytes = 0, off = 0, stage_off = 0;
     char *d = nullptr;             // device block: state | programs | maps | pass tables | partials
     ReadoutPartial result{};
 };
@@ -418,8 +418,11 @@ void planner_loop(hgm_server *s) {
             r->n_tiles = int64_t(1) << (r->qubits - p.shape.r);
             r->lane = r->n_tiles == 1 ? 0 : 1;
             r->state_bytes = align_up((size_t(1) << r->qubits) * amp_bytes(s->cfg.dtype));
-            r->prog_bytes = align_up(p.rops.size() * sizeof(RegOp)) + align_up(p.maps.size() * sizeof(PhaseMap)) +
-                            align_up(p.mems.size() * sizeof(PassMem));
+            // on the device: the compiled passes' register programs and the interpreted passes' programs
+            r->rop_bytes = 0;
+            for (int k : r->kernel)
+                if (k >= 0) r->rop_bytes = align_up(p.rops.size() * sizeof(RegOp));
+            r->prog_bytes = r->rop_bytes + align_up(p.xprog.size() * sizeof(uint64_t));
             r->part_bytes = align_up((size_t)r->n_tiles * sizeof(ReadoutPartial));
             r->total_bytes = r->state_bytes + r->prog_bytes + r->part_bytes;
             if (r->total_bytes > s->arena.size() || r->prog_bytes > s->staging.size()) {
@@ -468,12 +471,9 @@ bool admit(hgm_server *s) {
         const Plan &p = r->plan;
         // programs go through pinned memory, so that the copy is queued on the
         // lane's stream without waiting for the steps already in flight
-        char *h = s->staging.base() + soff, *q = h;
-        if (!p.rops.empty()) std::memcpy(q, p.rops.data(), p.rops.size() * sizeof(RegOp));
-        q += align_up(p.rops.size() * sizeof(RegOp));
-        if (!p.maps.empty()) std::memcpy(q, p.maps.data(), p.maps.size() * sizeof(PhaseMap));
-        q += align_up(p.maps.size() * sizeof(PhaseMap));
-        if (!p.mems.empty()) std::memcpy(q, p.mems.data(), p.mems.size() * sizeof(PassMem));
+        char *h = s->staging.base() + soff;
+        if (r->rop_bytes) std::memcpy(h, p.rops.data(), p.rops.size() * sizeof(RegOp));
+        if (!p.xprog.empty()) std::memcpy(h + r->rop_bytes, p.xprog.data(), p.xprog.size() * sizeof(uint64_t));
         hipError_t e = hipMemcpyAsync(r->d + r->state_bytes, h, r->prog_bytes, hipMemcpyHostToDevice, L.stream);
         if (e == hipSuccess)
             e = launch_set_basis(s->cfg.dtype, r->d, uint64_t(1) << r->qubits, r->basis, L.stream);
@@ -494,13 +494,7 @@ bool admit(hgm_server *s) {
 }
 
 RegOp *dev_rops(Req *r) { return reinterpret_cast<RegOp *>(r->d + r->state_bytes); }
-PhaseMap *dev_maps(Req *r) {
-    return reinterpret_cast<PhaseMap *>(r->d + r->state_bytes + align_up(r->plan.rops.size() * sizeof(RegOp)));
-}
-PassMem *dev_mems(Req *r) {
-    return reinterpret_cast<PassMem *>(r->d + r->state_bytes + align_up(r->plan.rops.size() * sizeof(RegOp)) +
-                                       align_up(r->plan.maps.size() * sizeof(PhaseMap)));
-}
+char *dev_xprog(Req *r) { return r->d + r->state_bytes + r->rop_bytes; }
 ReadoutPartial *dev_partials(Req *r) {
     return reinterpret_cast<ReadoutPartial *>(r->d + r->state_bytes + r->prog_bytes);
 }
@@ -518,9 +512,15 @@ bool launch_step(hgm_server *s, Lane &L) {
 
     std::vector<Req *> order(L.active.begin(), L.active.end());
     auto kern = [](const Req *r) { return r->kernel[r->next]; };
+    // the next pass's workgroup shape: the plan's tile for compiled kernels, the interpreter's own for the rest
+    auto amps = [&](const Req *r) { return kern(r) >= 0 ? 2 * r->plan.shape.R : r->plan.exec.A; };
+    auto threads = [&](const Req *r) { return kern(r) >= 0 ? r->plan.shape.B : r->plan.exec.B; };
+    auto tiles = [&](const Req *r) {
+        return int64_t(1) << (r->qubits - (kern(r) >= 0 ? r->plan.shape.r : r->plan.exec.r));
+    };
     std::stable_sort(order.begin(), order.end(), [&](const Req *a, const Req *b) {
-        if (a->plan.shape.R != b->plan.shape.R) return a->plan.shape.R < b->plan.shape.R;
-        if (a->plan.shape.B != b->plan.shape.B) return a->plan.shape.B < b->plan.shape.B;
+        if (amps(a) != amps(b)) return amps(a) < amps(b);
+        if (threads(a) != threads(b)) return threads(a) < threads(b);
         return kern(a) < kern(b);
     });
     // one launch per workgroup shape and kernel: the interpreter (-1) or a
@@ -532,7 +532,7 @@ bool launch_step(hgm_server *s, Lane &L) {
     int n_tasks = 0;
     for (int i = 0; i < (int)order.size(); ++i) {
         Req *r = order[i];
-        const int A = 2 * r->plan.shape.R, B = r->plan.shape.B, K = kern(r);
+        const int A = amps(r), B = threads(r), K = kern(r);
         if (groups.empty() || groups.back().A != A || groups.back().B != B || groups.back().kernel != K)
             groups.push_back({A, B, K, i, 0, 0, 0});
         Group &g = groups.back();
@@ -542,20 +542,19 @@ bool launch_step(hgm_server *s, Lane &L) {
         char *const arena = s->arena.base();
         it.state_off = (uint64_t)(r->d - arena);
         it.ops_off = (uint64_t)(reinterpret_cast<char *>(dev_rops(r) + ps.rop_begin) - arena);
-        it.maps_off = (uint64_t)(reinterpret_cast<char *>(dev_maps(r)) - arena);
-        it.pm_off = (uint64_t)(reinterpret_cast<char *>(dev_mems(r) + ps.mem) - arena);
-        it.nonlocal_mask = ((uint64_t(1) << r->qubits) - 1) & ~ps.local_mask;
+        it.xpass_off = (uint64_t)(dev_xprog(r) + ps.x_off - arena);
+        it.pad[0] = it.pad[1] = 0;
         it.tile_begin = g.tiles;
         it.partials_off = last ? (int64_t)(reinterpret_cast<char *>(dev_partials(r)) - arena) : -1;
-        it.n_ops = (int32_t)ps.rop_count;
-        it.pad = 0;
+        it.sync = r->plan.exec.sync;
+        it.pad2 = 0;
         g.count++;
-        g.tiles += r->n_tiles;
-        if (ps.phases > 1)
-            g.lds = std::max(g.lds, (size_t(1) << r->plan.shape.r) * amp_bytes(s->cfg.dtype));
+        g.tiles += tiles(r);
+        if (K < 0 && ps.x_stages > 1)
+            g.lds = std::max(g.lds, (size_t(1) << r->plan.exec.r) * amp_bytes(s->cfg.dtype));
         if (last) {
             tasks[n_tasks].partials = dev_partials(r);
-            tasks[n_tasks].n = r->n_tiles;
+            tasks[n_tasks].n = tiles(r);
             tasks[n_tasks].out = d_results + n_tasks;
             ++n_tasks;
             step.finishing.push_back(r);
