@@ -27,11 +27,11 @@ hipError_t launch_pass_lds(int dtype, void *state, const DevOp *ops, int n_ops, 
 // launches into a graph.
 hipError_t prepare_pass_kernels(int dtype);
 
-// One full-state pass of the register kernel: the program at xp (device) on a
-// state of `qubits` qubits in execution shape e; lds_bytes is 0 for a pass of
-// one stage.
-hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, void *state, const XPass *xp, size_t lds_bytes,
-                           hipStream_t s);
+// One full-state pass of the register kernel: the program of xp_bytes bytes at
+// xp (device) on a state of `qubits` qubits in execution shape e; lds_bytes is
+// 0 for a pass of one stage.
+hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, void *state, const XPass *xp, uint32_t xp_bytes,
+                           size_t lds_bytes, hipStream_t s);
 
 // Readout of one tile or of a whole state: FP64 sum of |a|^2 and the largest
 // |a|^2 with its index (lowest index on ties).
@@ -55,7 +55,7 @@ struct BatchItem {
     int64_t tile_begin;          // first workgroup of this item in the launch
     int64_t partials_off;        // >= 0: per-tile readout of the pass output (ReadoutPartial[])
     int32_t sync;                // interpreter: remaps need barriers
-    int32_t pad2;
+    uint32_t xpass_bytes;
 };
 static_assert(sizeof(BatchItem) == 64, "shared with the kernels");
 

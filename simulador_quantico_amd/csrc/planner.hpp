@@ -85,6 +85,7 @@ struct Pass {
     int64_t mem = -1;                 // PassMem index of the register program
     int32_t phases = 0;               // register phases (LDS remaps = phases - 1)
     int64_t x_off = 0;                // interpreter's program: byte offset of its XPass in Plan::xprog
+    int32_t x_bytes = 0;              // its size
     int32_t x_stages = 0;             // its stages (LDS remaps = stages - 1)
 };
 

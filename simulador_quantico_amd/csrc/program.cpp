@@ -77,12 +77,17 @@ bool real_middle(const C v[2][2], C x[2], C *y, R o[2][2]) {
                 if (have_c[j] && !have_r[i]) { row[i] = u * std::conj(col[j]); have_r[i] = true; }
                 else if (have_r[i] && !have_c[j]) { col[j] = u * std::conj(row[i]); have_c[j] = true; }
             }
+    const C closing = v[1][1] * std::conj(row[1] * col[1]);
+    if (std::abs(closing.imag()) > 16 * 0x1p-52L * std::abs(closing)) return false;
+    if (v[0][0] != C(0, 0) && v[0][1] != C(0, 0) && v[1][0] != C(0, 0) && v[1][1] != C(0, 0)) {
+        // what the fourth phase misses by is the entries' own rounding: a quarter to each
+        const R miss = closing.imag() / closing.real();
+        row[0] *= std::polar(R(1), -miss / 4);
+        row[1] *= std::polar(R(1), miss / 4);
+        col[1] *= std::polar(R(1), miss / 2);
+    }
     for (int i = 0; i < 2; ++i)
-        for (int j = 0; j < 2; ++j) {
-            const C w = v[i][j] * std::conj(row[i] * col[j]);
-            if (std::abs(w.imag()) > 16 * 0x1p-52L * std::abs(w)) return false;
-            o[i][j] = w.real();
-        }
+        for (int j = 0; j < 2; ++j) o[i][j] = (v[i][j] * std::conj(row[i] * col[j])).real();
     x[0] = row[0];
     x[1] = row[1];
     *y = col[1];
@@ -498,6 +503,7 @@ void build(Plan &plan) {
         xp.table = (int64_t)table_at;
         const size_t at = plan.xprog.size();
         plan.xprog.resize(at + (table_at + recs.table.size() * sizeof(T) + 63) / 64 * 8, 0);
+        ps.x_bytes = (int32_t)((plan.xprog.size() - at) * 8);
         char *to = reinterpret_cast<char *>(&plan.xprog[at]);
         std::memcpy(to, &xp, sizeof xp);
         if (!recs.ops.empty()) std::memcpy(to + sizeof xp, recs.ops.data(), recs.ops.size() * sizeof(XOp<T>));
@@ -507,15 +513,21 @@ void build(Plan &plan) {
 
 // The execution shape of a plan: the plan's own threads and amplitudes per
 // thread, with more amplitudes per thread where the tuning asks for fewer than
-// a register kernel does well with, and several tiles per workgroup where a
-// tile has less than a wave.
+// the kernel does well with, and several tiles per workgroup where a tile has
+// less than a wave. 16 amplitudes per thread halve the records and the remaps
+// of 8 (default tuning, random layers: 25 qubits FP32 4 / 8 / 16 amplitudes
+// 3589 / 1938 / 1192 us, FP64 3910 / 2879 / 2484); up to 12 qubits a pass is
+// one chain of records on few waves, and 8 make each shorter (QFT at 11
+// qubits 35 / 27 / 28 us). FP64 of 13-19 qubits gains nothing either way (15
+// qubits: 92 / 96 / 94).
 ExecShape choose_shape(const Plan &plan) {
     const int r = plan.shape.r, c = plan.shape.c, n = plan.qubits;
     int a = 0;
     while ((2 << a) <= 2 * plan.shape.R) ++a;
-    const int want = plan.dtype == HGM_C64 ? 4 : 3;
-    if (n - want >= 16)
-        while (a < want && a < r - c) ++a;
+    int want = a;
+    if (n <= 12) want = 3;
+    else if (n >= 20 || plan.dtype == HGM_C64) want = 4;
+    while (a < want && a < r - c) ++a;
     ExecShape e;
     e.A = 1 << a;
     e.r = r;

@@ -361,7 +361,7 @@ int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const void 
             if (int rc = launch_jit_pass_locked(s, p, jm, pi, stream)) return rc;
         } else if (reg) {
             const XPass *xp = reinterpret_cast<const XPass *>(static_cast<const char *>(table) + ps.x_off);
-            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, s->d, xp, ps.x_stages > 1 ? tile_bytes : 0, stream),
+            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, s->d, xp, (uint32_t)ps.x_bytes, ps.x_stages > 1 ? tile_bytes : 0, stream),
                     "pass launch");
         } else {
             std::memcpy(a.local_pos, ps.local_pos, sizeof(a.local_pos));

@@ -547,7 +547,7 @@ bool launch_step(hgm_server *s, Lane &L) {
         it.tile_begin = g.tiles;
         it.partials_off = last ? (int64_t)(reinterpret_cast<char *>(dev_partials(r)) - arena) : -1;
         it.sync = r->plan.exec.sync;
-        it.pad2 = 0;
+        it.xpass_bytes = (uint32_t)ps.x_bytes;
         g.count++;
         g.tiles += tiles(r);
         if (K < 0 && ps.x_stages > 1)
