@@ -135,7 +135,8 @@ typedef struct hgm_tuning {
  * the HBM bytes one read and one write of every loaded amplitude costs. */
 typedef struct hgm_stats {
     int64_t gates;           /* gates applied (iterations included) */
-    int64_t passes;          /* kernel launches over the state */
+    int64_t passes;          /* passes over the state (launches; the interpreted kernels may run several passes of a
+                                state of up to 13 qubits in one) */
     int64_t amp_updates;     /* gates * 2^qubits */
     double bytes_alg;        /* algorithmic HBM bytes of all passes */
     double plan_ms;          /* host planning time */

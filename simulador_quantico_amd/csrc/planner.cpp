@@ -656,7 +656,7 @@ void rotate_rows(int qubits, const hgm_op *ops, int64_t n_ops, std::vector<hgm_o
 }
 
 int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iterations, const hgm_tuning &t,
-               Plan *out, std::string *err, bool program_only) {
+               Plan *out, std::string *err, bool program_only, bool pass_by_pass) {
     auto t0 = std::chrono::steady_clock::now();
     Plan plan;
     plan.qubits = qubits;
@@ -890,7 +890,7 @@ int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iter
     if (t.kernel == HGM_KERNEL_REG || t.kernel == HGM_KERNEL_JIT || (t.kernel == HGM_KERNEL_AUTO && reg_ok)) {
         plan.kernel = t.kernel == HGM_KERNEL_JIT ? HGM_KERNEL_JIT : HGM_KERNEL_REG;
         build_register_program(plan);
-        if (plan.kernel == HGM_KERNEL_REG) build_exec_program(plan);
+        if (plan.kernel == HGM_KERNEL_REG) build_exec_program(plan, pass_by_pass);
         if (plan.kernel == HGM_KERNEL_JIT) {
             // one workgroup per tile: a dispatch holds at most 2^32 - 1 work-items
             const uint64_t items = (uint64_t(1) << (qubits - plan.shape.r)) * (uint64_t)plan.shape.B;

@@ -84,9 +84,6 @@ struct Pass {
     int64_t rop_count = 0;
     int64_t mem = -1;                 // PassMem index of the register program
     int32_t phases = 0;               // register phases (LDS remaps = phases - 1)
-    int64_t x_off = 0;                // interpreter's program: byte offset of its XPass in Plan::xprog
-    int32_t x_bytes = 0;              // its size
-    int32_t x_stages = 0;             // its stages (LDS remaps = stages - 1)
 };
 
 // ---- register kernel program --------------------------------------------
@@ -154,6 +151,13 @@ struct ExecShape {
     bool sync;
 };
 
+// One launch of an interpreted kernel: a program in Plan::xprog.
+struct XLaunch {
+    int64_t off = 0;       // byte offset of its XPass
+    int32_t bytes = 0;
+    int32_t stages = 0;    // LDS remaps = stages - 1
+};
+
 struct Plan {
     int qubits = 0;
     int dtype = HGM_C128;
@@ -172,6 +176,7 @@ struct Plan {
     int max_phases = 0;
     ExecShape exec{};
     std::vector<uint64_t> xprog;      // the interpreted kernels' programs (XPass and XOp records)
+    std::vector<XLaunch> xlaunch;     // in order: one per non-empty pass, or fewer where one workgroup holds the state
     std::shared_ptr<JitCode> jit;     // HGM_KERNEL_JIT: generated and compiled pass kernels
 };
 
@@ -255,7 +260,9 @@ void fuse_gates(int qubits, const hgm_op *ops, int64_t n_ops, std::vector<hgm_op
 // tuning gets its tile shape checked and its register program built, but no
 // kernels generated or compiled: the plan (kernel HGM_KERNEL_REG) is for
 // kernels compiled from its passes' structure elsewhere (the serving engine).
+// With pass_by_pass every non-empty pass is a launch of its own (the serving
+// engine advances its states by passes).
 int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iterations, const hgm_tuning &t,
-               Plan *out, std::string *err, bool program_only = false);
+               Plan *out, std::string *err, bool program_only = false, bool pass_by_pass = false);
 
 }  // namespace hgm

@@ -350,6 +350,9 @@ struct Records {
     }
 };
 
+// Gates of one launch of a whole-state workgroup, at most (about 10 ms).
+constexpr size_t kMaxLaunchItems = size_t(1) << 15;
+
 // Runs of an ascending bit deposit: index bit j goes to state bit pos[j].
 int deposit_runs(const int *pos, int n, XRun *out, int cap) {
     int runs = 0;
@@ -363,152 +366,152 @@ int deposit_runs(const int *pos, int n, XRun *out, int cap) {
     return runs;
 }
 
+// The gates of a pass as items in tile coordinates: tile bit j is state bit
+// pos[j].
+void pass_items(const Plan &plan, const Pass &ps, const int *pos, int r, std::vector<Item> &items) {
+    int tile_of[64];
+    std::fill(tile_of, tile_of + 64, -1);
+    for (int j = 0; j < r; ++j) tile_of[pos[j]] = j;
+    for (int64_t i = 0; i < ps.op_count; ++i) {
+        const DevOp &d = plan.ops[ps.op_begin + i];
+        Item it{&d, d.kind, d.tbit, 0, 0, 0, 0, 0, 0, 0};
+        auto cond = [&](int b, uint64_t v) {   // state bit b has value v
+            if (tile_of[b] >= 0) {
+                it.lmask |= 1u << tile_of[b];
+                it.lval |= (uint32_t)v << tile_of[b];
+            } else {
+                it.gmask |= uint64_t(1) << b;
+                it.gval |= v << b;
+            }
+        };
+        for (uint32_t m = d.lmask; m; m &= m - 1) cond(ps.local_pos[__builtin_ctz(m)], (d.lval >> __builtin_ctz(m)) & 1);
+        for (uint64_t m = d.gmask; m; m &= m - 1) cond(__builtin_ctzll(m), (d.gval >> __builtin_ctzll(m)) & 1);
+        const int target = d.kind == K_DIAG_GLOBAL ? d.tbit : ps.local_pos[d.tbit];
+        if (tile_of[target] >= 0) {
+            if (d.kind == K_DIAG_GLOBAL) it.kind = K_DIAG;
+            it.tbit = tile_of[target];
+        } else {
+            it.tbit = target;
+        }
+        it.rd = it.lmask;
+        if (it.kind == K_DENSE || it.kind == K_ANTI) it.need = it.wr = 1u << it.tbit;
+        else if (it.kind == K_DIAG) {
+            it.rd |= 1u << it.tbit;
+            if (plan.pre_phase[ps.op_begin + i]) it.need = it.wr = 1u << it.tbit;
+        }
+        items.push_back(it);
+    }
+}
+
+// Appends the program of one launch: `items` on tiles of 2^rx amplitudes whose
+// bit j is state bit pos[j]; gates mix the first r tile bits only, and the
+// first c stay on consecutive threads at the load and the store.
 template <class T>
-void build(Plan &plan) {
+void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c) {
     constexpr int F = sizeof(T) == 4 ? 5 : 4;
     const ExecShape &ex = plan.exec;
-    const int r = plan.shape.r, c = plan.shape.c, rx = ex.r, n = plan.qubits;
+    const int n = plan.qubits;
     int a = 0;
     while ((1 << a) < ex.A) ++a;
     const uint32_t own = (uint32_t)((uint64_t(1) << r) - 1);
     const uint32_t forbid = (r - c >= a) ? (uint32_t)((1u << c) - 1) : 0u;
-    plan.xprog.clear();
-    std::vector<Item> items;
+    uint64_t local = 0;
+    for (int j = 0; j < rx; ++j) local |= uint64_t(1) << pos[j];
     std::vector<ROp> ops;
-    for (Pass &ps : plan.passes) {
-        // tile bits of the execution shape: the plan's, then the lowest non-local state bits
-        int pos[32];
-        for (int j = 0; j < r; ++j) pos[j] = ps.local_pos[j];
-        uint64_t local = ps.local_mask;
-        for (int j = r, b = 0; j < rx; ++b)
-            if (!((local >> b) & 1)) { pos[j++] = b; local |= uint64_t(1) << b; }
-        int tile_of[64];
-        std::fill(tile_of, tile_of + 64, -1);
-        for (int j = r; j < rx; ++j) tile_of[pos[j]] = j;
-        items.clear();
-        for (int64_t i = 0; i < ps.op_count; ++i) {
-            const DevOp &d = plan.ops[ps.op_begin + i];
-            Item it{&d, d.kind, d.tbit, d.lmask, d.lval, 0, 0, 0, 0, 0};
-            for (uint64_t g = d.gmask; g; g &= g - 1) {
-                const int b = __builtin_ctzll(g);
-                const uint64_t v = (d.gval >> b) & 1;
-                if (tile_of[b] >= 0) {
-                    it.lmask |= 1u << tile_of[b];
-                    it.lval |= (uint32_t)v << tile_of[b];
-                } else {
-                    it.gmask |= uint64_t(1) << b;
-                    it.gval |= v << b;
-                }
+    // stages: the same greedy as the pass planner, with the tile as the state and the register bits as the
+    // tile; the first and last keep the coalesced bits on the threads
+    std::vector<uint32_t> sets;
+    std::vector<std::vector<int>> lists;
+    std::vector<char> done(items.size(), 0);
+    for (size_t head = 0; head < items.size();) {
+        uint32_t S = 0, bw = 0, br = 0;
+        int nS = 0;
+        std::vector<int> list;
+        for (size_t k = head; k < items.size(); ++k) {
+            if (done[k]) continue;
+            const Item &it = items[k];
+            bool ok = !(it.wr & (bw | br)) && !(it.rd & bw);
+            if (ok && (it.need & ~S)) {
+                if (nS < a && !(sets.empty() && (it.need & forbid))) { S |= it.need; ++nS; }
+                else ok = false;
             }
-            if (it.kind == K_DIAG_GLOBAL && tile_of[it.tbit] >= 0) {
-                it.kind = K_DIAG;
-                it.tbit = tile_of[it.tbit];
-            }
-            it.rd = it.lmask;
-            if (it.kind == K_DENSE || it.kind == K_ANTI) it.need = it.wr = 1u << it.tbit;
-            else if (it.kind == K_DIAG) {
-                it.rd |= 1u << it.tbit;
-                if (plan.pre_phase[ps.op_begin + i]) it.need = it.wr = 1u << it.tbit;
-            }
-            items.push_back(it);
+            if (ok) { list.push_back((int)k); done[k] = 1; }
+            else { bw |= it.wr; br |= it.rd; if ((bw & own) == own) break; }
         }
-        // stages: the same greedy as the pass planner, with the tile as the state and the register bits as the
-        // tile; the first and last keep the coalesced bits on the threads
-        std::vector<uint32_t> sets;
-        std::vector<std::vector<int>> lists;
-        std::vector<char> done(items.size(), 0);
-        for (size_t head = 0; head < items.size();) {
-            uint32_t S = 0, bw = 0, br = 0;
-            int nS = 0;
-            std::vector<int> list;
-            for (size_t k = head; k < items.size(); ++k) {
-                if (done[k]) continue;
-                const Item &it = items[k];
-                bool ok = !(it.wr & (bw | br)) && !(it.rd & bw);
-                if (ok && (it.need & ~S)) {
-                    if (nS < a && !(sets.empty() && (it.need & forbid))) { S |= it.need; ++nS; }
-                    else ok = false;
-                }
-                if (ok) { list.push_back((int)k); done[k] = 1; }
-                else { bw |= it.wr; br |= it.rd; if ((bw & own) == own) break; }
-            }
-            while (head < items.size() && done[head]) ++head;
-            sets.push_back(S);
-            lists.push_back(std::move(list));
-        }
-        if (sets.empty() || (sets.back() & forbid)) { sets.push_back(0); lists.emplace_back(); }
-        for (size_t i = 0; i < sets.size(); ++i) {
-            const bool edge = i == 0 || i + 1 == sets.size();
-            for (int b = r - 1; b >= 0 && popc(sets[i]) < a; --b)
-                if (!((sets[i] >> b) & 1) && !(edge && ((forbid >> b) & 1))) sets[i] |= 1u << b;
-            for (int b = r - 1; b >= 0 && popc(sets[i]) < a; --b) sets[i] |= 1u << b;
-        }
-        // records
-        auto map_of = [&](uint32_t S) {
-            XMap m;
-            std::memset(&m, 0, sizeof m);
-            int i = 0;
-            for (int b = 0; b < rx; ++b)
-                if ((S >> b) & 1) {
-                    m.low[i] = (uint16_t)((1u << b) - 1);
-                    m.sw[i++] = (uint16_t)x_swizzle<F>(1u << b);
-                }
-            return m;
-        };
-        Records<T> recs;
-        recs.A = (uint32_t)ex.A;
-        uint32_t flip = 0;
-        for (size_t i = 0; i < sets.size(); ++i) {
-            if (i > 0) {
-                XOp<T> x;
-                std::memset(&x, 0, sizeof x);
-                x.kind = X_REMAP;
-                const XMap m = map_of(sets[i]);
-                std::memcpy(x.m, &m, sizeof m);
-                recs.ops.push_back(x);
-            }
-            ops.clear();
-            for (int k : lists[i]) {
-                emit(items[k], sets[i], flip, recs.scale, ops);
-                if (ops.size() >= 64) { recs.stage(ops); recs.flush(false); ops.clear(); }
-            }
-            recs.stage(ops);
-            recs.flush(i + 1 == sets.size());
-        }
-        XPass xp;
-        std::memset(&xp, 0, sizeof xp);
-        xp.n_ops = (int32_t)recs.ops.size();
-        xp.first = map_of(sets.front());
-        auto lanes = [&](uint32_t S, uint64_t *bit, XRun *runs) {
-            int p[32], np = 0, i = 0;
-            for (int b = 0; b < rx; ++b) {
-                if ((S >> b) & 1) bit[i++] = uint64_t(1) << pos[b];
-                else p[np++] = pos[b];
-            }
-            return deposit_runs(p, np, runs, kXLaneRuns);
-        };
-        xp.n_load = lanes(sets.front(), xp.lbit, xp.load);
-        xp.n_store = lanes(sets.back(), xp.sbit, xp.store);
-        for (int b = 0; b < rx; ++b)
-            if ((flip >> b) & 1) ((sets.back() >> b) & 1 ? xp.rflip : xp.sflip) |= uint64_t(1) << pos[b];
-        int p[64], np = 0;
-        for (int b = 0; b < n; ++b)
-            if (!((local >> b) & 1)) p[np++] = b;
-        xp.n_base = deposit_runs(p, np, xp.base, kXBaseRuns);
-        ps.x_stages = (int32_t)sets.size();
-        ps.x_off = (int64_t)(plan.xprog.size() * 8);
-        // one zero record past the end (the kernel loads ahead), then the factor table
-        const size_t op_bytes = (recs.ops.size() + 1) * sizeof(XOp<T>);
-        const size_t table_at = (sizeof(XPass) + op_bytes + 63) / 64 * 64;
-        xp.table = (int64_t)table_at;
-        const size_t at = plan.xprog.size();
-        plan.xprog.resize(at + (table_at + recs.table.size() * sizeof(T) + 63) / 64 * 8, 0);
-        ps.x_bytes = (int32_t)((plan.xprog.size() - at) * 8);
-        char *to = reinterpret_cast<char *>(&plan.xprog[at]);
-        std::memcpy(to, &xp, sizeof xp);
-        if (!recs.ops.empty()) std::memcpy(to + sizeof xp, recs.ops.data(), recs.ops.size() * sizeof(XOp<T>));
-        if (!recs.table.empty()) std::memcpy(to + table_at, recs.table.data(), recs.table.size() * sizeof(T));
+        while (head < items.size() && done[head]) ++head;
+        sets.push_back(S);
+        lists.push_back(std::move(list));
     }
+    if (sets.empty() || (sets.back() & forbid)) { sets.push_back(0); lists.emplace_back(); }
+    for (size_t i = 0; i < sets.size(); ++i) {
+        const bool edge = i == 0 || i + 1 == sets.size();
+        for (int b = r - 1; b >= 0 && popc(sets[i]) < a; --b)
+            if (!((sets[i] >> b) & 1) && !(edge && ((forbid >> b) & 1))) sets[i] |= 1u << b;
+        for (int b = r - 1; b >= 0 && popc(sets[i]) < a; --b) sets[i] |= 1u << b;
+    }
+    // records
+    auto map_of = [&](uint32_t S) {
+        XMap m;
+        std::memset(&m, 0, sizeof m);
+        int i = 0;
+        for (int b = 0; b < rx; ++b)
+            if ((S >> b) & 1) {
+                m.low[i] = (uint16_t)((1u << b) - 1);
+                m.sw[i++] = (uint16_t)x_swizzle<F>(1u << b);
+            }
+        return m;
+    };
+    Records<T> recs;
+    recs.A = (uint32_t)ex.A;
+    uint32_t flip = 0;
+    for (size_t i = 0; i < sets.size(); ++i) {
+        if (i > 0) {
+            XOp<T> x;
+            std::memset(&x, 0, sizeof x);
+            x.kind = X_REMAP;
+            const XMap m = map_of(sets[i]);
+            std::memcpy(x.m, &m, sizeof m);
+            recs.ops.push_back(x);
+        }
+        ops.clear();
+        for (int k : lists[i]) {
+            emit(items[k], sets[i], flip, recs.scale, ops);
+            if (ops.size() >= 64) { recs.stage(ops); recs.flush(false); ops.clear(); }
+        }
+        recs.stage(ops);
+        recs.flush(i + 1 == sets.size());
+    }
+    XPass xp;
+    std::memset(&xp, 0, sizeof xp);
+    xp.n_ops = (int32_t)recs.ops.size();
+    xp.first = map_of(sets.front());
+    auto lanes = [&](uint32_t S, uint64_t *bit, XRun *runs) {
+        int p[32], np = 0, i = 0;
+        for (int b = 0; b < rx; ++b) {
+            if ((S >> b) & 1) bit[i++] = uint64_t(1) << pos[b];
+            else p[np++] = pos[b];
+        }
+        return deposit_runs(p, np, runs, kXLaneRuns);
+    };
+    xp.n_load = lanes(sets.front(), xp.lbit, xp.load);
+    xp.n_store = lanes(sets.back(), xp.sbit, xp.store);
+    for (int b = 0; b < rx; ++b)
+        if ((flip >> b) & 1) ((sets.back() >> b) & 1 ? xp.rflip : xp.sflip) |= uint64_t(1) << pos[b];
+    int p[64], np = 0;
+    for (int b = 0; b < n; ++b)
+        if (!((local >> b) & 1)) p[np++] = b;
+    xp.n_base = deposit_runs(p, np, xp.base, kXBaseRuns);
+    // one zero record past the end (the kernel loads ahead), then the factor table
+    const size_t op_bytes = (recs.ops.size() + 1) * sizeof(XOp<T>);
+    const size_t table_at = (sizeof(XPass) + op_bytes + 63) / 64 * 64;
+    xp.table = (int64_t)table_at;
+    const size_t at = plan.xprog.size();
+    plan.xprog.resize(at + (table_at + recs.table.size() * sizeof(T) + 63) / 64 * 8, 0);
+    plan.xlaunch.push_back({(int64_t)(at * 8), (int32_t)((plan.xprog.size() - at) * 8), (int32_t)sets.size()});
+    char *to = reinterpret_cast<char *>(&plan.xprog[at]);
+    std::memcpy(to, &xp, sizeof xp);
+    if (!recs.ops.empty()) std::memcpy(to + sizeof xp, recs.ops.data(), recs.ops.size() * sizeof(XOp<T>));
+    if (!recs.table.empty()) std::memcpy(to + table_at, recs.table.data(), recs.table.size() * sizeof(T));
 }
 
 // The execution shape of a plan: the plan's own threads and amplitudes per
@@ -520,13 +523,14 @@ void build(Plan &plan) {
 // one chain of records on few waves, and 8 make each shorter (QFT at 11
 // qubits 35 / 27 / 28 us). FP64 of 13-19 qubits gains nothing either way (15
 // qubits: 92 / 96 / 94).
-ExecShape choose_shape(const Plan &plan) {
-    const int r = plan.shape.r, c = plan.shape.c, n = plan.qubits;
+ExecShape choose_shape(const Plan &plan, bool whole) {
+    const int n = plan.qubits, r = whole ? n : plan.shape.r, c = std::min(plan.shape.c, r);
     int a = 0;
     while ((2 << a) <= 2 * plan.shape.R) ++a;
     int want = a;
     if (n <= 12) want = 3;
     else if (n >= 20 || plan.dtype == HGM_C64) want = 4;
+    if (whole) a = std::max(a, n <= 12 ? std::min(3, n) : 4);
     while (a < want && a < r - c) ++a;
     ExecShape e;
     e.A = 1 << a;
@@ -537,12 +541,48 @@ ExecShape choose_shape(const Plan &plan) {
     return e;
 }
 
+// Whether one workgroup runs the whole state, all passes in one launch: their
+// launches cost about 5 us each, and merged passes share remaps, while a pass
+// on its own spreads its tiles over workgroups. Default tuning, FP32, passes
+// on their own against one launch: Grover (8 iterations, 10-17 passes) at 9 /
+// 11 / 13 qubits 108 / 115 / 182 against 47 / 71 / 112 us, random layers (3-5
+// passes) 32 / 38 / 48 against 27 / 36 / 46, QFT (2-3 passes) 19 / 25 / 35
+// against 17 / 24 / 38.
+bool whole_state(const Plan &plan) {
+    int64_t passes = 0;
+    for (const Pass &ps : plan.passes) passes += ps.op_count > 0;
+    return passes > 1 && (plan.qubits <= 11 || (plan.qubits <= 13 && passes >= 6));
+}
+
 }  // namespace
 
-void build_exec_program(Plan &plan) {
-    plan.exec = choose_shape(plan);
-    if (plan.dtype == HGM_C64) build<float>(plan);
-    else build<double>(plan);
+void build_exec_program(Plan &plan, bool pass_by_pass) {
+    const bool whole = !pass_by_pass && whole_state(plan);
+    plan.exec = choose_shape(plan, whole);
+    plan.xprog.clear();
+    plan.xlaunch.clear();
+    const int n = plan.qubits, r = whole ? n : plan.shape.r, rx = plan.exec.r;
+    std::vector<Item> items;
+    int pos[32];
+    auto launch = [&] {
+        if (plan.dtype == HGM_C64) build<float>(plan, items, pos, r, rx, std::min(plan.shape.c, r));
+        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r));
+        items.clear();
+    };
+    for (const Pass &ps : plan.passes) {
+        if (!ps.op_count) {
+            if (pass_by_pass) plan.xlaunch.push_back({});   // launches are indexed by pass there
+            continue;
+        }
+        // tile bits: the state's, or the plan's, then the lowest non-local ones
+        uint64_t local = 0;
+        for (int j = 0; j < r; ++j) pos[j] = whole ? j : ps.local_pos[j], local |= uint64_t(1) << pos[j];
+        for (int j = r, b = 0; j < rx; ++b)
+            if (!((local >> b) & 1)) { pos[j++] = b; local |= uint64_t(1) << b; }
+        pass_items(plan, ps, pos, rx, items);
+        if (!whole || items.size() >= kMaxLaunchItems) launch();
+    }
+    if (!items.empty()) launch();
 }
 
 }  // namespace hgm

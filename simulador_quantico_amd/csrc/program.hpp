@@ -106,8 +106,9 @@ constexpr uint32_t x_swizzle(uint32_t x) {
     return x ^ ((x >> F) & M) ^ ((x >> (2 * F)) & M) ^ ((x >> (3 * F)) & M);
 }
 
-// Chooses the execution shape (plan.exec) and builds plan.xprog and every
-// pass's x_off / x_stages.
-void build_exec_program(Plan &plan);
+// Chooses the execution shape (plan.exec) and builds plan.xprog and
+// plan.xlaunch: one launch per non-empty pass, or, unless pass_by_pass, whole
+// runs of passes where the state fits one workgroup.
+void build_exec_program(Plan &plan, bool pass_by_pass);
 
 }  // namespace hgm

@@ -352,17 +352,22 @@ int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const void 
     a.r = p.shape.r; a.c = p.shape.c; a.B = p.shape.B; a.R = p.shape.R;
     a.n_tiles = int64_t(1) << (p.qubits - p.shape.r);
     const uint64_t all = (uint64_t(1) << p.qubits) - 1;
-    const size_t tile_bytes = reg ? (size_t(1) << p.exec.r) * amp_bytes(p.dtype) : 0;
+    if (reg) {
+        const size_t tile_bytes = (size_t(1) << p.exec.r) * amp_bytes(p.dtype);
+        for (const XLaunch &x : p.xlaunch) {
+            const XPass *xp = reinterpret_cast<const XPass *>(static_cast<const char *>(table) + x.off);
+            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, s->d, xp, (uint32_t)x.bytes, x.stages > 1 ? tile_bytes : 0,
+                                    stream),
+                    "pass launch");
+        }
+        return HGM_OK;
+    }
     for (size_t pi = 0; pi < p.passes.size(); ++pi) {
         const Pass &ps = p.passes[pi];
         if (ps.op_count == 0) continue;
         a.nonlocal_mask = all & ~ps.local_mask;
         if (jit) {
             if (int rc = launch_jit_pass_locked(s, p, jm, pi, stream)) return rc;
-        } else if (reg) {
-            const XPass *xp = reinterpret_cast<const XPass *>(static_cast<const char *>(table) + ps.x_off);
-            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, s->d, xp, (uint32_t)ps.x_bytes, ps.x_stages > 1 ? tile_bytes : 0, stream),
-                    "pass launch");
         } else {
             std::memcpy(a.local_pos, ps.local_pos, sizeof(a.local_pos));
             HGM_HIP(launch_pass_lds(p.dtype, s->d, static_cast<const DevOp *>(table) + ps.op_begin, (int)ps.op_count, a,

@@ -388,8 +388,8 @@ void planner_loop(hgm_server *s) {
             lt = s->large[r->qubits];
         }
         std::string err;
-        int rc = build_plan(r->qubits, s->cfg.dtype, r->ops.data(), (int64_t)r->ops.size(), r->iterations, t,
-                            &r->plan, &err);
+    int rc = build_plan(r->qubits, s->cfg.dtype, r->ops.data(), (int64_t)r->ops.size(), r->iterations, t,
+                            &r->plan, &err, false, true);
         if (rc == HGM_OK && r->plan.kernel != HGM_KERNEL_REG) {
             rc = HGM_E_TUNING;
             err = "serving needs the register kernel for this tile shape";
@@ -542,15 +542,16 @@ bool launch_step(hgm_server *s, Lane &L) {
         char *const arena = s->arena.base();
         it.state_off = (uint64_t)(r->d - arena);
         it.ops_off = (uint64_t)(reinterpret_cast<char *>(dev_rops(r) + ps.rop_begin) - arena);
-        it.xpass_off = (uint64_t)(dev_xprog(r) + ps.x_off - arena);
+        const XLaunch x = K < 0 ? r->plan.xlaunch[r->passes[r->next]] : XLaunch{};
+        it.xpass_off = (uint64_t)(dev_xprog(r) + x.off - arena);
         it.pad[0] = it.pad[1] = 0;
         it.tile_begin = g.tiles;
         it.partials_off = last ? (int64_t)(reinterpret_cast<char *>(dev_partials(r)) - arena) : -1;
         it.sync = r->plan.exec.sync;
-        it.xpass_bytes = (uint32_t)ps.x_bytes;
+        it.xpass_bytes = (uint32_t)x.bytes;
         g.count++;
         g.tiles += tiles(r);
-        if (K < 0 && ps.x_stages > 1)
+        if (K < 0 && x.stages > 1)
             g.lds = std::max(g.lds, (size_t(1) << r->plan.exec.r) * amp_bytes(s->cfg.dtype));
         if (last) {
             tasks[n_tasks].partials = dev_partials(r);
@@ -866,7 +867,7 @@ int hgm_server_precompile(hgm_server *s, int qubits, const hgm_op *ops, int64_t 
     }
     Plan plan, large;
     std::string err;
-    int rc = build_plan(qubits, s->cfg.dtype, ops, n_ops, iterations, t, &plan, &err);
+    int rc = build_plan(qubits, s->cfg.dtype, ops, n_ops, iterations, t, &plan, &err, false, true);
     if (rc) { set_error(err); return rc; }
     if (plan.kernel != HGM_KERNEL_REG) { set_error("serving needs the register kernel for this tile shape"); return HGM_E_TUNING; }
     auto busy = [](const Plan &p) {
