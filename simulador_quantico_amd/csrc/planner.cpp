@@ -3,6 +3,7 @@
 
 #include <complex>
 
+#include <atomic>
 #include <chrono>
 #include <cstring>
 
@@ -658,7 +659,9 @@ void rotate_rows(int qubits, const hgm_op *ops, int64_t n_ops, std::vector<hgm_o
 int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iterations, const hgm_tuning &t,
                Plan *out, std::string *err, bool program_only, bool pass_by_pass) {
     auto t0 = std::chrono::steady_clock::now();
+    static std::atomic<uint64_t> builds{0};
     Plan plan;
+    plan.id = ++builds;
     plan.qubits = qubits;
     plan.dtype = dtype;
     int st = make_shape(qubits, dtype, t, &plan.shape, err);

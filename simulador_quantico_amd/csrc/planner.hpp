@@ -162,6 +162,7 @@ struct Plan {
     int qubits = 0;
     int dtype = HGM_C128;
     int kernel = HGM_KERNEL_LDS;
+    uint64_t id = 0;                  // of this build (nonzero, unique in the process)
     TileShape shape{};
     std::vector<Pass> passes;
     std::vector<DevOp> ops;

@@ -86,6 +86,19 @@ namespace {
 
 thread_local std::string t_err;
 
+// Device copy of a plan's table (grow-only). The last kProgSlots plans keep
+// theirs, so that a plan that runs again launches at once; another plan takes
+// the slot that was used longest ago. Plans are told apart by their build
+// (Plan::id), never by address. Runs are synchronous under the context lock,
+// so no kernel reads a slot that is being rewritten.
+struct ProgSlot {
+    void *buf = nullptr;
+    size_t cap = 0;
+    uint64_t plan = 0;          // 0: none
+    uint64_t use = 0;
+};
+constexpr int kProgSlots = 8;
+
 struct Ctx {
     std::mutex mu;
     bool ready = false;
@@ -93,8 +106,8 @@ struct Ctx {
     hipStream_t stream = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr, e4 = nullptr, e5 = nullptr;
     int cus = 0;
-    void *prog = nullptr;       // register-kernel programs or op tables of the current call (grow-only)
-    size_t prog_cap = 0;
+    ProgSlot prog[kProgSlots];  // register-kernel programs or op tables of the plans that ran last
+    uint64_t prog_tick = 0;
     void *cache = nullptr;      // device buffer of hgm_execute (grow-only)
     size_t cache_cap = 0;
     // reduction partials, in pinned host memory that the kernels write directly
@@ -157,6 +170,13 @@ int hip_fail(hipError_t e, const char *what) {
         if (e_ != hipSuccess) return hip_fail(e_, what); \
     } while (0)
 
+void drop_programs(Ctx &c) {
+    for (ProgSlot &p : c.prog) {
+        if (p.buf) hipFree(p.buf);
+        p = ProgSlot{};
+    }
+}
+
 int init_locked(int device) {
     Ctx &c = ctx();
     if (c.ready && (device < 0 || device == c.device)) return HGM_OK;
@@ -171,6 +191,7 @@ int init_locked(int device) {
     if (c.stream) {   // re-init on another device
         hipStreamDestroy(c.stream);
         c.stream = nullptr;
+        drop_programs(c);
     }
     HGM_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking), "hipStreamCreate");
     for (hipEvent_t *e : {&c.e0, &c.e1, &c.e2, &c.e3, &c.e4, &c.e5}) {
@@ -395,12 +416,28 @@ int run_plan_locked(hgm_state *s, const Plan &p, hgm_stats *st, double plan_ms, 
         if ((rc = jit_load_locked(*p.jit, &jm))) return rc;
     } else {
         const size_t bytes = plan_table_bytes(p);
+        bool there = false;
         if (!table) {
-            if ((rc = reserve(&c.prog, &c.prog_cap, bytes, "hipMalloc(programs)"))) return rc;
-            table = c.prog;
+            ProgSlot *slot = c.prog;
+            for (ProgSlot &q : c.prog) {
+                if (q.plan == p.id) { slot = &q; break; }
+                if (q.use < slot->use) slot = &q;
+            }
+            there = slot->plan == p.id;
+            if (!there) {
+                slot->plan = 0;
+                if ((rc = reserve(&slot->buf, &slot->cap, bytes, "hipMalloc(programs)"))) return rc;
+            }
+            table = slot->buf;
+            slot->use = ++c.prog_tick;
+            if (!there && bytes)
+                HGM_HIP(hipMemcpyAsync(table, plan_table(p), bytes, hipMemcpyHostToDevice, c.stream),
+                        "hipMemcpyAsync(programs)");
+            slot->plan = p.id;
+        } else if (bytes) {
+            HGM_HIP(hipMemcpyAsync(table, plan_table(p), bytes, hipMemcpyHostToDevice, c.stream),
+                    "hipMemcpyAsync(programs)");
         }
-        if (bytes) HGM_HIP(hipMemcpyAsync(table, plan_table(p), bytes, hipMemcpyHostToDevice, c.stream),
-                           "hipMemcpyAsync(programs)");
     }
     HGM_HIP(hipEventRecord(c.e0, c.stream), "hipEventRecord");
     if ((rc = launch_passes_locked(s, p, jm, table, c.stream))) return rc;
@@ -639,7 +676,7 @@ int hgm_release_cache(void) {
         *cap = 0;
     };
     drop(&c.cache, &c.cache_cap);
-    drop(&c.prog, &c.prog_cap);
+    drop_programs(c);
     for (char *&h : c.h_stage) {
         if (h) hipHostFree(h);
         h = nullptr;
