@@ -283,11 +283,13 @@ double hgm_plan_compile_seconds(const hgm_plan *p);
 
 /* A batch of n resident states of any qubit counts, state i advanced by the
  * plan plans[i] (any kernel family: the tables of register and LDS plans are
- * copied to the device once, here), captured as one hipGraph: the graph forks
- * into up to 64 branches (one per state; beyond 64 states, spread over them
- * by their plans' bytes, largest first), each branch runs its states' passes
- * in order, and the branches join, so passes of different states can run at
- * once. One
+ * copied to the device once, here), captured as one hipGraph: states whose
+ * plans launch the same kernels with the same programs (one plan shared by
+ * many states, or equal plans) advance together, one launch per pass for all
+ * of them; the graph forks into up to 64 branches (one per such group, more
+ * spread over them by their plans' bytes, largest first), each branch runs its
+ * groups' passes in order, and the branches join, so passes of different
+ * groups can run at once. One
  * hgm_batch_run is one graph launch for the whole batch. States must be
  * distinct and match their plan's qubit count and dtype; the plan-compiled
  * plans' modules (at most 16 distinct) are kept loaded while the batch runs,

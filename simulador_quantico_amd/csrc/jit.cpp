@@ -257,7 +257,8 @@ std::string kernel_body(const Gen &g, const Plan &plan, const Pass &ps, const st
     }
     std::string o;
     o += "extern \"C\" __global__ void __launch_bounds__(" + std::to_string(B) + ") " + name + "(" + g.V +
-         " *__restrict__ s) {\n";
+         " *__restrict__ s, const long long *__restrict__ offs) {\n";
+    o += "    if (offs) s = (" + g.V + " *)((char *)s + offs[blockIdx.y]);\n";   // one of several states
     if (ps.phases > 1) o += "    extern __shared__ " + (g.split ? g.T : g.V) + " lds[];\n";
     o += "    const unsigned t = threadIdx.x;\n";
     o += "    const unsigned long long lt = " + thread_or(lt, tb) + ";\n";

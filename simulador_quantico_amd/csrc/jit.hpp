@@ -27,7 +27,9 @@ struct JitCode {
     double compile_s = 0;
 };
 
-// Generates the source of every pass kernel of a register-kernel plan.
+// Generates the source of every pass kernel of a register-kernel plan. The
+// kernels take the state and, for one launch over several states, their byte
+// offsets from it (state blockIdx.y; null: the state itself).
 void jit_generate(const Plan &plan, JitCode *out);
 
 // Compiles out->source with hipRTC for gfx950 (cached by source hash within

@@ -432,9 +432,10 @@ constexpr uint32_t kStreamLoads = 1, kStreamStores = 2, kBarriers = 4;
 
 template <class T, int A>
 __global__ void __launch_bounds__(reg_kernel_max_threads(A, sizeof(typename Vec<T>::type)))
-    k_pass_reg(typename Vec<T>::type *__restrict__ state, const XPass *__restrict__ xp, uint32_t xp_bytes, int64_t n_tiles,
-               uint32_t mode) {
+    k_pass_reg(typename Vec<T>::type *__restrict__ state, const int64_t *__restrict__ offs, const XPass *__restrict__ xp,
+               uint32_t xp_bytes, int64_t n_tiles, uint32_t mode) {
     using V = typename Vec<T>::type;
+    if (offs) state = reinterpret_cast<V *>(reinterpret_cast<char *>(state) + offs[blockIdx.y]);
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t t = threadIdx.x;
     const uint32_t warm = warm_program(xp, xp_bytes, blockIdx.x);
@@ -761,17 +762,17 @@ hipError_t pass_lds(void *state, const DevOp *ops, int n_ops, const PassArgs &a,
 }
 
 template <class T, int A>
-hipError_t pass_reg(void *state, const XPass *xp, uint32_t xp_bytes, int64_t n_tiles, int B, size_t lds, uint32_t mode,
-                    hipStream_t s) {
+hipError_t pass_reg(const StateSet &set, const XPass *xp, uint32_t xp_bytes, int64_t n_tiles, int B, size_t lds,
+                    uint32_t mode, hipStream_t s) {
     pass_reg_attr<T, A>();
-    const int64_t grid = tile_grid(n_tiles, B);
-    hipLaunchKernelGGL((k_pass_reg<T, A>), dim3((unsigned)grid), dim3(B), lds, s,
-                       reinterpret_cast<typename Vec<T>::type *>(state), xp, xp_bytes, n_tiles, mode);
+    const int64_t grid = tile_grid(n_tiles, B * set.count);
+    hipLaunchKernelGGL((k_pass_reg<T, A>), dim3((unsigned)grid, (unsigned)set.count), dim3(B), lds, s,
+                       reinterpret_cast<typename Vec<T>::type *>(set.first), set.offs, xp, xp_bytes, n_tiles, mode);
     return hipGetLastError();
 }
 
 template <class T>
-hipError_t pass_reg_any(int A, void *state, const XPass *xp, uint32_t xp_bytes, int64_t n_tiles, int B, size_t lds,
+hipError_t pass_reg_any(int A, const StateSet &state, const XPass *xp, uint32_t xp_bytes, int64_t n_tiles, int B, size_t lds,
                         uint32_t mode, hipStream_t s) {
     switch (A) {
         case 2: return pass_reg<T, 2>(state, xp, xp_bytes, n_tiles, B, lds, mode, s);
@@ -811,9 +812,9 @@ hipError_t batch_reg_any(int A, const BatchItem *items, int n_items, int64_t tot
 
 }  // namespace
 
-hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, void *state, const XPass *xp, uint32_t xp_bytes,
-                           size_t lds_bytes, hipStream_t s) {
-    const size_t bytes = (size_t(1) << qubits) * amp_bytes(dtype);
+hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, const StateSet &state, const XPass *xp,
+                           uint32_t xp_bytes, size_t lds_bytes, hipStream_t s) {
+    const size_t bytes = (size_t(1) << qubits) * amp_bytes(dtype) * (size_t)state.count;
     bool ld, st;
     state_streams(bytes, &ld, &st);
     const uint32_t mode = (ld ? kStreamLoads : 0) | (st ? kStreamStores : 0) | (e.sync ? kBarriers : 0);

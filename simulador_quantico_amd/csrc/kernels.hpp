@@ -27,11 +27,19 @@ hipError_t launch_pass_lds(int dtype, void *state, const DevOp *ops, int n_ops, 
 // launches into a graph.
 hipError_t prepare_pass_kernels(int dtype);
 
+// The states of one launch: `count` of one size and type, at byte offsets
+// offs[i] (device memory) from `first`; offs null: the one state.
+struct StateSet {
+    void *first;
+    const int64_t *offs = nullptr;
+    int count = 1;
+};
+
 // One full-state pass of the register kernel: the program of xp_bytes bytes at
-// xp (device) on a state of `qubits` qubits in execution shape e; lds_bytes is
+// xp (device) on states of `qubits` qubits in execution shape e; lds_bytes is
 // 0 for a pass of one stage.
-hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, void *state, const XPass *xp, uint32_t xp_bytes,
-                           size_t lds_bytes, hipStream_t s);
+hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, const StateSet &states, const XPass *xp,
+                           uint32_t xp_bytes, size_t lds_bytes, hipStream_t s);
 
 // Readout of one tile or of a whole state: FP64 sum of |a|^2 and the largest
 // |a|^2 with its index (lowest index on ties).

@@ -256,7 +256,7 @@ void state_streams(size_t bytes, bool *loads, bool *stores) {
     const size_t mib = size_t(1) << 20;
     const bool cached = bytes >= 64 * mib && bytes <= 256 * mib;
     *loads = !cached && bytes > 8 * mib;
-    *stores = !cached;
+    *stores = !cached && bytes > 4 * mib;
 }
 
 int make_shape(int qubits, int dtype, const hgm_tuning &t, TileShape *out, std::string *err) {

@@ -202,9 +202,10 @@ size_t amp_bytes(int dtype);
 // where the hint is worth 3-5% (26 qubits 41.3 against 42.7 ms). 16-32 MiB:
 // about the 32 MiB of the eight L2s, whose dirty lines every kernel boundary
 // writes back; with the hint they leave early (20 qubits 642 against 738 us).
-// Up to 8 MiB plain loads hit the L2s (16 qubits 305 -> 273 us), and the
-// stores keep the hint (20 qubits FP32, 8 MiB: 572 us; stores plain too 607;
-// both with the hint 587).
+// Up to 8 MiB plain loads hit the L2s (16 qubits 305 -> 273 us); at 8 MiB the
+// stores keep the hint (20 qubits FP32: 572 us; stores plain too 607; both
+// with the hint 587), below it makes no difference to one state, and a batch
+// of small states as a whole lives in the last-level cache.
 void state_streams(size_t bytes, bool *loads, bool *stores);
 
 // Validates a tuning tuple (the reference's rules of src/core/dgm_core.cpp:177-241

@@ -55,21 +55,32 @@ struct hgm_plan {
     }
 };
 
+// States of a batch that run the same kernels: one launch per pass advances
+// all of them.
+struct BatchGroup {
+    std::vector<int> members;     // state indices; the group's plan is the first one's
+    int branch = 0;
+    int64_t table_off = -1;       // device copy of a register or LDS plan's table (byte offset in tables)
+    int64_t offs_off = -1;        // the members' byte offsets from the first state (byte offset in tables)
+};
+
 // A batch of states advanced by their plans as one captured graph
-// (hgm_batch_create): branch[i] is the fork branch of state i. 64 states of
-// 12-19 qubits (Grover, 1016 passes) replay in 3.78 ms on 4 branches, 3.14 ms
-// on 16 and 2.91 ms on 64, against 7.1 ms plan by plan.
+// (hgm_batch_create). A graph node costs about 2 us whatever it launches, so
+// states with the same plan share their launches: 64 FP32 states of 12-19
+// qubits, 8 of each size (Grover, 960 passes), replay in 0.68 ms as 120
+// nodes against 2.1 ms as 960 nodes on 64 branches. Groups run side by side,
+// one branch each (the 8 groups of that batch on 1 / 2 / 4 branches: 1.05 /
+// 0.94 / 0.74 ms).
 constexpr int kBatchBranches = 64;
 struct hgm_batch {
     std::vector<hgm_state *> states;
     std::vector<const hgm_plan *> plans;
-    std::vector<int> branch;
+    std::vector<BatchGroup> groups;
     int n_branches = 0;
     hipStream_t streams[kBatchBranches] = {};
     hipEvent_t fork = nullptr, join[kBatchBranches] = {};
     std::vector<uint64_t> gens;   // load generation of each plan's module when the graph was captured
-    void *tables = nullptr;       // device copies of the register / LDS plans' tables
-    std::vector<int64_t> table_off;   // per state: byte offset of its plan's tables (-1: plan-compiled)
+    void *tables = nullptr;       // device: the groups' tables and offsets
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     void drop_graph() {
@@ -272,17 +283,16 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
 }
 
 // One pass of a plan-compiled plan: one tile per workgroup, LDS slots padded
-// by 1/16 + 1/256. On the context stream unless `stream` is given. Assumes
-// the lock.
-int launch_jit_pass_locked(hgm_state *s, const Plan &p, JitModule *jm, size_t pi, hipStream_t stream = nullptr) {
-    Ctx &c = ctx();
+// by 1/16 + 1/256. Assumes the lock.
+int launch_jit_pass_locked(const StateSet &set, const Plan &p, JitModule *jm, size_t pi, hipStream_t stream) {
     const Pass &ps = p.passes[pi];
     const size_t jit_lds = p.jit->lds_bytes;
     const int64_t n_tiles = int64_t(1) << (p.qubits - p.shape.r);
-    void *state = s->d;
-    void *args[] = {&state};
-    HGM_HIP(hipModuleLaunchKernel(jm->fns[p.jit->pass_kernel[pi]], (unsigned)n_tiles, 1, 1, (unsigned)p.shape.B, 1,
-                                  1, ps.phases > 1 ? (unsigned)jit_lds : 0u, stream ? stream : c.stream, args,
+    void *state = set.first;
+    const int64_t *offs = set.offs;
+    void *args[] = {&state, &offs};
+    HGM_HIP(hipModuleLaunchKernel(jm->fns[p.jit->pass_kernel[pi]], (unsigned)n_tiles, (unsigned)set.count, 1,
+                                  (unsigned)p.shape.B, 1, 1, ps.phases > 1 ? (unsigned)jit_lds : 0u, stream, args,
                                   nullptr),
             "pass launch");
     return HGM_OK;
@@ -316,7 +326,7 @@ int run_plan_graph_locked(hgm_state *s, const hgm_plan *hp, hgm_stats *st) {
         hp->drop_graph();
         HGM_HIP(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         for (size_t pi = 0; pi < p.passes.size() && !rc; ++pi)
-            if (p.passes[pi].op_count) rc = launch_jit_pass_locked(s, p, jm, pi);
+            if (p.passes[pi].op_count) rc = launch_jit_pass_locked({s->d}, p, jm, pi, c.stream);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(c.stream, &g);
         if (rc || e != hipSuccess) {
@@ -363,9 +373,9 @@ size_t register_program_bytes(const Plan &p) {
 }
 
 // Launches every non-empty pass of the plan on `stream`, with no events or
-// waits (jm: the plan's loaded module, for plan-compiled plans; table: the
+// waits, for a state or a set of them (LDS plans: one state; jm: the plan's loaded module, for plan-compiled plans; table: the
 // plan's table on the device, for the others). Assumes the lock.
-int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const void *table, hipStream_t stream) {
+int launch_passes_locked(const StateSet &set, const Plan &p, JitModule *jm, const void *table, hipStream_t stream) {
     const bool reg = p.kernel == HGM_KERNEL_REG;
     const bool jit = p.kernel == HGM_KERNEL_JIT;
     PassArgs a;
@@ -377,7 +387,7 @@ int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const void 
         const size_t tile_bytes = (size_t(1) << p.exec.r) * amp_bytes(p.dtype);
         for (const XLaunch &x : p.xlaunch) {
             const XPass *xp = reinterpret_cast<const XPass *>(static_cast<const char *>(table) + x.off);
-            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, s->d, xp, (uint32_t)x.bytes, x.stages > 1 ? tile_bytes : 0,
+            HGM_HIP(launch_pass_reg(p.dtype, p.qubits, p.exec, set, xp, (uint32_t)x.bytes, x.stages > 1 ? tile_bytes : 0,
                                     stream),
                     "pass launch");
         }
@@ -388,10 +398,10 @@ int launch_passes_locked(hgm_state *s, const Plan &p, JitModule *jm, const void 
         if (ps.op_count == 0) continue;
         a.nonlocal_mask = all & ~ps.local_mask;
         if (jit) {
-            if (int rc = launch_jit_pass_locked(s, p, jm, pi, stream)) return rc;
+            if (int rc = launch_jit_pass_locked(set, p, jm, pi, stream)) return rc;
         } else {
             std::memcpy(a.local_pos, ps.local_pos, sizeof(a.local_pos));
-            HGM_HIP(launch_pass_lds(p.dtype, s->d, static_cast<const DevOp *>(table) + ps.op_begin, (int)ps.op_count, a,
+            HGM_HIP(launch_pass_lds(p.dtype, set.first, static_cast<const DevOp *>(table) + ps.op_begin, (int)ps.op_count, a,
                                     stream),
                     "pass launch");
         }
@@ -440,7 +450,7 @@ int run_plan_locked(hgm_state *s, const Plan &p, hgm_stats *st, double plan_ms, 
         }
     }
     HGM_HIP(hipEventRecord(c.e0, c.stream), "hipEventRecord");
-    if ((rc = launch_passes_locked(s, p, jm, table, c.stream))) return rc;
+    if ((rc = launch_passes_locked({s->d}, p, jm, table, c.stream))) return rc;
     HGM_HIP(hipEventRecord(c.e1, c.stream), "hipEventRecord");
     HGM_HIP(hipEventSynchronize(c.e1), "pass execution");
     add_stats(st, p, elapsed(c.e0, c.e1), plan_ms);
@@ -480,12 +490,27 @@ int batch_modules_locked(hgm_batch *b, std::vector<JitModule *> *jms, bool *stal
     return HGM_OK;
 }
 
-// The batch's device copy of state i's register or LDS plan's table.
-const void *batch_table(const hgm_batch *b, size_t i) {
-    return b->table_off[i] < 0 ? nullptr : static_cast<const char *>(b->tables) + b->table_off[i];
+// Whether two plans launch the same kernels with the same programs.
+bool same_launches(const Plan &a, const Plan &b) {
+    if (a.qubits != b.qubits || a.dtype != b.dtype || a.kernel != b.kernel || a.passes.size() != b.passes.size()) return false;
+    if (a.kernel == HGM_KERNEL_JIT)
+        return a.shape.r == b.shape.r && a.shape.B == b.shape.B && a.jit->hash == b.jit->hash &&
+               a.jit->source == b.jit->source && a.jit->pass_kernel == b.jit->pass_kernel;
+    if (a.kernel != HGM_KERNEL_REG || a.exec.r != b.exec.r || a.exec.A != b.exec.A || a.exec.sync != b.exec.sync ||
+        a.xlaunch.size() != b.xlaunch.size() || a.xprog != b.xprog)
+        return false;
+    for (size_t i = 0; i < a.xlaunch.size(); ++i)
+        if (a.xlaunch[i].off != b.xlaunch[i].off || a.xlaunch[i].stages != b.xlaunch[i].stages) return false;
+    return true;
 }
 
-// Captures the batch: a fork on the context stream, each state's passes in
+// States per launch of a plan: a dispatch holds at most 2^32 - 1 work-items.
+int max_group(const Plan &p) {
+    const uint64_t items = (uint64_t(1) << p.qubits) / (uint64_t)(p.kernel == HGM_KERNEL_REG ? p.exec.A : 2 * p.shape.R);
+    return (int)std::min<uint64_t>(65535, 0xffffffffull / std::max<uint64_t>(items, 1));
+}
+
+// Captures the batch: a fork on the context stream, each group's passes in
 // order on its branch stream, a join back. Assumes the lock.
 int capture_batch_locked(hgm_batch *b, const std::vector<JitModule *> &jms) {
     Ctx &c = ctx();
@@ -494,8 +519,25 @@ int capture_batch_locked(hgm_batch *b, const std::vector<JitModule *> &jms) {
     int rc = HGM_OK;
     hipError_t e = hipEventRecord(b->fork, c.stream);
     for (int k = 0; k < b->n_branches && e == hipSuccess; ++k) e = hipStreamWaitEvent(b->streams[k], b->fork, 0);
-    for (size_t i = 0; i < b->plans.size() && e == hipSuccess && !rc; ++i)
-        rc = launch_passes_locked(b->states[i], b->plans[i]->plan, jms[i], batch_table(b, i), b->streams[b->branch[i]]);
+    for (const BatchGroup &g : b->groups) {
+        if (e != hipSuccess || rc) break;
+        const size_t i = (size_t)g.members[0];
+        const Plan &p = b->plans[i]->plan;
+        const char *base = static_cast<const char *>(b->tables);
+        const void *table = g.table_off < 0 ? nullptr : base + g.table_off;
+        const hipStream_t st = b->streams[g.branch];
+        if (p.kernel == HGM_KERNEL_LDS) {
+            for (int k : g.members)
+                if (!rc) rc = launch_passes_locked({b->states[k]->d}, p, jms[i], table, st);
+            continue;
+        }
+        StateSet set{b->states[i]->d};
+        if (g.members.size() > 1) {
+            set.offs = reinterpret_cast<const int64_t *>(base + g.offs_off);
+            set.count = (int)g.members.size();
+        }
+        rc = launch_passes_locked(set, p, jms[i], table, st);
+    }
     for (int k = 0; k < b->n_branches && e == hipSuccess && !rc; ++k) {
         e = hipEventRecord(b->join[k], b->streams[k]);
         if (e == hipSuccess) e = hipStreamWaitEvent(c.stream, b->join[k], 0);
@@ -1249,22 +1291,41 @@ int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int
     auto b = std::make_unique<hgm_batch>();
     b->states.assign(states, states + n);
     b->plans.assign(plans, plans + n);
-    // states by bytes moved, largest first, each to the branch with the fewest so far
-    b->n_branches = std::min(n, kBatchBranches);
-    std::vector<int> order(n);
-    std::vector<double> bytes(n), load(b->n_branches, 0.0);
+    // states that share launches
     for (int i = 0; i < n; ++i) {
         const Plan &p = plans[i]->plan;
+        BatchGroup *to = nullptr;
+        for (BatchGroup &g : b->groups) {
+            const Plan &q = plans[g.members[0]]->plan;
+            if ((int)g.members.size() < max_group(q) &&
+                (plans[i] == plans[g.members[0]] || (p.kernel != HGM_KERNEL_LDS && same_launches(p, q)))) {
+                to = &g;
+                break;
+            }
+        }
+        if (!to) {
+            b->groups.emplace_back();
+            to = &b->groups.back();
+        }
+        to->members.push_back(i);
+    }
+    // groups by bytes moved, largest first, each to the branch with the fewest so far
+    const int n_groups = (int)b->groups.size();
+    b->n_branches = std::min(n_groups, kBatchBranches);
+    std::vector<int> order(n_groups);
+    std::vector<double> bytes(n_groups), load(b->n_branches, 0.0);
+    for (int i = 0; i < n_groups; ++i) {
+        const BatchGroup &g = b->groups[i];
+        const Plan &p = plans[g.members[0]]->plan;
         int64_t busy = 0;
         for (const Pass &ps : p.passes) busy += ps.op_count > 0;
-        bytes[i] = (double)busy * (double)(uint64_t(1) << p.qubits) * (double)amp_bytes(p.dtype);
+        bytes[i] = (double)busy * (double)(uint64_t(1) << p.qubits) * (double)amp_bytes(p.dtype) * (double)g.members.size();
         order[i] = i;
     }
     std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return bytes[a] > bytes[c]; });
-    b->branch.assign(n, 0);
     for (int i : order) {
         const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        b->branch[i] = k;
+        b->groups[i].branch = k;
         load[k] += bytes[i];
     }
     std::lock_guard<std::mutex> g(ctx().mu);
@@ -1284,27 +1345,29 @@ int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int
         e = hipStreamCreateWithFlags(&b->streams[k], hipStreamNonBlocking);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&b->join[k], hipEventDisableTiming);
     }
-    // one device copy of the tables of each distinct register or LDS plan
-    b->table_off.assign(n, -1);
-    size_t total = 0;
-    for (int i = 0; i < n; ++i) {
-        const Plan &p = plans[i]->plan;
-        if (p.kernel == HGM_KERNEL_JIT) continue;
-        int j = 0;
-        while (j < i && plans[j] != plans[i]) ++j;
-        if (j < i) { b->table_off[i] = b->table_off[j]; continue; }
-        b->table_off[i] = (int64_t)total;
-        total += align256(plan_table_bytes(p));
-        if (e == hipSuccess) e = prepare_pass_kernels(p.dtype);
+    // device copies of the groups' tables and offsets
+    std::vector<char> host;
+    auto place = [&](const void *p, size_t bytes) {
+        const size_t at = host.size();
+        host.resize(align256(at + std::max<size_t>(bytes, 1)));
+        if (bytes) std::memcpy(&host[at], p, bytes);
+        return (int64_t)at;
+    };
+    for (BatchGroup &g : b->groups) {
+        const Plan &p = plans[g.members[0]]->plan;
+        if (p.kernel != HGM_KERNEL_JIT) {
+            g.table_off = place(plan_table(p), plan_table_bytes(p));
+            if (e == hipSuccess) e = prepare_pass_kernels(p.dtype);
+        }
+        if (g.members.size() > 1 && p.kernel != HGM_KERNEL_LDS) {
+            std::vector<int64_t> offs;
+            for (int k : g.members)
+                offs.push_back((int64_t)(static_cast<char *>(states[k]->d) - static_cast<char *>(states[g.members[0]]->d)));
+            g.offs_off = place(offs.data(), offs.size() * sizeof(int64_t));
+        }
     }
-    if (e == hipSuccess && total) e = hipMalloc(&b->tables, total);
-    for (int i = 0; i < n && e == hipSuccess; ++i) {
-        const Plan &p = plans[i]->plan;
-        if (b->table_off[i] < 0 || (i > 0 && std::find(plans, plans + i, plans[i]) != plans + i)) continue;
-        if (const size_t bytes = plan_table_bytes(p))
-            e = hipMemcpy(const_cast<void *>(batch_table(b.get(), (size_t)i)), plan_table(p), bytes,
-                          hipMemcpyHostToDevice);
-    }
+    if (e == hipSuccess && !host.empty()) e = hipMalloc(&b->tables, host.size());
+    if (e == hipSuccess && !host.empty()) e = hipMemcpy(b->tables, host.data(), host.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         rc = hip_fail(e, "batch streams and tables");
         release();
