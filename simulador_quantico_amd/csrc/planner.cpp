@@ -6,6 +6,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstring>
+#include <mutex>
 
 #include "jit.hpp"
 #include "program.hpp"
@@ -657,7 +658,7 @@ void rotate_rows(int qubits, const hgm_op *ops, int64_t n_ops, std::vector<hgm_o
 }
 
 int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iterations, const hgm_tuning &t,
-               Plan *out, std::string *err, bool program_only, bool pass_by_pass) {
+               Plan *out, std::string *err, bool program_only, bool for_serving) {
     auto t0 = std::chrono::steady_clock::now();
     static std::atomic<uint64_t> builds{0};
     Plan plan;
@@ -892,8 +893,8 @@ int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iter
     }
     if (t.kernel == HGM_KERNEL_REG || t.kernel == HGM_KERNEL_JIT || (t.kernel == HGM_KERNEL_AUTO && reg_ok)) {
         plan.kernel = t.kernel == HGM_KERNEL_JIT ? HGM_KERNEL_JIT : HGM_KERNEL_REG;
-        build_register_program(plan);
-        if (plan.kernel == HGM_KERNEL_REG) build_exec_program(plan, pass_by_pass);
+        if (plan.kernel == HGM_KERNEL_JIT) build_register_program(plan);
+        else if (!for_serving) build_exec_program(plan, false);
         if (plan.kernel == HGM_KERNEL_JIT) {
             // one workgroup per tile: a dispatch holds at most 2^32 - 1 work-items
             const uint64_t items = (uint64_t(1) << (qubits - plan.shape.r)) * (uint64_t)plan.shape.B;
@@ -1062,7 +1063,14 @@ void schedule_waves(std::vector<RegOp> &ops) {
 // bits on the thread index so that HBM loads and stores stay contiguous
 // across lanes (an empty phase is added when a gate needs them earlier or the
 // schedule ends with them in registers).
+void need_register_program(const Plan &plan) {
+    static std::mutex mu;
+    std::lock_guard<std::mutex> g(mu);
+    if (!plan.has_program) build_register_program(const_cast<Plan &>(plan));
+}
+
 void build_register_program(Plan &plan) {
+    plan.has_program = true;
     const int r = plan.shape.r, c = plan.shape.c;
     const int A = 2 * plan.shape.R;
     int a = 0;

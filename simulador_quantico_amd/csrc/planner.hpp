@@ -170,19 +170,26 @@ struct Plan {
     std::vector<uint8_t> pre_phase;   // per DevOp: a kPrePhaseTag gate (kept with the next rotation)
     int64_t gates = 0;
     double plan_ms = 0;
-    // register kernel program (kernel == HGM_KERNEL_REG)
+    // register program (build_register_program)
     std::vector<RegOp> rops;
     std::vector<PhaseMap> maps;
     std::vector<PassMem> mems;
     int max_phases = 0;
+    bool has_program = false;         // rops, maps and mems are built
     ExecShape exec{};
     std::vector<uint64_t> xprog;      // the interpreted kernels' programs (XPass and XOp records)
     std::vector<XLaunch> xlaunch;     // in order: one per non-empty pass, or fewer where one workgroup holds the state
     std::shared_ptr<JitCode> jit;     // HGM_KERNEL_JIT: generated and compiled pass kernels
 };
 
-// Builds the register program of every pass (fills rops/maps/mems).
+// Builds the register program of every pass (fills rops/maps/mems): what the
+// plan-compiled and serving kernels are generated from, and what
+// hgm_plan_program shows. build_plan builds it for plan-compiled plans; the
+// interpreted kernels run their own programs (build_exec_program).
 void build_register_program(Plan &plan);
+
+// The register program of a plan that may already be in use by others.
+void need_register_program(const Plan &plan);
 
 // Reorders the ops between two remaps into waves: every phase whose
 // predecessors (the earlier ops it does not commute with) are done, then
@@ -262,9 +269,9 @@ void fuse_gates(int qubits, const hgm_op *ops, int64_t n_ops, std::vector<hgm_op
 // tuning gets its tile shape checked and its register program built, but no
 // kernels generated or compiled: the plan (kernel HGM_KERNEL_REG) is for
 // kernels compiled from its passes' structure elsewhere (the serving engine).
-// With pass_by_pass every non-empty pass is a launch of its own (the serving
-// engine advances its states by passes).
+// With for_serving a register-kernel plan gets neither its register program
+// nor its launches: the serving engine builds what its passes run on.
 int build_plan(int qubits, int dtype, const hgm_op *ops, int64_t n_ops, int iterations, const hgm_tuning &t,
-               Plan *out, std::string *err, bool program_only = false, bool pass_by_pass = false);
+               Plan *out, std::string *err, bool program_only = false, bool for_serving = false);
 
 }  // namespace hgm

@@ -73,18 +73,20 @@ bool real_middle(const C v[2][2], C x[2], C *y, R o[2][2]) {
         for (int i = 0; i < 2; ++i)
             for (int j = 0; j < 2; ++j) {
                 if (v[i][j] == C(0, 0)) continue;
-                const C u = v[i][j] / std::abs(v[i][j]);
+                const C u = v[i][j] / std::sqrt(std::norm(v[i][j]));
                 if (have_c[j] && !have_r[i]) { row[i] = u * std::conj(col[j]); have_r[i] = true; }
                 else if (have_r[i] && !have_c[j]) { col[j] = u * std::conj(row[i]); have_c[j] = true; }
             }
     const C closing = v[1][1] * std::conj(row[1] * col[1]);
-    if (std::abs(closing.imag()) > 16 * 0x1p-52L * std::abs(closing)) return false;
+    if (std::abs(closing.imag()) > 16 * 0x1p-52L * std::sqrt(std::norm(closing))) return false;
     if (v[0][0] != C(0, 0) && v[0][1] != C(0, 0) && v[1][0] != C(0, 0) && v[1][1] != C(0, 0)) {
         // what the fourth phase misses by is the entries' own rounding: a quarter to each
-        const R miss = closing.imag() / closing.real();
-        row[0] *= std::polar(R(1), -miss / 4);
-        row[1] *= std::polar(R(1), miss / 4);
-        col[1] *= std::polar(R(1), miss / 2);
+        const R miss = closing.imag() / closing.real();   // below 2^-47: e^(i miss) = 1 + i miss
+        if (miss != 0) {
+            row[0] *= C(1, -miss / 4);
+            row[1] *= C(1, miss / 4);
+            col[1] *= C(1, miss / 2);
+        }
     }
     for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j) o[i][j] = (v[i][j] * std::conj(row[i] * col[j])).real();
@@ -94,12 +96,66 @@ bool real_middle(const C v[2][2], C x[2], C *y, R o[2][2]) {
     return true;
 }
 
+// U = e0 * diag(1, e1) * M * diag(1, y) with M = [[1, t0], [t1, 1]] and, where
+// the off-diagonal entries are the larger, the rows of U exchanged.
+struct Rotation {
+    bool ok = false, exchanged = false;
+    R t0 = 0, t1 = 0;
+    C e0, e1, y;
+};
+
+Rotation split_rotation(const double m[8]) {
+    Rotation t;
+    const C v[2][2] = {{C(m[0], m[1]), C(m[2], m[3])}, {C(m[4], m[5]), C(m[6], m[7])}};
+    C x[2];
+    R w[2][2];
+    if (!real_middle(v, x, &t.y, w)) return t;
+    const int ex = std::abs(w[0][0]) < std::abs(w[0][1]) ? 1 : 0;
+    const R d0 = w[ex][0], d1 = w[1 - ex][1];   // of the new rows 0 and 1
+    if (d0 == 0 || d1 == 0) return t;
+    t.t0 = w[ex][1] / d0;
+    t.t1 = w[1 - ex][0] / d1;
+    if (!(std::abs(t.t0) <= kMaxTurn && std::abs(t.t1) <= kMaxTurn)) return t;
+    t.exchanged = ex != 0;
+    t.e0 = x[ex] * d0;
+    t.e1 = x[1 - ex] * d1 / t.e0;
+    t.ok = true;
+    return t;
+}
+
+// The rotations of the gates seen last: circuits repeat their gates, and a
+// split takes longer than the rest of a gate's record.
+struct RotationMemo {
+    static constexpr int kEntries = 16;
+    struct Entry {
+        double m[8];
+        Rotation t;
+        bool used = false;
+    } entry[kEntries];
+
+    const Rotation &of(const double m[8]) {
+        uint64_t h = 0;
+        for (int i = 0; i < 8; ++i) {
+            uint64_t b;
+            std::memcpy(&b, &m[i], 8);
+            h = (h ^ b) * 0x9e3779b97f4a7c15ull;
+        }
+        Entry &e = entry[h >> 60];
+        if (!e.used || std::memcmp(e.m, m, sizeof e.m)) {
+            std::memcpy(e.m, m, sizeof e.m);
+            e.t = split_rotation(m);
+            e.used = true;
+        }
+        return e.t;
+    }
+};
+
 // Emits one item as register operations. `flip` holds the tile bits whose two
 // values are exchanged in the registers (physical = logical ^ flip): an
 // uncontrolled X, anti-diagonal gate or row-exchanged gate toggles its bit
 // instead of moving amplitudes. `scale` is a factor of the whole state that is
 // still to be applied.
-void emit(const Item &it, uint32_t S, uint32_t &flip, C &scale, std::vector<ROp> &out) {
+void emit(const Item &it, uint32_t S, uint32_t &flip, C &scale, RotationMemo &memo, std::vector<ROp> &out) {
     const DevOp &d = *it.d;
     const uint32_t lval = it.lval ^ (flip & it.lmask);
     auto phase = [&](C f, uint32_t lm, uint32_t lv, uint64_t gm, uint64_t gv) {
@@ -126,7 +182,7 @@ void emit(const Item &it, uint32_t S, uint32_t &flip, C &scale, std::vector<ROp>
             phase(C(d.m[6 * v], d.m[6 * v + 1]), it.lmask | tb, lval | ((v ^ f) << it.tbit), it.gmask, it.gval);
         return;
     }
-    R m[8];   // row-major on the physical pair
+    double m[8];   // row-major on the physical pair
     for (int row = 0; row < 2; ++row)
         for (int col = 0; col < 2; ++col)
             for (int c = 0; c < 2; ++c) m[4 * row + 2 * col + c] = d.m[4 * (row ^ (int)f) + 2 * (col ^ (int)f) + c];
@@ -141,28 +197,17 @@ void emit(const Item &it, uint32_t S, uint32_t &flip, C &scale, std::vector<ROp>
     o.phase = false;
     o.bit = popc(S & (tb - 1));
     if (free_gate) {
-        const C v[2][2] = {{C(m[0], m[1]), C(m[2], m[3])}, {C(m[4], m[5]), C(m[6], m[7])}};
-        C x[2], y;
-        R w[2][2];
-        if (real_middle(v, x, &y, w)) {
-            // the larger entry of each row becomes 1; with the off-diagonal ones the larger, rows are exchanged
-            const int ex = std::abs(w[0][0]) < std::abs(w[0][1]) ? 1 : 0;
-            const R d0 = w[ex][0], d1 = w[1 - ex][1];   // of the new rows 0 and 1
-            if (d0 != 0 && d1 != 0) {
-                const R t0 = w[ex][1] / d0, t1 = w[1 - ex][0] / d1;
-                if (std::abs(t0) <= kMaxTurn && std::abs(t1) <= kMaxTurn) {
-                    phase(y, tb, tb, 0, 0);
-                    if (ex) flip ^= tb;
-                    o.kind = X_ROT;
-                    o.m[0] = t0;
-                    o.m[1] = t1;
-                    out.push_back(o);
-                    const C e0 = x[ex] * d0, e1 = x[1 - ex] * d1;
-                    scale *= e0;
-                    phase(e1 / e0, tb, tb, 0, 0);
-                    return;
-                }
-            }
+        const Rotation &t = memo.of(m);
+        if (t.ok) {
+            phase(t.y, tb, tb, 0, 0);
+            if (t.exchanged) flip ^= tb;
+            o.kind = X_ROT;
+            o.m[0] = t.t0;
+            o.m[1] = t.t1;
+            out.push_back(o);
+            scale *= t.e0;
+            phase(t.e1, tb, tb, 0, 0);
+            return;
         }
     }
     split_cond(it.lmask, lval, S, o);
@@ -178,11 +223,19 @@ void emit(const Item &it, uint32_t S, uint32_t &flip, C &scale, std::vector<ROp>
     out.push_back(o);
 }
 
+// Stable insertion sort: the lists are short (kChunk) and nearly in order.
+template <class I, class F>
+void sort_stable(I b, I e, F less) {
+    for (I i = b; i != e; ++i)
+        for (I j = i; j != b && less(*j, *(j - 1)); --j) std::swap(*j, *(j - 1));
+}
+
 // Orders a stage's operations into waves (phases as early as they commute,
 // then gates), keeping the order of every pair that does not commute: gates
 // on a register bit conflict with gates on it and with whatever tests it.
-void into_waves(std::vector<ROp> &ops) {
+void into_waves(std::vector<ROp> &ops, std::vector<const ROp *> &order) {
     int gate[8] = {0}, test[8] = {0};
+    order.clear();
     for (ROp &o : ops) {
         int s = 0;
         for (uint32_t m = o.rmask; m; m &= m - 1) s = std::max(s, gate[__builtin_ctz(m)]);
@@ -191,8 +244,9 @@ void into_waves(std::vector<ROp> &ops) {
         o.slot = s;
         for (uint32_t m = o.rmask; m; m &= m - 1) test[__builtin_ctz(m)] = std::max(test[__builtin_ctz(m)], s);
         if (!o.phase) gate[o.bit] = std::max(gate[o.bit], s);
+        order.push_back(&o);
     }
-    std::stable_sort(ops.begin(), ops.end(), [](const ROp &a, const ROp &b) { return a.slot < b.slot; });
+    sort_stable(order.begin(), order.end(), [](const ROp *a, const ROp *b) { return a->slot < b->slot; });
 }
 
 template <class T>
@@ -224,13 +278,17 @@ struct Records {
     std::vector<T> table;
     C scale = C(1, 0);   // factor of the whole state still to be applied
 
-    // A factor per register, the pending scale included.
-    void vec(std::vector<C> &f) {
+    std::vector<const ROp *> order;   // scratch
+    std::vector<ROp> group;
+    C f[kMaxRegAmps];
+
+    // A factor per register (f), the pending scale included.
+    void vec() {
         bool real = true, one = true;
-        for (C &z : f) {
-            z *= scale;
-            real = real && (T)z.imag() == T(0);
-            one = one && z == C(1, 0);
+        for (uint32_t k = 0; k < A; ++k) {
+            if (scale != C(1, 0)) f[k] *= scale;
+            real = real && (T)f[k].imag() == T(0);
+            one = one && f[k] == C(1, 0);
         }
         scale = C(1, 0);
         if (one) return;
@@ -238,50 +296,58 @@ struct Records {
         std::memset(&x, 0, sizeof x);
         x.kind = real ? X_VEC_REAL : X_VEC;
         x.pmask = (uint32_t)table.size();
-        for (const C &z : f) {
-            table.push_back((T)z.real());
-            if (!real) table.push_back((T)z.imag());
+        for (uint32_t k = 0; k < A; ++k) {
+            table.push_back((T)f[k].real());
+            if (!real) table.push_back((T)f[k].imag());
         }
         ops.push_back(x);
     }
 
+    using It = std::vector<const ROp *>::const_iterator;
+
     // The phases [b, e) of a wave that test register bits only: one record when
     // a pattern of set (or one clear) register bits says it, else one factor
     // per register.
-    void uniform(const ROp *b, const ROp *e) {
+    void uniform(It b, It e) {
         if (b == e) return;
         if (e - b == 1 && scale == C(1, 0)) {
-            XOp<T> x = record<T>(*b, A);
+            XOp<T> x = record<T>(**b, A);
             if (x.pat != X_PAT_MASK) {
-                x.flags = (uint8_t)(X_FIRST | X_LAST | (b->m[1] == 0.0 ? X_REAL : 0));
+                x.flags = (uint8_t)(X_FIRST | X_LAST | ((*b)->m[1] == 0 ? X_REAL : 0));
                 ops.push_back(x);
                 return;
             }
         }
-        std::vector<C> f(A, C(1, 0));
-        for (const ROp *o = b; o != e; ++o)
-            for (uint32_t k = 0; k < A; ++k)
-                if ((k & o->rmask) == o->rval) f[k] *= C(o->m[0], o->m[1]);
-        vec(f);
+        std::fill(f, f + A, C(1, 0));
+        for (; b != e; ++b) {
+            const ROp &o = **b;
+            for (uint32_t k = 0; k < A; ++k) {
+                if ((k & o.rmask) != o.rval) continue;
+                if (o.m[1] == 0) f[k] *= o.m[0];
+                else f[k] *= C(o.m[0], o.m[1]);
+            }
+        }
+        vec();
     }
 
     // Phases with conditions on threads or tiles, grouped by the registers they
     // act on (the caller sorted them), equal conditions multiplied together.
-    void groups(const ROp *b, const ROp *e) {
+    void groups(It b, It e) {
         while (b != e) {
-            std::vector<ROp> group;
-            const ROp head = *b;
-            for (; b != e && b->rmask == head.rmask && b->rval == head.rval; ++b) {
+            group.clear();
+            const ROp &head = **b;
+            for (; b != e && (*b)->rmask == head.rmask && (*b)->rval == head.rval; ++b) {
+                const ROp &o = **b;
                 auto same = std::find_if(group.begin(), group.end(), [&](const ROp &g) {
-                    return g.tmask == b->tmask && g.tval == b->tval && g.gmask == b->gmask && g.gval == b->gval;
+                    return g.tmask == o.tmask && g.tval == o.tval && g.gmask == o.gmask && g.gval == o.gval;
                 });
-                if (same == group.end()) { group.push_back(*b); continue; }
-                const C f = C(same->m[0], same->m[1]) * C(b->m[0], b->m[1]);
-                same->m[0] = f.real();
-                same->m[1] = f.imag();
+                if (same == group.end()) { group.push_back(o); continue; }
+                const C z = C(same->m[0], same->m[1]) * C(o.m[0], o.m[1]);
+                same->m[0] = z.real();
+                same->m[1] = z.imag();
             }
             bool real = true;
-            for (const ROp &g : group) real = real && g.m[1] == 0.0;
+            for (const ROp &g : group) real = real && g.m[1] == 0;
             for (size_t k = 0; k < group.size(); ++k) {
                 XOp<T> x = record<T>(group[k], A);
                 x.flags = (uint8_t)((k == 0 ? X_FIRST : 0) | (k + 1 == group.size() ? X_LAST : 0) | (real ? X_REAL : 0));
@@ -293,49 +359,49 @@ struct Records {
     // A run of rotations: those on different register bits commute, and three
     // of a full set of four (two of two or three) already cost less as one
     // record than one by one.
-    void rotations(const ROp *b, const ROp *e) {
+    void rotations(It b, It e) {
         const int bits = A == 2 ? 1 : A == 4 ? 2 : A == 8 ? 3 : 4;
         while (b != e) {
             uint32_t used = 0;
-            const ROp *n = b;
-            for (; n != e && n->bit < bits && !((used >> n->bit) & 1u); ++n) used |= 1u << n->bit;
+            It n = b;
+            for (; n != e && (*n)->bit < bits && !((used >> (*n)->bit) & 1u); ++n) used |= 1u << (*n)->bit;
             if (n == b) ++n;   // a fifth register bit
             if (popc(used) >= (bits + 2) / 2 && bits > 1) {
                 XOp<T> x;
                 std::memset(&x, 0, sizeof x);
                 x.kind = X_ROTS;
                 for (; b != n; ++b) {
-                    x.m[2 * b->bit] = (T)b->m[0];
-                    x.m[2 * b->bit + 1] = (T)b->m[1];
+                    x.m[2 * (*b)->bit] = (T)(*b)->m[0];
+                    x.m[2 * (*b)->bit + 1] = (T)(*b)->m[1];
                 }
                 ops.push_back(x);
             } else {
-                for (; b != n; ++b) ops.push_back(record<T>(*b, A));
+                for (; b != n; ++b) ops.push_back(record<T>(**b, A));
             }
         }
     }
 
     void stage(std::vector<ROp> &list) {
-        into_waves(list);
-        for (size_t i = 0; i < list.size();) {
-            size_t e = i;
-            if (!list[i].phase) {
-                if (list[i].kind != X_ROT) { ops.push_back(record<T>(list[i++], A)); continue; }
-                while (e < list.size() && !list[e].phase && list[e].kind == X_ROT) ++e;
-                rotations(list.data() + i, list.data() + e);
+        into_waves(list, order);
+        for (auto i = order.begin(); i != order.end();) {
+            auto e = i;
+            if (!(*i)->phase) {
+                if ((*i)->kind != X_ROT) { ops.push_back(record<T>(**i++, A)); continue; }
+                while (e != order.end() && !(*e)->phase && (*e)->kind == X_ROT) ++e;
+                rotations(i, e);
                 i = e;
                 continue;
             }
-            while (e < list.size() && list[e].phase && list[e].slot == list[i].slot) ++e;
-            auto uniform_op = [](const ROp &o) { return !o.tmask && !o.gmask; };
-            std::stable_sort(list.begin() + i, list.begin() + e, [&](const ROp &a, const ROp &b) {
+            while (e != order.end() && (*e)->phase && (*e)->slot == (*i)->slot) ++e;
+            auto uniform_op = [](const ROp *o) { return !o->tmask && !o->gmask; };
+            sort_stable(i, e, [&](const ROp *a, const ROp *b) {
                 if (uniform_op(a) != uniform_op(b)) return uniform_op(a);
-                return a.rmask != b.rmask ? a.rmask < b.rmask : a.rval < b.rval;
+                return a->rmask != b->rmask ? a->rmask < b->rmask : a->rval < b->rval;
             });
-            size_t u = i;
-            while (u < e && uniform_op(list[u])) ++u;
-            uniform(list.data() + i, list.data() + u);
-            groups(list.data() + u, list.data() + e);
+            auto u = i;
+            while (u != e && uniform_op(*u)) ++u;
+            uniform(i, u);
+            groups(u, e);
             i = e;
         }
     }
@@ -345,10 +411,13 @@ struct Records {
     void flush(bool end) {
         const R s = std::abs(scale);
         if (scale == C(1, 0) || (!end && s >= 0x1p-20L && s <= 0x1p20L)) return;
-        std::vector<C> f(A, C(1, 0));
-        vec(f);
+        std::fill(f, f + A, C(1, 0));
+        vec();
     }
 };
+
+// Operations of a stage put into waves together.
+constexpr size_t kChunk = 64;
 
 // Gates of one launch of a whole-state workgroup, at most (about 10 ms).
 constexpr size_t kMaxLaunchItems = size_t(1) << 15;
@@ -407,7 +476,7 @@ void pass_items(const Plan &plan, const Pass &ps, const int *pos, int r, std::ve
 // bit j is state bit pos[j]; gates mix the first r tile bits only, and the
 // first c stay on consecutive threads at the load and the store.
 template <class T>
-void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c) {
+void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c, RotationMemo &memo) {
     constexpr int F = sizeof(T) == 4 ? 5 : 4;
     const ExecShape &ex = plan.exec;
     const int n = plan.qubits;
@@ -475,8 +544,8 @@ void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, in
         }
         ops.clear();
         for (int k : lists[i]) {
-            emit(items[k], sets[i], flip, recs.scale, ops);
-            if (ops.size() >= 64) { recs.stage(ops); recs.flush(false); ops.clear(); }
+            emit(items[k], sets[i], flip, recs.scale, memo, ops);
+            if (ops.size() >= kChunk) { recs.stage(ops); recs.flush(false); ops.clear(); }
         }
         recs.stage(ops);
         recs.flush(i + 1 == sets.size());
@@ -563,10 +632,11 @@ void build_exec_program(Plan &plan, bool pass_by_pass) {
     plan.xlaunch.clear();
     const int n = plan.qubits, r = whole ? n : plan.shape.r, rx = plan.exec.r;
     std::vector<Item> items;
+    RotationMemo memo;
     int pos[32];
     auto launch = [&] {
-        if (plan.dtype == HGM_C64) build<float>(plan, items, pos, r, rx, std::min(plan.shape.c, r));
-        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r));
+        if (plan.dtype == HGM_C64) build<float>(plan, items, pos, r, rx, std::min(plan.shape.c, r), memo);
+        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r), memo);
         items.clear();
     };
     for (const Pass &ps : plan.passes) {

@@ -366,6 +366,7 @@ size_t plan_table_bytes(const Plan &p) {
 // Bytes of a register plan's inspectable program (hgm_plan_program,
 // hgm_plan_maps): part of the size limit of hgm_state_apply_noalloc.
 size_t register_program_bytes(const Plan &p) {
+    if (p.kernel == HGM_KERNEL_REG) need_register_program(p);
     return p.kernel == HGM_KERNEL_REG ? align256(p.rops.size() * sizeof(RegOp)) +
                                             align256(p.maps.size() * sizeof(PhaseMap)) +
                                             align256(p.mems.size() * sizeof(PassMem))
@@ -1223,6 +1224,7 @@ int hgm_plan_serving_source(const hgm_plan *p, int64_t pass, char *out, size_t c
         t_err = "serving kernels are generated for the non-empty passes of register-program plans";
         return HGM_E_ARG;
     }
+    need_register_program(p->plan);
     size_t lds = 0;
     const std::string src = serving_kernel_source(p->plan, p->plan.passes[pass], "hgm_serve", &lds);
     *len = src.size();
@@ -1235,6 +1237,7 @@ double hgm_plan_compile_seconds(const hgm_plan *p) { return (p && p->plan.jit) ?
 int hgm_plan_program(const hgm_plan *p, int64_t i, void *rops, int64_t *n_rops, int32_t *first_map,
                      int32_t *last_map, int8_t *local_pos) {
     if (!p || i < 0 || i >= (int64_t)p->plan.passes.size() || !n_rops) { t_err = "bad arguments"; return HGM_E_ARG; }
+    if (p->plan.kernel == HGM_KERNEL_REG) need_register_program(p->plan);
     const Pass &ps = p->plan.passes[i];
     *n_rops = p->plan.kernel == HGM_KERNEL_REG ? ps.rop_count : 0;
     if (rops && *n_rops)
@@ -1247,6 +1250,7 @@ int hgm_plan_program(const hgm_plan *p, int64_t i, void *rops, int64_t *n_rops, 
 
 int hgm_plan_maps(const hgm_plan *p, void *maps, int64_t *n_maps) {
     if (!p || !n_maps) { t_err = "bad arguments"; return HGM_E_ARG; }
+    if (p->plan.kernel == HGM_KERNEL_REG) need_register_program(p->plan);
     *n_maps = (int64_t)p->plan.maps.size();
     if (maps && *n_maps) std::memcpy(maps, p->plan.maps.data(), p->plan.maps.size() * sizeof(PhaseMap));
     return HGM_OK;

@@ -33,6 +33,7 @@
 #include "jit.hpp"
 #include "kernels.hpp"
 #include "planner.hpp"
+#include "program.hpp"
 #include "runtime.hpp"
 
 namespace hgm {
@@ -405,14 +406,23 @@ void planner_loop(hgm_server *s) {
         }
         if (rc == HGM_OK) {   // the compiled kernel of each pass, where one exists
             r->kernel.assign(r->passes.size(), -1);
-            std::lock_guard<std::mutex> g(s->kmu);
-            if (!s->kernel_of.empty() && r->qubits > r->plan.shape.r)   // one-tile states stay interpreted
+            bool any = false;
+            {
+                std::lock_guard<std::mutex> g(s->kmu);
+                any = !s->kernel_of.empty();
+            }
+            if (any && r->qubits > r->plan.shape.r) {   // one-tile states stay interpreted
+                build_register_program(r->plan);
+                std::lock_guard<std::mutex> g(s->kmu);
                 for (size_t i = 0; i < r->passes.size(); ++i) {
                     auto it = s->kernel_of.find(serving_pass_key(r->plan, r->plan.passes[r->passes[i]]));
                     if (it != s->kernel_of.end()) r->kernel[i] = it->second;
                 }
+            }
         }
         if (rc == HGM_OK && lt.block_size > 0) try_large_tile(s, r, lt);
+        if (rc == HGM_OK && std::find(r->kernel.begin(), r->kernel.end(), -1) != r->kernel.end())
+            build_exec_program(r->plan, true);   // for the passes left to the interpreter
         if (rc == HGM_OK) {
             const Plan &p = r->plan;
             r->n_tiles = int64_t(1) << (r->qubits - p.shape.r);
@@ -870,6 +880,7 @@ int hgm_server_precompile(hgm_server *s, int qubits, const hgm_op *ops, int64_t 
     int rc = build_plan(qubits, s->cfg.dtype, ops, n_ops, iterations, t, &plan, &err, false, true);
     if (rc) { set_error(err); return rc; }
     if (plan.kernel != HGM_KERNEL_REG) { set_error("serving needs the register kernel for this tile shape"); return HGM_E_TUNING; }
+    build_register_program(plan);
     auto busy = [](const Plan &p) {
         size_t k = 0;
         for (const Pass &ps : p.passes) k += ps.op_count > 0;
