@@ -89,26 +89,97 @@ std::string thread_or(const uint64_t *contrib, int nbits) {
     return s.empty() ? "0ull" : s;
 }
 
-// Sum of ((t >> j) & 1) * contrib_j.
-std::string thread_sum(const uint32_t *contrib, int nbits) {
-    std::string s;
-    for (int j = 0; j < nbits; ++j) {
-        if (!contrib[j]) continue;
-        char b[96];
-        std::snprintf(b, sizeof b, "(((t >> %d) & 1u) * %uu)", j, contrib[j]);
-        s += (s.empty() ? "" : " + ") + std::string(b);
-    }
-    return s.empty() ? "0u" : s;
-}
-
 // The interpreter's phase maps hold XOR-swizzled tile indices; the swizzle is
 // its own inverse.
 uint32_t unswizzle(uint32_t x) { return x ^ ((x >> 4) & 15u) ^ ((x >> 8) & 15u) ^ ((x >> 12) & 15u); }
 
-// LDS slot of tile index x in the generated kernels: one padding slot per 16
-// and per 256 entries. Additive over disjoint bit sets, so a slot is a
+// LDS slot of tile index x in the generated kernels: one padding slot per 2^lo
+// and per 2^hi entries. Additive over disjoint bit sets, so a slot is a
 // per-thread part plus a per-register constant (an immediate offset).
-uint32_t padded(uint32_t x) { return x + (x >> 4) + (x >> 8); }
+struct Pad {
+    int lo, hi;
+    uint32_t operator()(uint32_t x) const { return x + (x >> lo) + (x >> hi); }
+};
+
+// Plan-compiled kernels pad at bits 4 and 8; the FP32 serving kernels at 5 and
+// 9. Measured both ways: 12 Grover requests of 22-23 qubits served 5.96 -> 5.79
+// ms with 5 and 9, 20 random layers at 30 qubits 50.5 -> 51.5 ms in FP32 and
+// 97.1 -> 97.9 in FP64.
+constexpr Pad kPad = {4, 8}, kServingPad32 = {5, 9};
+
+// The LDS exchanges between the phases of one pass. In place, a thread writes
+// to the slots it read last, so nothing has to wait before the writes, and one
+// barrier stands between them and the reads: one per exchange, two where real
+// and imaginary parts go one after the other. Each exchange then permutes where
+// an element lies: slot bit of every thread and register bit, updated here at
+// generation time. With fixed places (an element's slot is its tile index) the
+// writes wait for the reads before, twice as many barriers. FP32 kernels
+// exchange in place: 20 random layers at 30 qubits 51.9 -> 50.8 ms. FP64 kernels
+// keep fixed places: 96.7 against 97.1 ms in place.
+struct Exchange {
+    int tb, a;                       // thread bits, register bits
+    int thr[kMaxThreadBits], reg[8]; // slot bit of thread bit j / register bit i: where the next write goes
+    const bool in_place;
+    const Pad pad;
+    int n = 0;                       // thread parts emitted
+
+    static int bit_of(uint32_t one) { return __builtin_ctz(unswizzle(one)); }
+    static int thr_bit(const PhaseMap &m, int j) { return bit_of(m.thr[j / 5][1 << (j % 5)]); }
+    static int reg_bit(const PhaseMap &m, int i) { return bit_of(m.reg[1 << i]); }
+
+    Exchange(int B, int A, const PhaseMap &first, bool in_place, Pad pad) : tb(0), a(0), in_place(in_place), pad(pad) {
+        while ((1 << tb) < B) ++tb;
+        while ((1 << a) < A) ++a;
+        place(first);
+    }
+
+    void place(const PhaseMap &m) {   // slots of fixed places
+        for (int j = 0; j < tb; ++j) thr[j] = thr_bit(m, j);
+        for (int i = 0; i < a; ++i) reg[i] = reg_bit(m, i);
+    }
+
+    // Declares the thread part of the current slots.
+    std::string declare() {
+        uint64_t c[kMaxThreadBits] = {0};
+        for (int j = 0; j < tb; ++j) c[j] = uint64_t(1) << thr[j];
+        const std::string x = "x" + std::to_string(n), f = "f" + std::to_string(n);
+        ++n;
+        return "        const unsigned " + x + " = (unsigned)(" + thread_or(c, tb) + ");\n        const unsigned " + f + " = " +
+               x + " + (" + x + " >> " + std::to_string(pad.lo) + ") + (" + x + " >> " + std::to_string(pad.hi) + ");\n";
+    }
+
+    std::string slot(int k) const {   // of register k, by the part declared last
+        uint32_t x = 0;
+        for (int i = 0; i < a; ++i)
+            if ((k >> i) & 1) x |= 1u << reg[i];
+        return "lds[f" + std::to_string(n - 1) + " + " + std::to_string(pad(x)) + "u]";
+    }
+
+    // One exchange of the registers' `part` (whole amplitudes, or a component).
+    void move(std::string &o, const PhaseMap &from, const PhaseMap &to, const std::string &part) {
+        const int A = 1 << a;
+        if (!in_place) {
+            o += "        __syncthreads();\n";
+            place(from);
+        }
+        if (!n || !in_place) o += declare();
+        for (int k = 0; k < A; ++k) o += "        " + slot(k) + " = a" + std::to_string(k) + part + ";\n";
+        // the reader of tile bit b finds it at the slot bit of whichever bit held b
+        int t2[kMaxThreadBits], r2[8];
+        auto held = [&](int b) {
+            for (int j = 0; j < tb; ++j) if (thr_bit(from, j) == b) return thr[j];
+            for (int i = 0; i < a; ++i) if (reg_bit(from, i) == b) return reg[i];
+            return 0;   // not reached: both maps cover the tile
+        };
+        for (int j = 0; j < tb; ++j) t2[j] = held(thr_bit(to, j));
+        for (int i = 0; i < a; ++i) r2[i] = held(reg_bit(to, i));
+        std::copy(t2, t2 + tb, thr);
+        std::copy(r2, r2 + a, reg);
+        o += declare();
+        o += "        __syncthreads();\n";
+        for (int k = 0; k < A; ++k) o += "        a" + std::to_string(k) + part + " = " + slot(k) + ";\n";
+    }
+};
 
 // Amplitude types of the generated kernels and their state accessors: with
 // the nontemporal (streaming) hint (hgm_ld, hgm_st) and without (hgm_ldp,
@@ -263,14 +334,8 @@ std::string kernel_body(const Gen &g, const Plan &plan, const Pass &ps, const st
     o += "    const unsigned t = threadIdx.x;\n";
     o += "    const unsigned long long lt = " + thread_or(lt, tb) + ";\n";
     o += "    const unsigned long long st = " + thread_or(st, tb) + ";\n";
-    // thread parts of the LDS slot of every phase map of this pass
-    const int m_first = pm.first_map, m_last = pm.last_map;
-    if (ps.phases > 1)
-        for (int mi = m_first; mi <= m_last; ++mi) {
-            uint32_t c[kMaxThreadBits] = {0};
-            for (int j = 0; j < tb; ++j) c[j] = padded(unswizzle(plan.maps[mi].thr[j / 5][1 << (j % 5)]));
-            o += "    const unsigned f" + std::to_string(mi - m_first) + " = " + thread_sum(c, tb) + ";\n";
-        }
+    const int m_first = pm.first_map;
+    Exchange ex(B, A, plan.maps[m_first], g.f32, kPad);
     // one tile per workgroup: no loop, so the matrix literals are not kept
     // live across tiles
     (void)n_tiles;
@@ -333,20 +398,9 @@ std::string kernel_body(const Gen &g, const Plan &plan, const Pass &ps, const st
         if (!is_phase(op)) flush_factors();   // other phases commute with the pending factors
         if (op.kind == R_REMAP) {
             flush_scales();
-            const int nxt = op.rbit;
-            const char *parts[2][2] = {{"", nullptr}, {".x", ".y"}};
-            for (int h = 0; h < 2 && parts[g.split][h]; ++h) {
-                const std::string part = parts[g.split][h];
-                o += "        __syncthreads();\n";
-                for (int k = 0; k < A; ++k)
-                    o += "        lds[f" + std::to_string(cur - m_first) + " + " +
-                         std::to_string(padded(unswizzle(plan.maps[cur].reg[k]))) + "u] = " + reg(k) + part + ";\n";
-                o += "        __syncthreads();\n";
-                for (int k = 0; k < A; ++k)
-                    o += "        " + reg(k) + part + " = lds[f" + std::to_string(nxt - m_first) + " + " +
-                         std::to_string(padded(unswizzle(plan.maps[nxt].reg[k]))) + "u];\n";
-            }
-            cur = nxt;
+            for (const char *part : {g.split ? ".x" : "", g.split ? ".y" : (const char *)nullptr})
+                if (part) ex.move(o, plan.maps[cur], plan.maps[op.rbit], part);
+            cur = op.rbit;
             continue;
         }
         std::string body;
@@ -425,7 +479,7 @@ void jit_generate(const Plan &plan, JitCode *out) {
     // above 32 KiB moves through LDS in two halves of scalars instead, which
     // doubles the resident workgroups for two more barriers per remap
     const uint64_t last = (uint64_t(1) << plan.shape.r) - 1;
-    const size_t entries = (size_t)padded((uint32_t)last) + 1;
+    const size_t entries = (size_t)kPad((uint32_t)last) + 1;
     g.split = entries * amp_bytes(plan.dtype) > 32 * 1024;
     bool ld, st;
     state_streams((size_t(1) << plan.qubits) * amp_bytes(plan.dtype), &ld, &st);
@@ -602,7 +656,8 @@ std::string serving_kernel_source(const Plan &plan, const Pass &ps, const std::s
     g.V = g.f32 ? "hgm_f2" : "hgm_d2";
     g.T = g.f32 ? "float" : "double";
     const uint64_t last = (uint64_t(1) << plan.shape.r) - 1;
-    const size_t entries = (size_t)padded((uint32_t)last) + 1;
+    const Pad pad = g.f32 ? kServingPad32 : kPad;
+    const size_t entries = (size_t)pad((uint32_t)last) + 1;
     g.split = entries * amp_bytes(plan.dtype) > 32 * 1024;
     *lds_bytes = ps.phases > 1 ? entries * amp_bytes(plan.dtype) / (g.split ? 2 : 1) : 0;
     const int B = plan.shape.B, A = 2 * plan.shape.R;
@@ -644,13 +699,8 @@ std::string serving_kernel_source(const Plan &plan, const Pass &ps, const std::s
     o += "    const unsigned long long base = " + base_expr(nonlocal) + ";\n";
     o += "    const unsigned long long lt = " + thread_or(lt, tb) + ";\n";
     o += "    const unsigned long long st = " + thread_or(st, tb) + ";\n";
-    const int m_first = pm.first_map, m_last = pm.last_map;
-    if (ps.phases > 1)
-        for (int mi = m_first; mi <= m_last; ++mi) {
-            uint32_t c[kMaxThreadBits] = {0};
-            for (int j = 0; j < tb; ++j) c[j] = padded(unswizzle(plan.maps[mi].thr[j / 5][1 << (j % 5)]));
-            o += "    const unsigned f" + std::to_string(mi - m_first) + " = " + thread_sum(c, tb) + ";\n";
-        }
+    const int m_first = pm.first_map;
+    Exchange ex(B, A, plan.maps[m_first], g.f32, pad);
     for (int k = 0; k < A; ++k)
         o += "    " + g.V + " " + reg(k) + " = s[(base | " + hex64(pm.lreg[k]) + ") + lt];\n";
     int cur = m_first;
@@ -658,20 +708,9 @@ std::string serving_kernel_source(const Plan &plan, const Pass &ps, const std::s
         const RegOp &op = plan.rops[ps.rop_begin + i];
         const std::string oi = "ops[" + std::to_string(i) + "]";
         if (op.kind == R_REMAP) {
-            const int nxt = op.rbit;
-            const char *parts[2][2] = {{"", nullptr}, {".x", ".y"}};
-            for (int h = 0; h < 2 && parts[g.split][h]; ++h) {
-                const std::string part = parts[g.split][h];
-                o += "    __syncthreads();\n";
-                for (int k = 0; k < A; ++k)
-                    o += "    lds[f" + std::to_string(cur - m_first) + " + " +
-                         std::to_string(padded(unswizzle(plan.maps[cur].reg[k]))) + "u] = " + reg(k) + part + ";\n";
-                o += "    __syncthreads();\n";
-                for (int k = 0; k < A; ++k)
-                    o += "    " + reg(k) + part + " = lds[f" + std::to_string(nxt - m_first) + " + " +
-                         std::to_string(padded(unswizzle(plan.maps[nxt].reg[k]))) + "u];\n";
-            }
-            cur = nxt;
+            for (const char *part : {g.split ? ".x" : "", g.split ? ".y" : (const char *)nullptr})
+                if (part) ex.move(o, plan.maps[cur], plan.maps[op.rbit], part);
+            cur = op.rbit;
             continue;
         }
         // the op's coefficients and control values are read from the item's
