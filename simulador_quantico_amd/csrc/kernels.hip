@@ -385,7 +385,9 @@ __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const
         if (!tile) continue;
         const auto lane = [&] { return (t & o.tmask) == o.tval; };
         switch (o.kind) {
-            case X_ROTS: rotations<T, A>(a, o.m); break;
+            case X_ROTS:
+                if constexpr (sizeof(T) == 4) rotations<T, A>(a, o.m);
+                break;
             case X_VEC: {
                 const T *__restrict__ f = table + o.pmask;
 #pragma unroll
@@ -401,7 +403,9 @@ __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const
                 }
                 break;
             }
-            case X_ROT: gate<T, A, X_ROT>(a, o.m, o.bit); break;
+            case X_ROT:
+                if constexpr (sizeof(T) == 4) gate<T, A, X_ROT>(a, o.m, o.bit);
+                break;
             case X_DENSE: gate<T, A, X_DENSE>(a, o.m, o.bit); break;
             case X_DENSE_REAL: gate<T, A, X_DENSE_REAL>(a, o.m, o.bit); break;
             case X_SWAP: gate<T, A, X_SWAP>(a, o.m, o.bit, lane()); break;

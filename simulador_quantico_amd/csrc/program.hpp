@@ -9,7 +9,8 @@
 // otherwise work out per workgroup is worked out here once: coefficients are
 // in the amplitude type, register conditions are masks of registers or pairs,
 // an uncontrolled X is a renaming of the two values of a tile bit that costs
-// nothing, and an uncontrolled unitary gate is a real rotation between phases:
+// nothing, and in FP32 an uncontrolled unitary gate is a real rotation between
+// phases:
 //   U = diag(e0, e1) * [[1, t0], [t1, 1]] * diag(1, y)
 // (rows exchanged where the off-diagonal entries are the larger ones). The
 // rotation costs 4 multiply-adds per pair where U costs 16; the phases of all
@@ -28,7 +29,7 @@ enum XKind : uint32_t {
     // gates on the register pairs (x, y) that differ in register bit `bit`
     X_DENSE = 0,       // 2x2 complex matrix m[0..7]
     X_DENSE_REAL = 1,  // real matrix m[0], m[2], m[4], m[6]
-    X_ROT = 2,         // x + m0 y, y + m1 x
+    X_ROT = 2,         // x + m0 y, y + m1 x (FP32 programs only, as X_ROTS)
     X_ROTS = 3,        // X_ROT with m[2 b], m[2 b + 1] on every register bit b (up to 4)
     // under a condition on threads (tmask, tval): y, x; a 2x2 matrix; a real one
     X_SWAP = 4, X_DENSE_LANE = 5, X_REAL_LANE = 6,
