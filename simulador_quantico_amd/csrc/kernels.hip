@@ -183,8 +183,13 @@ __device__ __forceinline__ void pair_update(typename Vec<T>::type &x, typename V
         x.y = m[0] * p.y + m[2] * q.y;
         y.x = m[4] * p.x + m[6] * q.x;
         y.y = m[4] * p.y + m[6] * q.y;
+    } else if constexpr (KIND == X_ROT && sizeof(T) == 8) {
+        x.x = p.x + m[0] * q.x - m[1] * q.y;
+        x.y = p.y + m[0] * q.y + m[1] * q.x;
+        y.x = q.x + m[2] * p.x - m[3] * p.y;
+        y.y = q.y + m[2] * p.y + m[3] * p.x;
     } else {
-        static_assert(KIND == X_ROT);
+        static_assert(KIND == X_ROT || KIND == X_ROTS);
         x.x = p.x + m[0] * q.x;
         x.y = p.y + m[0] * q.y;
         y.x = q.x + m[1] * p.x;
@@ -290,7 +295,7 @@ __device__ __forceinline__ void rotations(typename Vec<T>::type (&a)[A], const T
         const T u[8] = {m[2 * b], m[2 * b + 1]};
 #pragma unroll
         for (int k = 0; k < A; ++k)
-            if (!((k >> b) & 1)) pair_update<T, X_ROT>(a[k], a[k | (1 << b)], u);
+            if (!((k >> b) & 1)) pair_update<T, X_ROTS>(a[k], a[k | (1 << b)], u);
     }
 }
 
@@ -385,9 +390,7 @@ __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const
         if (!tile) continue;
         const auto lane = [&] { return (t & o.tmask) == o.tval; };
         switch (o.kind) {
-            case X_ROTS:
-                if constexpr (sizeof(T) == 4) rotations<T, A>(a, o.m);
-                break;
+            case X_ROTS: rotations<T, A>(a, o.m); break;
             case X_VEC: {
                 const T *__restrict__ f = table + o.pmask;
 #pragma unroll
@@ -403,9 +406,7 @@ __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const
                 }
                 break;
             }
-            case X_ROT:
-                if constexpr (sizeof(T) == 4) gate<T, A, X_ROT>(a, o.m, o.bit);
-                break;
+            case X_ROT: gate<T, A, X_ROT>(a, o.m, o.bit); break;
             case X_DENSE: gate<T, A, X_DENSE>(a, o.m, o.bit); break;
             case X_DENSE_REAL: gate<T, A, X_DENSE_REAL>(a, o.m, o.bit); break;
             case X_SWAP: gate<T, A, X_SWAP>(a, o.m, o.bit, lane()); break;

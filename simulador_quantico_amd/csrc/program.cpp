@@ -207,10 +207,28 @@ void emit(const Item &it, uint32_t S, bool split, uint32_t &flip, C &scale, Rota
             if (t.exchanged) flip ^= tb;
             o.kind = X_ROT;
             o.m[0] = t.t0;
-            o.m[1] = t.t1;
+            o.m[2] = t.t1;
             out.push_back(o);
             scale *= t.e0;
             phase(t.e1, tb, tb, 0, 0);
+            return;
+        }
+    }
+    // Rows that each hold an exact 1 (HGM_PLAN_PIVOT), in different columns: half
+    // the multiply-adds, and no rounding that the whole gate does not have. 8
+    // random layers at 26 qubits, complex128: 6.6 -> 5.5 ms; Grover at 22: 1.36 ->
+    // 1.19. A record kind of its own beside the real rotation made the kernels
+    // larger: 6 layers at 12 qubits, which run neither, 59 -> 62 us.
+    if (free_gate && !split) {
+        const int ex = is_one(m[0], m[1]) && is_one(m[6], m[7]) ? 0 : is_one(m[2], m[3]) && is_one(m[4], m[5]) ? 1 : -1;
+        if (ex >= 0 && it.kind != K_ANTI) {
+            // rows exchanged (ex): the new row 0 is row 1, the new row 1 is row 0
+            const double *t0 = m + (ex ? 6 : 2), *t1 = m + (ex ? 0 : 4);
+            o.kind = X_ROT;
+            std::copy(t0, t0 + 2, o.m);
+            std::copy(t1, t1 + 2, o.m + 2);
+            if (ex) flip ^= tb;
+            out.push_back(o);
             return;
         }
     }
@@ -360,6 +378,13 @@ struct Records {
         }
     }
 
+    // A rotation by itself: FP32 ones are real, FP64 ones may be complex.
+    XOp<T> rotation(const ROp &o) {
+        XOp<T> x = record<T>(o, A);
+        if (sizeof(T) == 4) x.m[1] = x.m[2];
+        return x;
+    }
+
     // A run of rotations: those on different register bits commute, and three
     // of a full set of four (two of two or three) already cost less as one
     // record than one by one.
@@ -368,22 +393,24 @@ struct Records {
         while (b != e) {
             uint32_t used = 0;
             It n = b;
-            for (; n != e && (*n)->bit < bits && !((used >> (*n)->bit) & 1u); ++n) used |= 1u << (*n)->bit;
-            if (n == b) ++n;   // a fifth register bit
+            for (; n != e && (*n)->bit < bits && !((used >> (*n)->bit) & 1u) && real(**n); ++n) used |= 1u << (*n)->bit;
+            if (n == b) ++n;   // a fifth register bit, or complex
             if (popc(used) >= (bits + 2) / 2 && bits > 1) {
                 XOp<T> x;
                 std::memset(&x, 0, sizeof x);
                 x.kind = X_ROTS;
                 for (; b != n; ++b) {
                     x.m[2 * (*b)->bit] = (T)(*b)->m[0];
-                    x.m[2 * (*b)->bit + 1] = (T)(*b)->m[1];
+                    x.m[2 * (*b)->bit + 1] = (T)(*b)->m[2];
                 }
                 ops.push_back(x);
             } else {
-                for (; b != n; ++b) ops.push_back(record<T>(**b, A));
+                for (; b != n; ++b) ops.push_back(rotation(**b));
             }
         }
     }
+
+    static bool real(const ROp &o) { return o.m[1] == 0 && o.m[3] == 0; }
 
     void stage(std::vector<ROp> &list) {
         into_waves(list, order);

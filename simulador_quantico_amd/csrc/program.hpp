@@ -13,7 +13,8 @@
 // phases:
 //   U = diag(e0, e1) * [[1, t0], [t1, 1]] * diag(1, y)
 // (rows exchanged where the off-diagonal entries are the larger ones). The
-// rotation costs 4 multiply-adds per pair where U costs 16; the phases of all
+// rotation costs 4 multiply-adds per pair where U costs 16 (in FP64, 8 where
+// the planner scaled both rows to an exact 1); the phases of all
 // gates of a wave, with whatever else is diagonal there, are one factor per
 // register.
 #pragma once
@@ -29,8 +30,8 @@ enum XKind : uint32_t {
     // gates on the register pairs (x, y) that differ in register bit `bit`
     X_DENSE = 0,       // 2x2 complex matrix m[0..7]
     X_DENSE_REAL = 1,  // real matrix m[0], m[2], m[4], m[6]
-    X_ROT = 2,         // x + m0 y, y + m1 x (FP32 programs only, as X_ROTS)
-    X_ROTS = 3,        // X_ROT with m[2 b], m[2 b + 1] on every register bit b (up to 4)
+    X_ROT = 2,         // x + m0 y, y + m1 x; in FP64 x + (m0 + i m1) y, y + (m2 + i m3) x
+    X_ROTS = 3,        // real rotations with m[2 b], m[2 b + 1] on every register bit b (up to 4)
     // under a condition on threads (tmask, tval): y, x; a 2x2 matrix; a real one
     X_SWAP = 4, X_DENSE_LANE = 5, X_REAL_LANE = 6,
     // and only on the pairs in pmask (bit k: the pair whose lower register is k)
