@@ -429,13 +429,24 @@ void planner_loop(hgm_server *s) {
             r->lane = r->n_tiles == 1 ? 0 : 1;
             r->state_bytes = align_up((size_t(1) << r->qubits) * amp_bytes(s->cfg.dtype));
             // on the device: the compiled passes' register programs and the interpreted passes' programs
-            r->rop_bytes = 0;
-            for (int k : r->kernel)
-                if (k >= 0) r->rop_bytes = align_up(p.rops.size() * sizeof(RegOp));
-            r->prog_bytes = r->rop_bytes + align_up(p.xprog.size() * sizeof(uint64_t));
-            r->part_bytes = align_up((size_t)r->n_tiles * sizeof(ReadoutPartial));
-            r->total_bytes = r->state_bytes + r->prog_bytes + r->part_bytes;
-            if (r->total_bytes > s->arena.size() || r->prog_bytes > s->staging.size()) {
+            const auto fits = [&] {
+                r->rop_bytes = 0;
+                for (int k : r->kernel)
+                    if (k >= 0) r->rop_bytes = align_up(p.rops.size() * sizeof(RegOp));
+                r->prog_bytes = r->rop_bytes + align_up(p.xprog.size() * sizeof(uint64_t));
+                r->part_bytes = align_up((size_t)r->n_tiles * sizeof(ReadoutPartial));
+                r->total_bytes = r->state_bytes + r->prog_bytes + r->part_bytes;
+                return r->total_bytes <= s->arena.size() && r->prog_bytes <= s->staging.size();
+            };
+            // with passes of both kinds the two forms are up to 1.9 times the
+            // register program and its maps; the interpreter's alone is
+            // smaller than those: where both do not fit, it runs every pass
+            bool ok = fits();
+            if (!ok && !p.xprog.empty()) {
+                r->kernel.assign(r->passes.size(), -1);
+                ok = fits();
+            }
+            if (!ok) {
                 rc = HGM_E_ARG;
                 err = "the request's footprint exceeds the serving HBM budget";
             }
