@@ -546,7 +546,7 @@ void jit_generate(const Plan &plan, JitCode *out) {
     g.T = g.f32 ? "float" : "double";
     // LDS per workgroup caps the workgroups a CU holds (160 KiB each): a tile
     // above 32 KiB moves through LDS in two halves of scalars instead, which
-    // doubles the resident workgroups for two more barriers per remap
+    // doubles the resident workgroups for one more barrier per remap (two in FP64)
     const uint64_t last = (uint64_t(1) << plan.shape.r) - 1;
     const size_t entries = (size_t)kPad((uint32_t)last) + 1;
     g.split = entries * amp_bytes(plan.dtype) > 32 * 1024;
