@@ -340,6 +340,12 @@ __device__ __forceinline__ uint64_t reg_bits(int k, const uint64_t *__restrict__
     return flip;
 }
 
+// Real (0) or imaginary (1) part of a phase record's factor.
+__device__ __forceinline__ double phase_part(const XOp<double> &o, int part) { return o.m[part]; }
+__device__ __forceinline__ double phase_part(const XOp<float> &o, int part) {
+    return __hiloint2double(__float_as_int(o.m[2 * part + 1]), __float_as_int(o.m[2 * part]));
+}
+
 // Runs the records of a pass on the registers of one tile.
 template <class T, int A>
 __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const XPass *__restrict__ xp, uint64_t base,
@@ -351,7 +357,7 @@ __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const
     const int n = xp->n_ops;
     XMap cur = xp->first;
     uint32_t pos = lds_pos<T, A>(t, cur);
-    T fr = T(1), fi = T(0);
+    double fr = 1, fi = 0;
     XOp<T> next = ops[0];
     for (int i = 0; i < n; ++i) {
         const XOp<T> o = next;
@@ -373,18 +379,18 @@ __device__ __forceinline__ void run_program(typename Vec<T>::type (&a)[A], const
         if (o.kind == X_PHASE) {
             if (!tile && (o.flags & (X_FIRST | X_LAST)) == (X_FIRST | X_LAST)) continue;
             const bool on = tile && (t & o.tmask) == o.tval;
-            const T gr = on ? o.m[0] : T(1), gi = on ? o.m[1] : T(0);
+            const double gr = on ? phase_part(o, 0) : 1.0, gi = on ? phase_part(o, 1) : 0.0;
             if (o.flags & X_FIRST) {
                 fr = gr;
                 fi = gi;
             } else if (o.flags & X_REAL) {
                 fr *= gr;
             } else {
-                const T r = fr * gr - fi * gi;
+                const double r = fr * gr - fi * gi;
                 fi = fr * gi + fi * gr;
                 fr = r;
             }
-            if (o.flags & X_LAST) phase_apply<T, A>(a, fr, fi, (o.flags & X_REAL) != 0, o.pat, o.pmask);
+            if (o.flags & X_LAST) phase_apply<T, A>(a, (T)fr, (T)fi, (o.flags & X_REAL) != 0, o.pat, o.pmask);
             continue;
         }
         if (!tile) continue;

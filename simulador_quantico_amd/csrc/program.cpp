@@ -282,6 +282,10 @@ XOp<T> record(const ROp &o, uint32_t A) {
     x.gmask = o.gmask;
     x.gval = o.gval;
     for (int i = 0; i < 8; ++i) x.m[i] = (T)o.m[i];
+    if (o.phase) {
+        const double g[2] = {(double)o.m[0], (double)o.m[1]};
+        std::memcpy(x.m, g, sizeof g);
+    }
     for (uint32_t k = 0; k < A; ++k)
         if ((o.phase || !((k >> o.bit) & 1)) && (k & o.rmask) == o.rval) x.pmask |= 1u << k;
     if (o.phase) {

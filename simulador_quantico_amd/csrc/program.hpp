@@ -36,8 +36,8 @@ enum XKind : uint32_t {
     X_SWAP = 4, X_DENSE_LANE = 5, X_REAL_LANE = 6,
     // and only on the pairs in pmask (bit k: the pair whose lower register is k)
     X_DENSE_MASK = 7, X_REAL_MASK = 8,
-    // multiply registers by m0 + i m1: those whose bits in `pat` are all set, those whose bit pat - X_PAT_CLEAR is
-    // clear, or (X_PAT_MASK) those in pmask
+    // multiply registers by a factor, two doubles at m in either type: those whose bits in `pat` are all set, those
+    // whose bit pat - X_PAT_CLEAR is clear, or (X_PAT_MASK) those in pmask
     X_PHASE = 9,
     // multiply every register by a factor of its own: A complex or A real values at word pmask of the pass's table
     X_VEC = 10, X_VEC_REAL = 11,
@@ -46,7 +46,9 @@ enum XKind : uint32_t {
 
 enum XFlag : uint32_t {
     // consecutive phases on the same registers are multiplied into one factor
-    // per lane, applied by the last of them
+    // per lane, applied by the last of them; the product is FP64 in either
+    // type: rounded to FP32 at every phase, all registers of a lane share its
+    // error, and an adder's grows with its size (FP64 issues at the FP32 rate)
     X_FIRST = 1, X_LAST = 2,
     X_REAL = 4         // the whole group's factors are real
 };
