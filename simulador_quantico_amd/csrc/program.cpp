@@ -372,11 +372,17 @@ struct Records {
                 same->m[0] = z.real();
                 same->m[1] = z.imag();
             }
-            bool real = true;
-            for (const ROp &g : group) real = real && g.m[1] == 0;
-            for (size_t k = 0; k < group.size(); ++k) {
-                XOp<T> x = record<T>(group[k], A);
-                x.flags = (uint8_t)((k == 0 ? X_FIRST : 0) | (k + 1 == group.size() ? X_LAST : 0) | (real ? X_REAL : 0));
+            // Where no record of a group holds, its factor is 1, and an infinity times 1 + 0i is no infinity: complex
+            // phases that all wait for some tile are applied one by one, each in its tiles, and real ones (whose 1
+            // changes nothing) by themselves.
+            const auto real = [](const ROp &g) { return g.m[1] == 0; };
+            const bool everywhere = std::any_of(group.begin(), group.end(), [&](const ROp &g) { return !real(g) && !g.gmask; });
+            const auto mid = everywhere ? group.end() : std::stable_partition(group.begin(), group.end(), real);
+            for (auto g = group.begin(); g != group.end(); ++g) {
+                XOp<T> x = record<T>(*g, A);
+                const bool alone = g >= mid;
+                x.flags = (uint8_t)((alone || g == group.begin() ? X_FIRST : 0) | (alone || g + 1 == mid ? X_LAST : 0) |
+                                    (!alone && !everywhere ? X_REAL : 0));
                 ops.push_back(x);
             }
         }

@@ -68,3 +68,28 @@ def test_a_factor_of_many_phases_is_as_exact_as_one(count, n):
         want = a.astype(np.clongdouble) * _factors(n, gates)
         off = np.abs(s.download().astype(np.clongdouble) - want) / np.abs(a)
         assert float(off.max()) <= 3.5 * 2.0**-24, float(off.max()) * 2**24
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("real", [False, True])
+def test_an_infinity_in_a_tile_that_no_phase_holds_in_stays_one(real, dtype):
+    """Two phases of one group, each held in the tiles where its own state bit above the tile is set: one complex, the
+    other real or complex. An infinity stays one in the tiles where neither holds and where only a real one does; the
+    rest of the state has to be finite there."""
+    n = 14
+    print("infinity", real, np.dtype(dtype).name, flush=True)
+    sys.stdout.flush()
+    gates = [(0, 1 << 12, 1 << 12, np.diag([1, -1 if real else 1j])), (1, 1 << 13, 1 << 13, np.diag([1, np.exp(0.7j)]))]
+    a = np.ones(1 << n, dtype)
+    a[0b00 << 12 | 77] = np.inf
+    if real:
+        a[0b01 << 12 | 77] = np.inf
+    plan = hq.Plan(n, hq.make_ops(*zip(*gates)), _tuning(), 1, dtype)
+    s = hq.State(n, dtype)
+    s.upload(a)
+    plan.run(s)
+    got = s.download()
+    assert got[77] == np.inf
+    if real:
+        assert got[1 << 12 | 77] == -np.inf
+    assert np.isfinite(got[np.isfinite(a)]).all()
