@@ -286,7 +286,8 @@ double hgm_plan_compile_seconds(const hgm_plan *p);
  * copied to the device once, here), captured as one hipGraph: states whose
  * plans launch the same kernels with the same programs (one plan shared by
  * many states, or equal plans) advance together, one launch per pass for all
- * of them; the graph forks into up to 64 branches (one per such group, more
+ * of them (states on LDS plans, whose kernel takes one state per launch, each
+ * by itself); the graph forks into up to 64 branches (one per such group, more
  * spread over them by their plans' bytes, largest first), each branch runs its
  * groups' passes in order, and the branches join, so passes of different
  * groups can run at once. One
@@ -298,6 +299,9 @@ double hgm_plan_compile_seconds(const hgm_plan *p);
  * state per call: src/core/kernel.cu:192-282). */
 typedef struct hgm_batch hgm_batch;
 int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int n, hgm_batch **out);
+/* How a batch of states on these plans is laid out, for inspection (no device
+ * needed): for each state the group it advances with and the group's branch. */
+int hgm_batch_layout(const hgm_plan *const *plans, int n, int32_t *group, int32_t *branch);
 /* Launches the batch's graph and waits for it; stats sums the plans' gates,
  * passes and bytes, with the graph's device time as kernel_ms. */
 int hgm_batch_run(hgm_batch *b, hgm_stats *stats);

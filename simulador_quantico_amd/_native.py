@@ -132,6 +132,7 @@ SIGNATURES = [
     ("hgm_plan_compile_seconds", C.c_double, [_P]),
     ("hgm_plan_set_graph", C.c_int, [_P, C.c_int]),
     ("hgm_batch_create", C.c_int, [C.POINTER(_P), C.POINTER(_P), C.c_int, C.POINTER(_P)]),
+    ("hgm_batch_layout", C.c_int, [C.POINTER(_P), C.c_int, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
     ("hgm_batch_run", C.c_int, [_P, C.POINTER(Stats)]),
     ("hgm_batch_destroy", None, [_P]),
     ("hgm_validate_tuning", C.c_int, [C.c_int, C.c_int, C.POINTER(Tuning)]),

@@ -511,6 +511,50 @@ int max_group(const Plan &p) {
     return (int)std::min<uint64_t>(65535, 0xffffffffull / std::max<uint64_t>(items, 1));
 }
 
+// States that share launches, and the fork branch of each such group; returns
+// the number of branches. A state on an LDS plan is a group of its own: that
+// kernel takes one state per launch, and launches on one branch wait for each
+// other.
+int batch_groups(const hgm_plan *const *plans, int n, std::vector<BatchGroup> *groups) {
+    for (int i = 0; i < n; ++i) {
+        const Plan &p = plans[i]->plan;
+        BatchGroup *to = nullptr;
+        for (BatchGroup &g : *groups) {
+            const Plan &q = plans[g.members[0]]->plan;
+            if (p.kernel != HGM_KERNEL_LDS && (int)g.members.size() < max_group(q) &&
+                (plans[i] == plans[g.members[0]] || same_launches(p, q))) {
+                to = &g;
+                break;
+            }
+        }
+        if (!to) {
+            groups->emplace_back();
+            to = &groups->back();
+        }
+        to->members.push_back(i);
+    }
+    // groups by bytes moved, largest first, each to the branch with the fewest so far
+    const int n_groups = (int)groups->size();
+    const int n_branches = std::min(n_groups, kBatchBranches);
+    std::vector<int> order(n_groups);
+    std::vector<double> bytes(n_groups), load(n_branches, 0.0);
+    for (int i = 0; i < n_groups; ++i) {
+        const BatchGroup &g = (*groups)[i];
+        const Plan &p = plans[g.members[0]]->plan;
+        int64_t busy = 0;
+        for (const Pass &ps : p.passes) busy += ps.op_count > 0;
+        bytes[i] = (double)busy * (double)(uint64_t(1) << p.qubits) * (double)amp_bytes(p.dtype) * (double)g.members.size();
+        order[i] = i;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return bytes[a] > bytes[c]; });
+    for (int i : order) {
+        const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+        (*groups)[i].branch = k;
+        load[k] += bytes[i];
+    }
+    return n_branches;
+}
+
 // Captures the batch: a fork on the context stream, each group's passes in
 // order on its branch stream, a join back. Assumes the lock.
 int capture_batch_locked(hgm_batch *b, const std::vector<JitModule *> &jms) {
@@ -527,11 +571,6 @@ int capture_batch_locked(hgm_batch *b, const std::vector<JitModule *> &jms) {
         const char *base = static_cast<const char *>(b->tables);
         const void *table = g.table_off < 0 ? nullptr : base + g.table_off;
         const hipStream_t st = b->streams[g.branch];
-        if (p.kernel == HGM_KERNEL_LDS) {
-            for (int k : g.members)
-                if (!rc) rc = launch_passes_locked({b->states[k]->d}, p, jms[i], table, st);
-            continue;
-        }
         StateSet set{b->states[i]->d};
         if (g.members.size() > 1) {
             set.offs = reinterpret_cast<const int64_t *>(base + g.offs_off);
@@ -1295,43 +1334,7 @@ int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int
     auto b = std::make_unique<hgm_batch>();
     b->states.assign(states, states + n);
     b->plans.assign(plans, plans + n);
-    // states that share launches
-    for (int i = 0; i < n; ++i) {
-        const Plan &p = plans[i]->plan;
-        BatchGroup *to = nullptr;
-        for (BatchGroup &g : b->groups) {
-            const Plan &q = plans[g.members[0]]->plan;
-            if ((int)g.members.size() < max_group(q) &&
-                (plans[i] == plans[g.members[0]] || (p.kernel != HGM_KERNEL_LDS && same_launches(p, q)))) {
-                to = &g;
-                break;
-            }
-        }
-        if (!to) {
-            b->groups.emplace_back();
-            to = &b->groups.back();
-        }
-        to->members.push_back(i);
-    }
-    // groups by bytes moved, largest first, each to the branch with the fewest so far
-    const int n_groups = (int)b->groups.size();
-    b->n_branches = std::min(n_groups, kBatchBranches);
-    std::vector<int> order(n_groups);
-    std::vector<double> bytes(n_groups), load(b->n_branches, 0.0);
-    for (int i = 0; i < n_groups; ++i) {
-        const BatchGroup &g = b->groups[i];
-        const Plan &p = plans[g.members[0]]->plan;
-        int64_t busy = 0;
-        for (const Pass &ps : p.passes) busy += ps.op_count > 0;
-        bytes[i] = (double)busy * (double)(uint64_t(1) << p.qubits) * (double)amp_bytes(p.dtype) * (double)g.members.size();
-        order[i] = i;
-    }
-    std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return bytes[a] > bytes[c]; });
-    for (int i : order) {
-        const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        b->groups[i].branch = k;
-        load[k] += bytes[i];
-    }
+    b->n_branches = batch_groups(plans, n, &b->groups);
     std::lock_guard<std::mutex> g(ctx().mu);
     int rc = init_locked(-1);
     if (rc) return rc;
@@ -1360,10 +1363,12 @@ int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int
     for (BatchGroup &g : b->groups) {
         const Plan &p = plans[g.members[0]]->plan;
         if (p.kernel != HGM_KERNEL_JIT) {
-            g.table_off = place(plan_table(p), plan_table_bytes(p));
+            for (const BatchGroup &other : b->groups)   // one copy of a plan's table
+                if (&other == &g || plans[other.members[0]] == plans[g.members[0]]) { g.table_off = other.table_off; break; }
+            if (g.table_off < 0) g.table_off = place(plan_table(p), plan_table_bytes(p));
             if (e == hipSuccess) e = prepare_pass_kernels(p.dtype);
         }
-        if (g.members.size() > 1 && p.kernel != HGM_KERNEL_LDS) {
+        if (g.members.size() > 1) {
             std::vector<int64_t> offs;
             for (int k : g.members)
                 offs.push_back((int64_t)(static_cast<char *>(states[k]->d) - static_cast<char *>(states[g.members[0]]->d)));
@@ -1386,6 +1391,20 @@ int hgm_batch_create(hgm_state *const *states, const hgm_plan *const *plans, int
         return rc;
     }
     *out = b.release();
+    return HGM_OK;
+}
+
+int hgm_batch_layout(const hgm_plan *const *plans, int n, int32_t *group, int32_t *branch) {
+    if (!plans || n < 1 || !group || !branch) { t_err = "bad arguments"; return HGM_E_ARG; }
+    for (int i = 0; i < n; ++i)
+        if (!plans[i]) { t_err = "null plan"; return HGM_E_ARG; }
+    std::vector<BatchGroup> groups;
+    batch_groups(plans, n, &groups);
+    for (size_t g = 0; g < groups.size(); ++g)
+        for (int i : groups[g].members) {
+            group[i] = (int32_t)g;
+            branch[i] = groups[g].branch;
+        }
     return HGM_OK;
 }
 

@@ -430,6 +430,14 @@ class Batch:
             lib.hgm_batch_destroy(h)
             self._h = None
 
+    @staticmethod
+    def layout(plans):
+        """How a batch on these plans is laid out (needs no GPU): per state its launch group and the group's branch."""
+        n = len(plans)
+        group, branch = (C.c_int32 * max(1, n))(), (C.c_int32 * max(1, n))()
+        check(lib.hgm_batch_layout((C.c_void_p * max(1, n))(*[p._h for p in plans]), n, group, branch))
+        return list(group)[:n], list(branch)[:n]
+
     def run(self) -> dict:
         st = Stats()
         check(lib.hgm_batch_run(self._h, C.byref(st)))
