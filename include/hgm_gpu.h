@@ -255,7 +255,16 @@ int hgm_plan_shape(const hgm_plan *p, int32_t *region_bits, int32_t *block_size,
 int hgm_state_run_plan(hgm_state *s, const hgm_plan *p, hgm_stats *stats);
 /* Kernel family the plan runs on (HGM_KERNEL_LDS, HGM_KERNEL_REG or HGM_KERNEL_JIT; never AUTO). */
 int hgm_plan_kernel(const hgm_plan *p);
-/* Register-kernel program of pass i, for inspection: rops receives n_rops
+/* What the interpreted register kernels run for a plan of that family, for
+ * inspection: shape receives the tile bits, amplitudes per thread, threads and
+ * whether remaps have barriers, program the n_bytes bytes of all launches'
+ * programs (records of csrc/program.hpp), and launches, for each of n_launches,
+ * the byte offset of its program and its number of stages. NULL buffers query
+ * the sizes. */
+int hgm_plan_exec_program(const hgm_plan *p, int32_t *shape, void *program, int64_t *n_bytes, int64_t *launches,
+                          int64_t *n_launches);
+/* Register program of pass i (what the plan-compiled and serving kernels are
+ * generated from), for inspection: rops receives n_rops
  * records of 104 bytes, local_pos the 16 tile-bit -> state-bit entries, and
  * first/last the phase maps of the load and store assignments. Passing NULL
  * buffers queries n_rops. */

@@ -1295,6 +1295,29 @@ int hgm_plan_maps(const hgm_plan *p, void *maps, int64_t *n_maps) {
     return HGM_OK;
 }
 
+int hgm_plan_exec_program(const hgm_plan *p, int32_t *shape, void *program, int64_t *n_bytes, int64_t *launches,
+                          int64_t *n_launches) {
+    if (!p || !n_bytes || !n_launches || p->plan.kernel != HGM_KERNEL_REG) {
+        t_err = "launch programs belong to plans on the interpreted register kernels";
+        return HGM_E_ARG;
+    }
+    const Plan &q = p->plan;
+    *n_bytes = (int64_t)(q.xprog.size() * sizeof(uint64_t));
+    *n_launches = (int64_t)q.xlaunch.size();
+    if (shape) {
+        shape[0] = q.exec.r;
+        shape[1] = q.exec.A;
+        shape[2] = q.exec.B;
+        shape[3] = q.exec.sync;
+    }
+    if (program && *n_bytes) std::memcpy(program, q.xprog.data(), (size_t)*n_bytes);
+    for (size_t i = 0; launches && i < q.xlaunch.size(); ++i) {
+        launches[2 * i] = q.xlaunch[i].off;
+        launches[2 * i + 1] = q.xlaunch[i].stages;
+    }
+    return HGM_OK;
+}
+
 int hgm_state_run_plan(hgm_state *s, const hgm_plan *p, hgm_stats *stats) {
     if (!s || !p) { t_err = "null argument"; return HGM_E_ARG; }
     auto t0 = std::chrono::steady_clock::now();

@@ -388,8 +388,18 @@ class Plan:
         check(lib.hgm_plan_jit_source(self._h, buf, n.value + 1, C.byref(n)))
         return buf.value.decode()
 
+    def exec_program(self):
+        """What the interpreted register kernels run: (tile bits, amplitudes per thread, threads, barriers), the
+        programs' bytes, and per launch the byte offset of its program and its number of stages."""
+        shape = (C.c_int32 * 4)()
+        nb, nl = C.c_int64(), C.c_int64()
+        check(lib.hgm_plan_exec_program(self._h, shape, None, C.byref(nb), None, C.byref(nl)))
+        prog, at = np.zeros(nb.value, np.uint8), np.zeros((nl.value, 2), np.int64)
+        check(lib.hgm_plan_exec_program(self._h, shape, prog.ctypes.data, C.byref(nb), at.ctypes.data, C.byref(nl)))
+        return tuple(shape), prog, at
+
     def program(self, i: int):
-        """Register-kernel program of pass i: (structured ops, first map, last map, local_pos)."""
+        """Register program of pass i: (structured ops, first map, last map, local_pos)."""
         n = C.c_int64()
         f, l = C.c_int32(), C.c_int32()
         check(lib.hgm_plan_program(self._h, i, None, C.byref(n), C.byref(f), C.byref(l), None))
@@ -444,9 +454,24 @@ class Batch:
         return st.as_dict()
 
 
-# record layouts of csrc/planner.hpp (RegOp, PhaseMap)
+# record layouts of csrc/planner.hpp (RegOp, PhaseMap) and csrc/program.hpp
 REGOP_DTYPE = np.dtype([("kind", np.int32), ("rbit", np.int32), ("rmask", np.uint32), ("rval", np.uint32),
                         ("tmask", np.uint32), ("tval", np.uint32), ("gmask", np.uint64), ("gval", np.uint64),
                         ("m", np.float64, 8)])
+XRUN_DTYPE = np.dtype([("mask", np.uint32), ("from", np.uint16), ("to", np.uint16)])
+XMAP_DTYPE = np.dtype([("low", np.uint16, 5), ("sw", np.uint16, 5), ("pad", np.uint32, 3)])
+XPASS_DTYPE = np.dtype([("n_ops", np.int32), ("n_base", np.int32), ("n_load", np.int32), ("n_store", np.int32),
+                        ("table", np.int64), ("pad", np.int64, 7), ("first", XMAP_DTYPE), ("lbit", np.uint64, 5),
+                        ("sbit", np.uint64, 5), ("sflip", np.uint64), ("rflip", np.uint64), ("base", XRUN_DTYPE, 18),
+                        ("load", XRUN_DTYPE, 10), ("store", XRUN_DTYPE, 10)])
+
+
+def xop_dtype(real):
+    """A record of the interpreted kernels' programs (csrc/program.hpp XOp) for coefficients of type `real`."""
+    return np.dtype([("kind", np.uint8), ("bit", np.uint8), ("pat", np.uint8), ("flags", np.uint8), ("pmask", np.uint32),
+                     ("tmask", np.uint32), ("tval", np.uint32), ("gmask", np.uint64), ("gval", np.uint64), ("m", real, 8)])
+
+
 PHASEMAP_DTYPE = np.dtype([("reg", np.uint16, 64), ("thr", np.uint16, (2, 32))])
 assert REGOP_DTYPE.itemsize == 104 and PHASEMAP_DTYPE.itemsize == 256
+assert XPASS_DTYPE.itemsize == 512 and xop_dtype(np.float32).itemsize == 64 and xop_dtype(np.float64).itemsize == 96

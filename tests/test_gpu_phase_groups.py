@@ -70,6 +70,28 @@ def test_a_factor_of_many_phases_is_as_exact_as_one(count, n):
         assert float(off.max()) <= 3.5 * 2.0**-24, float(off.max()) * 2**24
 
 
+@pytest.mark.parametrize("n", [12, 14])
+@pytest.mark.parametrize("count", [5, 60])
+def test_the_compiled_kernels_factor_is_as_exact(count, n):
+    """The plan-compiled kernels gather such phases too (from 3 on), into an FP64 factor: the same bound."""
+    print("compiled phase groups", count, n, flush=True)
+    sys.stdout.flush()
+    t = _tuning()
+    t.kernel = N.HGM_KERNEL_JIT
+    for seed in range(2):
+        r = np.random.default_rng(1000 * n + 10 * count + seed)
+        gates = _phases(n, count, r)
+        plan = hq.Plan(n, hq.make_ops(*zip(*gates)), t, 1, np.complex64)
+        assert plan.kernel == N.HGM_KERNEL_JIT and len(plan) == 1
+        a = (r.standard_normal(1 << n) + 1j * r.standard_normal(1 << n)).astype(np.complex64)
+        s = hq.State(n, np.complex64)
+        s.upload(a)
+        plan.run(s)
+        want = a.astype(np.clongdouble) * _factors(n, gates)
+        off = np.abs(s.download().astype(np.clongdouble) - want) / np.abs(a)
+        assert float(off.max()) <= 3.5 * 2.0**-24, float(off.max()) * 2**24
+
+
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
 @pytest.mark.parametrize("real", [False, True])
 def test_an_infinity_in_a_tile_that_no_phase_holds_in_stays_one(real, dtype):
