@@ -147,13 +147,16 @@ uint64_t g_module_tick = 0;
 
 uint64_t g_module_gen = 0;
 
-// Workspace of hgm_state_apply_noalloc: the plan tables (register programs,
-// phase maps and pass tables, or op tables) of one call. Each GPU holds its
-// own copy for the life of the process. In host code `scratch` is only a
+// Workspace of hgm_state_apply_noalloc: the plan's table (the interpreted
+// kernels' programs, or op tables) of one call. Each GPU holds its own copy
+// for the life of the process. In host code `scratch` is only a
 // stand-in for the symbol: its device address is looked up once per device
 // (init_locked) and kept in g_scratch_ptr, and only that address is used.
 constexpr size_t kScratchBytes = size_t(8) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// Passes of a register plan that one such call takes: the call has refused
+// more since each of them took a pass table and a phase map of the workspace.
+constexpr size_t kNoallocPasses = kScratchBytes / (sizeof(PassMem) + sizeof(PhaseMap));
 constexpr int kMaxDevices = 64;
 void *g_scratch_ptr[kMaxDevices] = {};
 
@@ -361,16 +364,6 @@ const void *plan_table(const Plan &p) {
 }
 size_t plan_table_bytes(const Plan &p) {
     return p.kernel == HGM_KERNEL_REG ? p.xprog.size() * sizeof(uint64_t) : p.ops.size() * sizeof(DevOp);
-}
-
-// Bytes of a register plan's inspectable program (hgm_plan_program,
-// hgm_plan_maps): part of the size limit of hgm_state_apply_noalloc.
-size_t register_program_bytes(const Plan &p) {
-    if (p.kernel == HGM_KERNEL_REG) need_register_program(p);
-    return p.kernel == HGM_KERNEL_REG ? align256(p.rops.size() * sizeof(RegOp)) +
-                                            align256(p.maps.size() * sizeof(PhaseMap)) +
-                                            align256(p.mems.size() * sizeof(PassMem))
-                                      : 0;
 }
 
 // Launches every non-empty pass of the plan on `stream`, with no events or
@@ -1067,7 +1060,12 @@ int hgm_state_apply_noalloc(hgm_state *s, const hgm_op *ops, int64_t n_ops, cons
     double plan_ms = 0;
     int rc = cached_plan(s->qubits, s->dtype, ops, n_ops, iterations, t, &p, &plan_ms);
     if (rc) return rc;
-    const size_t need = std::max(plan_table_bytes(*p), register_program_bytes(*p));
+    if (p->kernel == HGM_KERNEL_REG && p->passes.size() > kNoallocPasses) {
+        t_err = "hgm_state_apply_noalloc: the plan has " + std::to_string(p->passes.size()) + " passes, above the " +
+                std::to_string(kNoallocPasses) + " of one call";
+        return HGM_E_ARG;
+    }
+    const size_t need = plan_table_bytes(*p);
     if (need > kScratchBytes) {
         t_err = "hgm_state_apply_noalloc: the plan's tables take " + std::to_string(need) + " bytes, above the " +
                 std::to_string(kScratchBytes) + "-byte workspace (fewer passes or gates per call)";
