@@ -260,9 +260,10 @@ int hgm_plan_kernel(const hgm_plan *p);
  * inspection: shape receives the tile bits, amplitudes per thread, threads and
  * whether remaps have barriers, program the n_bytes bytes of all launches'
  * programs (records of csrc/program.hpp), and launches, for each of n_launches,
- * the byte offset of its program and its number of stages. NULL buffers query
- * the sizes. */
-int hgm_plan_exec_program(const hgm_plan *p, int32_t *shape, void *program, int64_t *n_bytes, int64_t *launches,
+ * the byte offset of its program and its number of stages. compact: the form
+ * that is built where the usual one does not fit a given memory. NULL buffers
+ * query the sizes. */
+int hgm_plan_exec_program(const hgm_plan *p, int compact, int32_t *shape, void *program, int64_t *n_bytes, int64_t *launches,
                           int64_t *n_launches);
 /* Register program of pass i (what the plan-compiled and serving kernels are
  * generated from), for inspection: rops receives n_rops

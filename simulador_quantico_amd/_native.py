@@ -125,7 +125,7 @@ SIGNATURES = [
     ("hgm_state_run_plan", C.c_int, [_P, _P, C.POINTER(Stats)]),
     ("hgm_plan_kernel", C.c_int, [_P]),
     ("hgm_plan_serving_source", C.c_int, [_P, C.c_int64, C.c_char_p, C.c_size_t, C.POINTER(C.c_size_t)]),
-    ("hgm_plan_exec_program", C.c_int, [_P, C.POINTER(C.c_int32), _P, C.POINTER(C.c_int64), _P, C.POINTER(C.c_int64)]),
+    ("hgm_plan_exec_program", C.c_int, [_P, C.c_int, C.POINTER(C.c_int32), _P, C.POINTER(C.c_int64), _P, C.POINTER(C.c_int64)]),
     ("hgm_plan_program", C.c_int, [_P, C.c_int64, _P, C.POINTER(C.c_int64), C.POINTER(C.c_int32),
                                    C.POINTER(C.c_int32), _P]),
     ("hgm_plan_maps", C.c_int, [_P, _P, C.POINTER(C.c_int64)]),

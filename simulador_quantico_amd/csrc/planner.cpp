@@ -1063,9 +1063,18 @@ void schedule_waves(std::vector<RegOp> &ops) {
 // bits on the thread index so that HBM loads and stores stay contiguous
 // across lanes (an empty phase is added when a gate needs them earlier or the
 // schedule ends with them in registers).
+static std::mutex g_program_mu;   // register programs built on demand
+
+Plan compact_plan(const Plan &plan) {
+    std::unique_lock<std::mutex> g(g_program_mu);
+    Plan q = plan;
+    g.unlock();
+    build_exec_program(q, false, true);
+    return q;
+}
+
 void need_register_program(const Plan &plan) {
-    static std::mutex mu;
-    std::lock_guard<std::mutex> g(mu);
+    std::lock_guard<std::mutex> g(g_program_mu);
     if (!plan.has_program) build_register_program(const_cast<Plan &>(plan));
 }
 

@@ -159,7 +159,8 @@ struct RotationMemo {
 // error against 64 bits is 0.2 to 1.03 times that of whole gates (0.81 at 10
 // random layers, 14 qubits, default tuning); in FP64 it would be up to 1.7 times
 // (8.7e-16 -> 1.5e-15 there), for 1.37x the speed at 26 qubits (6.6 -> 4.8 ms).
-void emit(const Item &it, uint32_t S, bool split, uint32_t &flip, C &scale, RotationMemo &memo, std::vector<ROp> &out) {
+// `compact` (build_exec_program) makes at most one record per gate or phase.
+void emit(const Item &it, uint32_t S, bool f32, bool compact, uint32_t &flip, C &scale, RotationMemo &memo, std::vector<ROp> &out) {
     const DevOp &d = *it.d;
     const uint32_t lval = it.lval ^ (flip & it.lmask);
     auto phase = [&](C f, uint32_t lm, uint32_t lv, uint64_t gm, uint64_t gv) {
@@ -191,7 +192,9 @@ void emit(const Item &it, uint32_t S, bool split, uint32_t &flip, C &scale, Rota
         for (int col = 0; col < 2; ++col)
             for (int c = 0; c < 2; ++c) m[4 * row + 2 * col + c] = d.m[4 * (row ^ (int)f) + 2 * (col ^ (int)f) + c];
     const bool free_gate = !it.lmask && !it.gmask;
-    if (it.kind == K_ANTI && free_gate) {   // values exchanged, then a phase on each
+    const bool split = f32 && !compact;
+    const bool unit_anti = it.kind == K_ANTI && is_one(m[2], m[3]) && is_one(m[4], m[5]);
+    if (it.kind == K_ANTI && free_gate && (unit_anti || !compact)) {   // values exchanged, then a phase on each
         flip ^= tb;
         phase(C(m[4], m[5]), tb, 0, 0, 0);
         phase(C(m[2], m[3]), tb, tb, 0, 0);
@@ -219,7 +222,7 @@ void emit(const Item &it, uint32_t S, bool split, uint32_t &flip, C &scale, Rota
     // random layers at 26 qubits, complex128: 6.6 -> 5.5 ms; Grover at 22: 1.36 ->
     // 1.19. A record kind of its own beside the real rotation made the kernels
     // larger: 6 layers at 12 qubits, which run neither, 59 -> 62 us.
-    if (free_gate && !split) {
+    if (free_gate && !f32) {
         const int ex = is_one(m[0], m[1]) && is_one(m[6], m[7]) ? 0 : is_one(m[2], m[3]) && is_one(m[4], m[5]) ? 1 : -1;
         if (ex >= 0 && it.kind != K_ANTI) {
             // rows exchanged (ex): the new row 0 is row 1, the new row 1 is row 0
@@ -237,9 +240,8 @@ void emit(const Item &it, uint32_t S, bool split, uint32_t &flip, C &scale, Rota
     o.gval = it.gval;
     std::copy(m, m + 8, o.m);
     const bool real = m[1] == 0 && m[3] == 0 && m[5] == 0 && m[7] == 0;
-    const bool swap = it.kind == K_ANTI && is_one(m[2], m[3]) && is_one(m[4], m[5]);
     if (o.rmask) o.kind = real ? X_REAL_MASK : X_DENSE_MASK;
-    else if (swap) o.kind = X_SWAP;
+    else if (unit_anti) o.kind = X_SWAP;
     else if (o.tmask) o.kind = real ? X_REAL_LANE : X_DENSE_LANE;
     else o.kind = real ? X_DENSE_REAL : X_DENSE;
     out.push_back(o);
@@ -300,6 +302,7 @@ XOp<T> record(const ROp &o, uint32_t A) {
 template <class T>
 struct Records {
     uint32_t A;
+    bool compact;        // no factor tables
     std::vector<XOp<T>> ops;
     std::vector<T> table;
     C scale = C(1, 0);   // factor of the whole state still to be applied
@@ -336,6 +339,14 @@ struct Records {
     // per register.
     void uniform(It b, It e) {
         if (b == e) return;
+        if (compact) {
+            for (; b != e; ++b) {
+                XOp<T> x = record<T>(**b, A);
+                x.flags = (uint8_t)(X_FIRST | X_LAST | ((*b)->m[1] == 0 ? X_REAL : 0));
+                ops.push_back(x);
+            }
+            return;
+        }
         if (e - b == 1 && scale == C(1, 0)) {
             XOp<T> x = record<T>(**b, A);
             if (x.pat != X_PAT_MASK) {
@@ -517,7 +528,7 @@ void pass_items(const Plan &plan, const Pass &ps, const int *pos, int r, std::ve
 // bit j is state bit pos[j]; gates mix the first r tile bits only, and the
 // first c stay on consecutive threads at the load and the store.
 template <class T>
-void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c, RotationMemo &memo) {
+void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c, bool compact, RotationMemo &memo) {
     constexpr int F = sizeof(T) == 4 ? 5 : 4;
     const ExecShape &ex = plan.exec;
     const int n = plan.qubits;
@@ -573,6 +584,7 @@ void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, in
     };
     Records<T> recs;
     recs.A = (uint32_t)ex.A;
+    recs.compact = compact;
     uint32_t flip = 0;
     for (size_t i = 0; i < sets.size(); ++i) {
         if (i > 0) {
@@ -585,7 +597,7 @@ void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, in
         }
         ops.clear();
         for (int k : lists[i]) {
-            emit(items[k], sets[i], sizeof(T) == 4, flip, recs.scale, memo, ops);
+            emit(items[k], sets[i], sizeof(T) == 4, compact, flip, recs.scale, memo, ops);
             if (ops.size() >= kChunk) { recs.stage(ops); recs.flush(false); ops.clear(); }
         }
         recs.stage(ops);
@@ -666,7 +678,7 @@ bool whole_state(const Plan &plan) {
 
 }  // namespace
 
-void build_exec_program(Plan &plan, bool pass_by_pass) {
+void build_exec_program(Plan &plan, bool pass_by_pass, bool compact) {
     const bool whole = !pass_by_pass && whole_state(plan);
     plan.exec = choose_shape(plan, whole);
     plan.xprog.clear();
@@ -676,8 +688,8 @@ void build_exec_program(Plan &plan, bool pass_by_pass) {
     RotationMemo memo;
     int pos[32];
     auto launch = [&] {
-        if (plan.dtype == HGM_C64) build<float>(plan, items, pos, r, rx, std::min(plan.shape.c, r), memo);
-        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r), memo);
+        if (plan.dtype == HGM_C64) build<float>(plan, items, pos, r, rx, std::min(plan.shape.c, r), compact, memo);
+        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r), compact, memo);
         items.clear();
     };
     for (const Pass &ps : plan.passes) {

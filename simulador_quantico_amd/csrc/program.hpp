@@ -112,7 +112,16 @@ constexpr uint32_t x_swizzle(uint32_t x) {
 
 // Chooses the execution shape (plan.exec) and builds plan.xprog and
 // plan.xlaunch: one launch per non-empty pass, or, unless pass_by_pass, whole
-// runs of passes where the state fits one workgroup.
-void build_exec_program(Plan &plan, bool pass_by_pass);
+// runs of passes where the state fits one workgroup. A compact program has no
+// factor tables and no rotations split off: at most one record per gate, phase
+// and remap, so it is never larger than the plan's register program and its
+// maps. Others may be: every gate on one qubit, 16 amplitudes per thread, takes
+// 256 bytes in FP32 as a rotation and a factor per register, 64 compact, and 104
+// there. Where memory is given (hgm_state_apply_noalloc, the serving budget) a
+// program that does not fit is built compact.
+void build_exec_program(Plan &plan, bool pass_by_pass, bool compact = false);
+
+// A copy of a plan, which others may be using, with compact programs.
+Plan compact_plan(const Plan &plan);
 
 }  // namespace hgm

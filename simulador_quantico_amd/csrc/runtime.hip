@@ -1065,6 +1065,8 @@ int hgm_state_apply_noalloc(hgm_state *s, const hgm_op *ops, int64_t n_ops, cons
                 std::to_string(kNoallocPasses) + " of one call";
         return HGM_E_ARG;
     }
+    if (p->kernel == HGM_KERNEL_REG && plan_table_bytes(*p) > kScratchBytes)
+        p = std::make_shared<const Plan>(compact_plan(*p));
     const size_t need = plan_table_bytes(*p);
     if (need > kScratchBytes) {
         t_err = "hgm_state_apply_noalloc: the plan's tables take " + std::to_string(need) + " bytes, above the " +
@@ -1293,13 +1295,15 @@ int hgm_plan_maps(const hgm_plan *p, void *maps, int64_t *n_maps) {
     return HGM_OK;
 }
 
-int hgm_plan_exec_program(const hgm_plan *p, int32_t *shape, void *program, int64_t *n_bytes, int64_t *launches,
+int hgm_plan_exec_program(const hgm_plan *p, int compact, int32_t *shape, void *program, int64_t *n_bytes, int64_t *launches,
                           int64_t *n_launches) {
     if (!p || !n_bytes || !n_launches || p->plan.kernel != HGM_KERNEL_REG) {
         t_err = "launch programs belong to plans on the interpreted register kernels";
         return HGM_E_ARG;
     }
-    const Plan &q = p->plan;
+    Plan small;
+    if (compact) small = compact_plan(p->plan);
+    const Plan &q = compact ? small : p->plan;
     *n_bytes = (int64_t)(q.xprog.size() * sizeof(uint64_t));
     *n_launches = (int64_t)q.xlaunch.size();
     if (shape) {

@@ -439,11 +439,13 @@ void planner_loop(hgm_server *s) {
                 return r->total_bytes <= s->arena.size() && r->prog_bytes <= s->staging.size();
             };
             // with passes of both kinds the two forms are up to 1.9 times the
-            // register program and its maps; the interpreter's alone is
-            // smaller than those: where both do not fit, it runs every pass
+            // register program and its maps: where both do not fit, the
+            // interpreter runs every pass, on compact programs in the end
             bool ok = fits();
-            if (!ok && !p.xprog.empty()) {
+            for (const bool compact : {false, true}) {
+                if (ok || p.xprog.empty()) break;
                 r->kernel.assign(r->passes.size(), -1);
+                if (compact) build_exec_program(r->plan, true, true);
                 ok = fits();
             }
             if (!ok) {

@@ -388,14 +388,14 @@ class Plan:
         check(lib.hgm_plan_jit_source(self._h, buf, n.value + 1, C.byref(n)))
         return buf.value.decode()
 
-    def exec_program(self):
-        """What the interpreted register kernels run: (tile bits, amplitudes per thread, threads, barriers), the
+    def exec_program(self, compact: bool = False):
+        """What the interpreted register kernels run (compact: where the usual form does not fit): (tile bits, amplitudes per thread, threads, barriers), the
         programs' bytes, and per launch the byte offset of its program and its number of stages."""
         shape = (C.c_int32 * 4)()
         nb, nl = C.c_int64(), C.c_int64()
-        check(lib.hgm_plan_exec_program(self._h, shape, None, C.byref(nb), None, C.byref(nl)))
+        check(lib.hgm_plan_exec_program(self._h, int(compact), shape, None, C.byref(nb), None, C.byref(nl)))
         prog, at = np.zeros(nb.value, np.uint8), np.zeros((nl.value, 2), np.int64)
-        check(lib.hgm_plan_exec_program(self._h, shape, prog.ctypes.data, C.byref(nb), at.ctypes.data, C.byref(nl)))
+        check(lib.hgm_plan_exec_program(self._h, int(compact), shape, prog.ctypes.data, C.byref(nb), at.ctypes.data, C.byref(nl)))
         return tuple(shape), prog, at
 
     def program(self, i: int):

@@ -68,8 +68,8 @@ def _selected(o, A):
     return (k & pat) == pat
 
 
-def emulate(plan, n, psi, dtype):
-    (r, A, B, sync), prog, launches = plan.exec_program()
+def emulate(plan, n, psi, dtype, compact=False):
+    (r, A, B, sync), prog, launches = plan.exec_program(compact)
     a_bits, fold = A.bit_length() - 1, 5 if dtype == np.complex64 else 4
     k, t = np.arange(A), np.arange(B, dtype=np.uint64)
     psi = psi.astype(np.complex128).copy()
@@ -269,3 +269,51 @@ def test_conditional_phases_are_not_rounded(dtype):
     single = {v[0] for v in single.values() if len(v) == 1}
     found = {complex(*_phase_factor(o)) for at, _ in launches for o in _records(prog, int(at), dtype)[1] if int(o["kind"]) == X_PHASE}
     assert single and single <= found
+
+
+def _register_bytes(plan):
+    """The register program, its maps and its pass tables."""
+    rops = sum(len(plan.program(i)[0]) for i in range(len(plan)))
+    return 104 * rops + 256 * len(plan.maps()) + 2056 * len(plan)
+
+
+def _u3(r):
+    z, _ = np.linalg.qr(r.normal(size=(2, 2)) + 1j * r.normal(size=(2, 2)))
+    return z.reshape(4)
+
+
+def _families(n, r):
+    """Gate lists whose usual programs are large: little that merges, much that needs a factor per register."""
+    k = 300
+    one = [int(n // 2)] * k
+    yield "one qubit", (one, [0] * k, [0] * k, [_u3(r) for _ in range(k)])
+    rz = [np.array([np.exp(-1j * x), 0, 0, np.exp(1j * x)]) for x in r.uniform(0, 3, k)]
+    yield "turns", (one, [0] * k, [0] * k, [rz[i] if i % 2 else _u3(r) for i in range(k)])
+    other = 1 << (n // 2 + 1)
+    yield "controls", (one, [0 if i % 2 else other for i in range(k)], [0 if i % 2 else other * (i // 2 % 2) for i in range(k)],
+                       [_u3(r) if i % 2 else rz[i] for i in range(k)])
+    anti = [np.array([0, np.exp(1j * x), np.exp(-1j * x), 0]) for x in r.uniform(0, 3, k)]
+    yield "exchanges", (one, [0] * k, [0] * k, anti)
+    yield "any", _random_gate_list(r, n, k)
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n", [4, 9, 13])
+def test_compact_programs_take_no_more_than_the_register_program(n, dtype):
+    r = np.random.default_rng(n)
+    larger = 0
+    for name, (t, cm, cv, mats) in _families(n, r):
+        for amps in (2, 4, 16):
+            for ops_block in (1, 40, 1 << 30):
+                bits = min(n, 11) if n > 4 else 4
+                tuning = N.default_tuning(block_size=max(1, (1 << bits) // amps), repeat_count=amps // 2, gpu_region_bits=bits,
+                                          gpu_coalesced_bits=min(3, bits - 1), kernel=N.HGM_KERNEL_REG, ops_block=ops_block)
+                plan = hq.Plan(n, hq.make_ops(t, cm, cv, mats), tuning, 1, dtype)
+                limit = _register_bytes(plan)
+                assert len(plan.exec_program(True)[1]) <= limit, (name, amps, ops_block)
+                larger += len(plan.exec_program()[1]) > limit
+        psi = r.standard_normal(1 << n) + 1j * r.standard_normal(1 << n)
+        psi /= np.linalg.norm(psi)
+        off = np.linalg.norm(emulate(plan, n, psi, dtype, True) - oracle_run_gates(n, t, cm, cv, mats, state=psi))
+        assert off <= 16 * np.finfo(dtype).eps * len(t), (name, off)
+    assert larger   # what the compact form is for
