@@ -4,16 +4,24 @@
 #include <algorithm>
 #include <complex>
 #include <cstring>
+#include <type_traits>
 
 namespace hgm {
 
 namespace {
 
-// Factors are multiplied together in extended precision and rounded once, to
-// the amplitude type: a rotation's phases and coefficients are then as exact
-// as the entries of its gate.
-using R = long double;
-using C = std::complex<R>;
+// Factors are multiplied together in a wider type and rounded once, to the
+// amplitude type: a rotation's phases and coefficients are then as exact as
+// the entries of its gate. For FP32 that is double, which leaves 2^-40 of an
+// FP32 rounding (extended precision: 10 random layers at 12 qubits planned in
+// 0.15 ms, in double in 0.066), for FP64 extended precision.
+template <class T> using Wide = std::conditional_t<sizeof(T) == 4, double, long double>;
+
+// Products of factors, none of which is infinite.
+template <class R>
+std::complex<R> mul(const std::complex<R> &a, const std::complex<R> &b) {
+    return {a.real() * b.real() - a.imag() * b.imag(), a.real() * b.imag() + a.imag() * b.real()};
+}
 
 int popc(uint64_t v) { return __builtin_popcountll(v); }
 
@@ -29,6 +37,7 @@ struct Item {
 };
 
 // A physical operation on registers (coordinates of one stage).
+template <class R>
 struct ROp {
     bool phase;
     XKind kind;
@@ -39,7 +48,8 @@ struct ROp {
     int slot = 0;          // wave: phases even, gates odd
 };
 
-void split_cond(uint32_t mask, uint32_t val, uint32_t S, ROp &o) {
+template <class R>
+void split_cond(uint32_t mask, uint32_t val, uint32_t S, ROp<R> &o) {
     for (; mask; mask &= mask - 1) {
         const int b = __builtin_ctz(mask);
         const uint32_t v = (val >> b) & 1, below = (1u << b) - 1;
@@ -55,41 +65,43 @@ void split_cond(uint32_t mask, uint32_t val, uint32_t S, ROp &o) {
     }
 }
 
-bool is_one(R re, R im) { return re == 1.0 && im == 0.0; }
+bool is_one(double re, double im) { return re == 1.0 && im == 0.0; }
 
 // Largest entry beside the 1 of a rotation's row: 1 for a unitary gate, up to
 // the rounding of its entries.
-constexpr R kMaxTurn = 1.0L + 1e-6L;
+constexpr double kMaxTurn = 1.0 + 1e-6;
 
 // Phases x0, x1, y of modulus 1 with v[i][j] = x_i * o[i][j] * y_j (y_0 = 1)
 // and every o[i][j] real; false when there are none up to the rounding of v's
 // entries to double (16 units in the last place). Nonzero entries link rows to
 // columns: with column 0's phase 1 the links give the others, and the fourth
 // entry is the check. Every unitary matrix has them.
-bool real_middle(const C v[2][2], C x[2], C *y, R o[2][2]) {
+template <class R>
+bool real_middle(const std::complex<R> v[2][2], std::complex<R> x[2], std::complex<R> *y, R o[2][2]) {
+    using C = std::complex<R>;
     C row[2] = {C(1, 0), C(1, 0)}, col[2] = {C(1, 0), C(1, 0)};
     bool have_r[2] = {false, false}, have_c[2] = {true, false};
     for (int pass = 0; pass < 3; ++pass)
         for (int i = 0; i < 2; ++i)
             for (int j = 0; j < 2; ++j) {
-                if (v[i][j] == C(0, 0)) continue;
+                if (have_c[j] == have_r[i] || v[i][j] == C(0, 0)) continue;
                 const C u = v[i][j] / std::sqrt(std::norm(v[i][j]));
-                if (have_c[j] && !have_r[i]) { row[i] = u * std::conj(col[j]); have_r[i] = true; }
-                else if (have_r[i] && !have_c[j]) { col[j] = u * std::conj(row[i]); have_c[j] = true; }
+                if (have_c[j]) { row[i] = mul(u, std::conj(col[j])); have_r[i] = true; }
+                else { col[j] = mul(u, std::conj(row[i])); have_c[j] = true; }
             }
-    const C closing = v[1][1] * std::conj(row[1] * col[1]);
-    if (std::abs(closing.imag()) > 16 * 0x1p-52L * std::sqrt(std::norm(closing))) return false;
+    const C closing = mul(v[1][1], std::conj(mul(row[1], col[1])));
+    if (std::abs(closing.imag()) > R(16 * 0x1p-52) * std::sqrt(std::norm(closing))) return false;
     if (v[0][0] != C(0, 0) && v[0][1] != C(0, 0) && v[1][0] != C(0, 0) && v[1][1] != C(0, 0)) {
         // what the fourth phase misses by is the entries' own rounding: a quarter to each
         const R miss = closing.imag() / closing.real();   // below 2^-47: e^(i miss) = 1 + i miss
         if (miss != 0) {
-            row[0] *= C(1, -miss / 4);
-            row[1] *= C(1, miss / 4);
-            col[1] *= C(1, miss / 2);
+            row[0] = mul(row[0], C(1, -miss / 4));
+            row[1] = mul(row[1], C(1, miss / 4));
+            col[1] = mul(col[1], C(1, miss / 2));
         }
     }
     for (int i = 0; i < 2; ++i)
-        for (int j = 0; j < 2; ++j) o[i][j] = (v[i][j] * std::conj(row[i] * col[j])).real();
+        for (int j = 0; j < 2; ++j) o[i][j] = mul(v[i][j], std::conj(mul(row[i], col[j]))).real();
     x[0] = row[0];
     x[1] = row[1];
     *y = col[1];
@@ -98,14 +110,17 @@ bool real_middle(const C v[2][2], C x[2], C *y, R o[2][2]) {
 
 // U = e0 * diag(1, e1) * M * diag(1, y) with M = [[1, t0], [t1, 1]] and, where
 // the off-diagonal entries are the larger, the rows of U exchanged.
+template <class R>
 struct Rotation {
     bool ok = false, exchanged = false;
     R t0 = 0, t1 = 0;
-    C e0, e1, y;
+    std::complex<R> e0, e1, y;
 };
 
-Rotation split_rotation(const double m[8]) {
-    Rotation t;
+template <class R>
+Rotation<R> split_rotation(const double m[8]) {
+    using C = std::complex<R>;
+    Rotation<R> t;
     const C v[2][2] = {{C(m[0], m[1]), C(m[2], m[3])}, {C(m[4], m[5]), C(m[6], m[7])}};
     C x[2];
     R w[2][2];
@@ -118,22 +133,23 @@ Rotation split_rotation(const double m[8]) {
     if (!(std::abs(t.t0) <= kMaxTurn && std::abs(t.t1) <= kMaxTurn)) return t;
     t.exchanged = ex != 0;
     t.e0 = x[ex] * d0;
-    t.e1 = x[1 - ex] * d1 / t.e0;
+    t.e1 = mul(x[1 - ex], std::conj(x[ex])) * (d1 / (d0 * std::norm(x[ex])));
     t.ok = true;
     return t;
 }
 
 // The rotations of the gates seen last: circuits repeat their gates, and a
 // split takes longer than the rest of a gate's record.
+template <class R>
 struct RotationMemo {
     static constexpr int kEntries = 16;
     struct Entry {
         double m[8];
-        Rotation t;
+        Rotation<R> t;
         bool used = false;
     } entry[kEntries];
 
-    const Rotation &of(const double m[8]) {
+    const Rotation<R> &of(const double m[8]) {
         uint64_t h = 0;
         for (int i = 0; i < 8; ++i) {
             uint64_t b;
@@ -143,7 +159,7 @@ struct RotationMemo {
         Entry &e = entry[h >> 60];
         if (!e.used || std::memcmp(e.m, m, sizeof e.m)) {
             std::memcpy(e.m, m, sizeof e.m);
-            e.t = split_rotation(m);
+            e.t = split_rotation<R>(m);
             e.used = true;
         }
         return e.t;
@@ -160,12 +176,15 @@ struct RotationMemo {
 // random layers, 14 qubits, default tuning); in FP64 it would be up to 1.7 times
 // (8.7e-16 -> 1.5e-15 there), for 1.37x the speed at 26 qubits (6.6 -> 4.8 ms).
 // `compact` (build_exec_program) makes at most one record per gate or phase.
-void emit(const Item &it, uint32_t S, bool f32, bool compact, uint32_t &flip, C &scale, RotationMemo &memo, std::vector<ROp> &out) {
+template <class R>
+void emit(const Item &it, uint32_t S, bool f32, bool compact, uint32_t &flip, std::complex<R> &scale, RotationMemo<R> &memo,
+          std::vector<ROp<R>> &out) {
+    using C = std::complex<R>;
     const DevOp &d = *it.d;
     const uint32_t lval = it.lval ^ (flip & it.lmask);
     auto phase = [&](C f, uint32_t lm, uint32_t lv, uint64_t gm, uint64_t gv) {
         if (f == C(1, 0)) return;
-        ROp o;
+        ROp<R> o;
         o.phase = true;
         o.kind = X_PHASE;
         split_cond(lm, lv, S, o);
@@ -200,11 +219,11 @@ void emit(const Item &it, uint32_t S, bool f32, bool compact, uint32_t &flip, C 
         phase(C(m[2], m[3]), tb, tb, 0, 0);
         return;
     }
-    ROp o;
+    ROp<R> o;
     o.phase = false;
     o.bit = popc(S & (tb - 1));
     if (free_gate && split) {
-        const Rotation &t = memo.of(m);
+        const Rotation<R> &t = memo.of(m);
         if (t.ok) {
             phase(t.y, tb, tb, 0, 0);
             if (t.exchanged) flip ^= tb;
@@ -212,7 +231,7 @@ void emit(const Item &it, uint32_t S, bool f32, bool compact, uint32_t &flip, C 
             o.m[0] = t.t0;
             o.m[2] = t.t1;
             out.push_back(o);
-            scale *= t.e0;
+            scale = mul(scale, t.e0);
             phase(t.e1, tb, tb, 0, 0);
             return;
         }
@@ -257,10 +276,11 @@ void sort_stable(I b, I e, F less) {
 // Orders a stage's operations into waves (phases as early as they commute,
 // then gates), keeping the order of every pair that does not commute: gates
 // on a register bit conflict with gates on it and with whatever tests it.
-void into_waves(std::vector<ROp> &ops, std::vector<const ROp *> &order) {
+template <class R>
+void into_waves(std::vector<ROp<R>> &ops, std::vector<const ROp<R> *> &order) {
     int gate[8] = {0}, test[8] = {0};
     order.clear();
-    for (ROp &o : ops) {
+    for (ROp<R> &o : ops) {
         int s = 0;
         for (uint32_t m = o.rmask; m; m &= m - 1) s = std::max(s, gate[__builtin_ctz(m)]);
         if (!o.phase) s = std::max({s, gate[o.bit], test[o.bit]});
@@ -270,11 +290,11 @@ void into_waves(std::vector<ROp> &ops, std::vector<const ROp *> &order) {
         if (!o.phase) gate[o.bit] = std::max(gate[o.bit], s);
         order.push_back(&o);
     }
-    sort_stable(order.begin(), order.end(), [](const ROp *a, const ROp *b) { return a->slot < b->slot; });
+    sort_stable(order.begin(), order.end(), [](const ROp<R> *a, const ROp<R> *b) { return a->slot < b->slot; });
 }
 
 template <class T>
-XOp<T> record(const ROp &o, uint32_t A) {
+XOp<T> record(const ROp<Wide<T>> &o, uint32_t A) {
     XOp<T> x;
     std::memset(&x, 0, sizeof x);
     x.kind = (uint8_t)o.kind;
@@ -301,6 +321,9 @@ XOp<T> record(const ROp &o, uint32_t A) {
 // Records of one pass, and the factors of its X_VEC records.
 template <class T>
 struct Records {
+    using C = std::complex<Wide<T>>;
+    using ROp = struct ROp<Wide<T>>;
+
     uint32_t A;
     bool compact;        // no factor tables
     std::vector<XOp<T>> ops;
@@ -315,7 +338,7 @@ struct Records {
     void vec() {
         bool real = true, one = true;
         for (uint32_t k = 0; k < A; ++k) {
-            if (scale != C(1, 0)) f[k] *= scale;
+            if (scale != C(1, 0)) f[k] = mul(f[k], scale);
             real = real && (T)f[k].imag() == T(0);
             one = one && f[k] == C(1, 0);
         }
@@ -332,7 +355,7 @@ struct Records {
         ops.push_back(x);
     }
 
-    using It = std::vector<const ROp *>::const_iterator;
+    using It = typename std::vector<const ROp *>::const_iterator;
 
     // The phases [b, e) of a wave that test register bits only: one record when
     // a pattern of set (or one clear) register bits says it, else one factor
@@ -361,7 +384,7 @@ struct Records {
             for (uint32_t k = 0; k < A; ++k) {
                 if ((k & o.rmask) != o.rval) continue;
                 if (o.m[1] == 0) f[k] *= o.m[0];
-                else f[k] *= C(o.m[0], o.m[1]);
+                else f[k] = mul(f[k], C(o.m[0], o.m[1]));
             }
         }
         vec();
@@ -379,7 +402,7 @@ struct Records {
                     return g.tmask == o.tmask && g.tval == o.tval && g.gmask == o.gmask && g.gval == o.gval;
                 });
                 if (same == group.end()) { group.push_back(o); continue; }
-                const C z = C(same->m[0], same->m[1]) * C(o.m[0], o.m[1]);
+                const C z = mul(C(same->m[0], same->m[1]), C(o.m[0], o.m[1]));
                 same->m[0] = z.real();
                 same->m[1] = z.imag();
             }
@@ -461,8 +484,8 @@ struct Records {
     // The pending scale, when it is due: at the end of the pass, and before it
     // moves the amplitudes far from 1.
     void flush(bool end) {
-        const R s = std::abs(scale);
-        if (scale == C(1, 0) || (!end && s >= 0x1p-20L && s <= 0x1p20L)) return;
+        const auto s = std::norm(scale);
+        if (scale == C(1, 0) || (!end && s >= 0x1p-40 && s <= 0x1p40)) return;
         std::fill(f, f + A, C(1, 0));
         vec();
     }
@@ -493,6 +516,7 @@ void pass_items(const Plan &plan, const Pass &ps, const int *pos, int r, std::ve
     int tile_of[64];
     std::fill(tile_of, tile_of + 64, -1);
     for (int j = 0; j < r; ++j) tile_of[pos[j]] = j;
+    items.reserve(items.size() + (size_t)ps.op_count);
     for (int64_t i = 0; i < ps.op_count; ++i) {
         const DevOp &d = plan.ops[ps.op_begin + i];
         Item it{&d, d.kind, d.tbit, 0, 0, 0, 0, 0, 0, 0};
@@ -528,7 +552,7 @@ void pass_items(const Plan &plan, const Pass &ps, const int *pos, int r, std::ve
 // bit j is state bit pos[j]; gates mix the first r tile bits only, and the
 // first c stay on consecutive threads at the load and the store.
 template <class T>
-void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c, bool compact, RotationMemo &memo) {
+void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, int rx, int c, bool compact, RotationMemo<Wide<T>> &memo) {
     constexpr int F = sizeof(T) == 4 ? 5 : 4;
     const ExecShape &ex = plan.exec;
     const int n = plan.qubits;
@@ -538,7 +562,8 @@ void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, in
     const uint32_t forbid = (r - c >= a) ? (uint32_t)((1u << c) - 1) : 0u;
     uint64_t local = 0;
     for (int j = 0; j < rx; ++j) local |= uint64_t(1) << pos[j];
-    std::vector<ROp> ops;
+    std::vector<ROp<Wide<T>>> ops;
+    ops.reserve(kChunk + 4);
     // stages: the same greedy as the pass planner, with the tile as the state and the register bits as the
     // tile; the first and last keep the coalesced bits on the threads
     std::vector<uint32_t> sets;
@@ -585,6 +610,7 @@ void build(Plan &plan, const std::vector<Item> &items, const int *pos, int r, in
     Records<T> recs;
     recs.A = (uint32_t)ex.A;
     recs.compact = compact;
+    recs.ops.reserve(items.size() + items.size() / 2 + 16);
     uint32_t flip = 0;
     for (size_t i = 0; i < sets.size(); ++i) {
         if (i > 0) {
@@ -685,11 +711,12 @@ void build_exec_program(Plan &plan, bool pass_by_pass, bool compact) {
     plan.xlaunch.clear();
     const int n = plan.qubits, r = whole ? n : plan.shape.r, rx = plan.exec.r;
     std::vector<Item> items;
-    RotationMemo memo;
+    RotationMemo<double> memo;
+    RotationMemo<long double> unused;   // FP64 programs hold whole gates
     int pos[32];
     auto launch = [&] {
         if (plan.dtype == HGM_C64) build<float>(plan, items, pos, r, rx, std::min(plan.shape.c, r), compact, memo);
-        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r), compact, memo);
+        else build<double>(plan, items, pos, r, rx, std::min(plan.shape.c, r), compact, unused);
         items.clear();
     };
     for (const Pass &ps : plan.passes) {
