@@ -1,13 +1,6 @@
-// gfx950 kernels of the t_GPU path.
-//
-// k_pass_lds: one workgroup per tile of 2^r amplitudes. The tile's local index
-// L maps to the state index base | (L & cmask) | deposit(L >> c), where the
-// low c bits stay contiguous (so a wave's loads cover runs of 2^c amplitudes)
-// and deposit() scatters the remaining r-c tile bits onto the pass's chosen
-// state-index bits through three 64-entry LDS tables. Thread t owns local
-// indices t + k*B (k < 2R) for loading, storing and diagonal gates; for a
-// pair-mixing gate it takes pairs t + k*B (k < R) and inserts a zero at the
-// target's tile bit. Barriers are placed only where ownership changes.
+// gfx950 kernels of the t_GPU path: the interpreted register kernels, state
+// set-up and copies, and readout.
+#include "device.hpp"
 #include "kernels.hpp"
 #include "program.hpp"
 
@@ -16,10 +9,6 @@
 namespace hgm {
 
 namespace {
-
-template <class T> struct Vec;
-template <> struct Vec<double> { using type = double2; };
-template <> struct Vec<float> { using type = float2; };
 
 // State accesses of a single-circuit pass, which reads and writes every
 // amplitude once per pass: nontemporal (streaming) hint (interpreted random30
@@ -37,122 +26,6 @@ __device__ __forceinline__ void store_stream(typename Vec<T>::type *p, const typ
     typedef T N __attribute__((ext_vector_type(2)));
     const N v = {a.x, a.y};
     __builtin_nontemporal_store(v, reinterpret_cast<N *>(p));
-}
-
-__device__ __forceinline__ uint64_t pdep64(uint64_t v, uint64_t mask) {
-    uint64_t r = 0;
-    for (uint64_t bb = 1; mask; bb <<= 1) {
-        uint64_t lowbit = mask & (~mask + 1);
-        if (v & bb) r |= lowbit;
-        mask &= mask - 1;
-    }
-    return r;
-}
-
-template <class V, class T>
-__device__ __forceinline__ V cmul(T mr, T mi, V a) {
-    V o;
-    o.x = mr * a.x - mi * a.y;
-    o.y = mr * a.y + mi * a.x;
-    return o;
-}
-
-template <class V, class T>
-__device__ __forceinline__ V cmul2(T ar, T ai, V x, T br, T bi, V y) {
-    V o;
-    o.x = ar * x.x - ai * x.y + br * y.x - bi * y.y;
-    o.y = ar * x.y + ai * x.x + br * y.y + bi * y.x;
-    return o;
-}
-
-template <class T>
-__global__ void __launch_bounds__(1024) k_pass_lds(typename Vec<T>::type *__restrict__ state,
-                                                   const DevOp *__restrict__ ops, int n_ops, PassArgs a) {
-    using V = typename Vec<T>::type;
-    extern __shared__ __align__(16) unsigned char smem[];
-    uint64_t *dep = reinterpret_cast<uint64_t *>(smem);      // 3 tables of 64 entries
-    V *tile = reinterpret_cast<V *>(smem + 3 * 64 * sizeof(uint64_t));
-
-    const int t = threadIdx.x;
-    const int hi_bits = a.r - a.c;
-    for (int x = t; x < 192; x += blockDim.x) {
-        const int tab = x >> 6, v = x & 63;
-        uint64_t acc = 0;
-        for (int j = 0; j < 6; ++j) {
-            const int lb = tab * 6 + j;
-            if (((v >> j) & 1) && lb < hi_bits) acc |= uint64_t(1) << a.local_pos[a.c + lb];
-        }
-        dep[x] = acc;
-    }
-    __syncthreads();
-
-    const int B = a.B, R = a.R, c = a.c;
-    const uint32_t cmask = (1u << c) - 1u;
-    for (int64_t tid = blockIdx.x; tid < a.n_tiles; tid += gridDim.x) {
-        const uint64_t base = pdep64((uint64_t)tid, a.nonlocal_mask);
-        // load
-        for (int k = 0; k < 2 * R; ++k) {
-            const uint32_t L = (uint32_t)(t + k * B);
-            const uint32_t h = L >> c;
-            const uint64_t g = base | (L & cmask) | dep[h & 63] | dep[64 + ((h >> 6) & 63)] | dep[128 + ((h >> 12) & 63)];
-            tile[L] = state[g];
-        }
-        bool last_pair = false;
-        for (int i = 0; i < n_ops; ++i) {
-            const DevOp &o = ops[i];
-            if ((base & o.gmask) != o.gval) continue;   // tile-uniform
-            const T m0r = (T)o.m[0], m0i = (T)o.m[1], m1r = (T)o.m[2], m1i = (T)o.m[3];
-            const T m2r = (T)o.m[4], m2i = (T)o.m[5], m3r = (T)o.m[6], m3i = (T)o.m[7];
-            if (o.kind == K_DENSE || o.kind == K_ANTI) {
-                __syncthreads();
-                const int tb = o.tbit;
-                const uint32_t tmask = 1u << tb;
-                for (int k = 0; k < R; ++k) {
-                    const uint32_t p = (uint32_t)(t + k * B);
-                    const uint32_t p0 = ((p >> tb) << (tb + 1)) | (p & (tmask - 1u));
-                    const uint32_t p1 = p0 | tmask;
-                    if ((p0 & o.lmask) != o.lval) continue;
-                    const V x = tile[p0], y = tile[p1];
-                    if (o.kind == K_DENSE) {
-                        tile[p0] = cmul2<V, T>(m0r, m0i, x, m1r, m1i, y);
-                        tile[p1] = cmul2<V, T>(m2r, m2i, x, m3r, m3i, y);
-                    } else {
-                        tile[p0] = cmul<V, T>(m1r, m1i, y);
-                        tile[p1] = cmul<V, T>(m2r, m2i, x);
-                    }
-                }
-                last_pair = true;
-            } else {
-                if (last_pair) { __syncthreads(); last_pair = false; }
-                if (o.kind == K_DIAG) {
-                    const int tb = o.tbit;
-                    for (int k = 0; k < 2 * R; ++k) {
-                        const uint32_t L = (uint32_t)(t + k * B);
-                        if ((L & o.lmask) != o.lval) continue;
-                        const bool one = (L >> tb) & 1u;
-                        tile[L] = one ? cmul<V, T>(m3r, m3i, tile[L]) : cmul<V, T>(m0r, m0i, tile[L]);
-                    }
-                } else {   // K_DIAG_GLOBAL
-                    const bool one = (base >> o.tbit) & 1u;
-                    const T pr = one ? m3r : m0r, pi = one ? m3i : m0i;
-                    for (int k = 0; k < 2 * R; ++k) {
-                        const uint32_t L = (uint32_t)(t + k * B);
-                        if ((L & o.lmask) != o.lval) continue;
-                        tile[L] = cmul<V, T>(pr, pi, tile[L]);
-                    }
-                }
-            }
-        }
-        if (last_pair) __syncthreads();
-        // store
-        for (int k = 0; k < 2 * R; ++k) {
-            const uint32_t L = (uint32_t)(t + k * B);
-            const uint32_t h = L >> c;
-            const uint64_t g = base | (L & cmask) | dep[h & 63] | dep[64 + ((h >> 6) & 63)] | dep[128 + ((h >> 12) & 63)];
-            state[g] = tile[L];
-        }
-        __syncthreads();   // the next tile reuses the LDS
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -724,8 +597,6 @@ __global__ void k_collapse(typename Vec<T>::type *state, uint64_t half, int bit,
     }
 }
 
-uint64_t max_blocks(int block) { return 0xffffffffull / (uint64_t)block; }
-
 int grid_for(uint64_t n, int block) {
     uint64_t g = (n + block - 1) / block;
     if (g > (uint64_t(1) << 24)) g = uint64_t(1) << 24;
@@ -734,20 +605,8 @@ int grid_for(uint64_t n, int block) {
     return (int)g;
 }
 
-int64_t tile_grid(int64_t n_tiles, int block) {
-    int64_t g = n_tiles < (int64_t(1) << 22) ? n_tiles : (int64_t(1) << 22);
-    if ((uint64_t)g > max_blocks(block)) g = (int64_t)max_blocks(block);
-    return g;
-}
-
 // The per-pass kernels' dynamic LDS limit, raised once per kernel (before the
 // first launch, and before any stream capture that launches it).
-template <class T>
-hipError_t pass_lds_attr() {
-    static const hipError_t e =
-        hipFuncSetAttribute((const void *)k_pass_lds<T>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    return e;
-}
 template <class T, int A>
 hipError_t pass_reg_attr() {
     static const hipError_t e =
@@ -756,20 +615,10 @@ hipError_t pass_reg_attr() {
 }
 template <class T>
 hipError_t pass_attrs() {
-    for (hipError_t e : {pass_lds_attr<T>(), pass_reg_attr<T, 2>(), pass_reg_attr<T, 4>(), pass_reg_attr<T, 8>(),
+    for (hipError_t e : {pass_reg_attr<T, 2>(), pass_reg_attr<T, 4>(), pass_reg_attr<T, 8>(),
                          pass_reg_attr<T, 16>(), pass_reg_attr<T, 32>()})
         if (e != hipSuccess) return e;
     return hipSuccess;
-}
-
-template <class T>
-hipError_t pass_lds(void *state, const DevOp *ops, int n_ops, const PassArgs &a, hipStream_t s) {
-    pass_lds_attr<T>();
-    const size_t lds = 3 * 64 * sizeof(uint64_t) + (size_t(1) << a.r) * sizeof(typename Vec<T>::type);
-    const int64_t grid = tile_grid(a.n_tiles, a.B);
-    hipLaunchKernelGGL(k_pass_lds<T>, dim3((unsigned)grid), dim3(a.B), lds, s,
-                       reinterpret_cast<typename Vec<T>::type *>(state), ops, n_ops, a);
-    return hipGetLastError();
 }
 
 template <class T, int A>
@@ -834,11 +683,10 @@ hipError_t launch_pass_reg(int dtype, int qubits, const ExecShape &e, const Stat
                             : pass_reg_any<double>(e.A, state, xp, xp_bytes, n_tiles, e.B, lds_bytes, mode, s);
 }
 
-hipError_t launch_pass_lds(int dtype, void *state, const DevOp *ops, int n_ops, const PassArgs &a, hipStream_t s) {
-    return dtype == HGM_C64 ? pass_lds<float>(state, ops, n_ops, a, s) : pass_lds<double>(state, ops, n_ops, a, s);
+hipError_t prepare_pass_kernels(int dtype) {
+    const hipError_t e = prepare_pass_lds(dtype);
+    return e != hipSuccess ? e : dtype == HGM_C64 ? pass_attrs<float>() : pass_attrs<double>();
 }
-
-hipError_t prepare_pass_kernels(int dtype) { return dtype == HGM_C64 ? pass_attrs<float>() : pass_attrs<double>(); }
 
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t s) {
     // one 16-byte element per thread over the whole buffer: a flat grid keeps

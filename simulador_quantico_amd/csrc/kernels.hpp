@@ -26,6 +26,7 @@ hipError_t launch_pass_lds(int dtype, void *state, const DevOp *ops, int n_ops, 
 // dtype (otherwise done on their first launch): call before capturing their
 // launches into a graph.
 hipError_t prepare_pass_kernels(int dtype);
+hipError_t prepare_pass_lds(int dtype);   // of the LDS kernel alone
 
 // The states of one launch: `count` of one size and type, at byte offsets
 // offs[i] (device memory) from `first`; offs null: the one state.
