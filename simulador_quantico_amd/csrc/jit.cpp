@@ -89,7 +89,7 @@ std::string thread_or(const uint64_t *contrib, int nbits) {
     return s.empty() ? "0ull" : s;
 }
 
-// The interpreter's phase maps hold XOR-swizzled tile indices; the swizzle is
+// The register program's phase maps hold XOR-swizzled tile indices; the swizzle is
 // its own inverse.
 uint32_t unswizzle(uint32_t x) { return x ^ ((x >> 4) & 15u) ^ ((x >> 8) & 15u) ^ ((x >> 12) & 15u); }
 

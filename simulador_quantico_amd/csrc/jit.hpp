@@ -43,7 +43,7 @@ size_t jit_compiled_count();
 // is a function of its structure only: op kinds, register bits, condition
 // masks, pivot columns, phase maps and load/store tables, the qubit count and
 // tile shape. Matrix entries and control values are read at run time from
-// the item's register program (as the interpreter reads them), so requests
+// the item's register program (RegOp), so requests
 // whose passes have equal keys share one kernel. The kernel takes the batched
 // interpreter's arguments (items, n_items, programs, states, partials) and
 // also reduces the readout of an item that asks for it.

@@ -1,4 +1,4 @@
-// Launch wrappers of the gfx950 kernels (defined in kernels.hip).
+// Launch wrappers of the gfx950 kernels (defined in kernels.hip and lds_kernel.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>

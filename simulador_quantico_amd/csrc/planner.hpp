@@ -87,7 +87,7 @@ struct Pass {
 };
 
 // ---- register kernel program --------------------------------------------
-// In the register kernel each thread holds A = 2R amplitudes of its tile in
+// In the plan-compiled and serving kernels each thread holds A = 2R amplitudes of its tile in
 // registers. A "phase" assigns log2(A) tile bits to the register index and the
 // other tile bits, in ascending order, to the thread index. Gates are applied
 // to registers only; a remap moves the tile through LDS into the next phase's
@@ -127,7 +127,7 @@ struct PhaseMap {
     uint16_t reg[64];
     uint16_t thr[2][32];
 };
-static_assert(sizeof(PhaseMap) == 256, "PhaseMap layout is shared with the kernels");
+static_assert(sizeof(PhaseMap) == 256, "PhaseMap layout is shared with hgm_plan_maps");
 
 // State-index offsets of the load (first phase) and store (last phase)
 // assignments: element (t, k) of tile `base` lives at
@@ -140,7 +140,7 @@ struct PassMem {
     int32_t first_map;
     int32_t last_map;
 };
-static_assert(sizeof(PassMem) == 2056, "PassMem layout is shared with the kernels");
+static_assert(sizeof(PassMem) == 2056, "PassMem layout is part of the generated kernels' keys");
 
 // How the interpreted kernels run a plan's tiles: workgroups of B threads with
 // A amplitudes each take tiles of 2^r amplitudes, the plan's own tile plus
@@ -212,7 +212,12 @@ size_t amp_bytes(int dtype);
 // Up to 8 MiB plain loads hit the L2s (16 qubits 305 -> 273 us); at 8 MiB the
 // stores keep the hint (20 qubits FP32: 572 us; stores plain too 607; both
 // with the hint 587), below it makes no difference to one state, and a batch
-// of small states as a whole lives in the last-level cache.
+// of small states as a whole lives in the last-level cache. The interpreted
+// kernels, which did with the hint at every size before, follow: 64-256 MiB
+// Grover 5-24% faster without it (24 qubits FP64, 2^12 tiles 2593 -> 2092 us;
+// FP32 1445 -> 1172), random layers 0-7%; 512 MiB FP64 Grover 11409 with it
+// against 12773 us; up to 16 MiB within 2% either way. At 32 MiB FP32 Grover
+// would take 386 us plain against 425, FP64 264 against 257: left as it is.
 void state_streams(size_t bytes, bool *loads, bool *stores);
 
 // Validates a tuning tuple (the reference's rules of src/core/dgm_core.cpp:177-241

@@ -132,7 +132,7 @@ struct Req {
     int lane = 0;
     int64_t n_tiles = 1;
     size_t state_bytes = 0, rop_bytes = 0, prog_bytes = 0, part_bytes = 0, total_bytes = 0, off = 0, stage_off = 0;
-    char *d = nullptr;             // device block: state | programs | maps | pass tables | partials
+    char *d = nullptr;             // device block: state | register programs | interpreted programs | partials
     ReadoutPartial result{};
 };
 
@@ -389,7 +389,7 @@ void planner_loop(hgm_server *s) {
             lt = s->large[r->qubits];
         }
         std::string err;
-    int rc = build_plan(r->qubits, s->cfg.dtype, r->ops.data(), (int64_t)r->ops.size(), r->iterations, t,
+        int rc = build_plan(r->qubits, s->cfg.dtype, r->ops.data(), (int64_t)r->ops.size(), r->iterations, t,
                             &r->plan, &err, false, true);
         if (rc == HGM_OK && r->plan.kernel != HGM_KERNEL_REG) {
             rc = HGM_E_TUNING;

@@ -1,7 +1,9 @@
-"""The register kernel's host-generated programs, executed by a numpy model of
-the kernel's semantics (test infrastructure), must reproduce the oracle.
+"""The register programs that the plan-compiled and serving kernels are generated
+from, executed by a numpy model of their semantics (test infrastructure), must
+reproduce the oracle. (The interpreted kernels run programs of their own:
+test_exec_program.py.)
 
-The model follows k_pass_reg: thread t holds A amplitudes; element (t, k)
+In the model, thread t holds A amplitudes; element (t, k)
 sits at tile index thr[0][t & 31] | thr[1][t >> 5] | reg[k] of the current
 phase map; R_REMAP moves the tile to the next map; R_DENSE / R_ANTI update
 register pairs differing in register bit `rbit`; R_PHASE multiplies where the
